@@ -36,9 +36,14 @@
 //
 // Per-wavefront specialisation of the backward kernels: a wavefront whose
 // row lies in the x or z C-PML runs only the adjoint part (the reverse part
-// covers the interior only), and one whose row is interior along x and z
-// drops every x/z C-PML term (there a = 0 and K = 1 exactly, on both grids);
-// the y C-PML terms are compiled in only for wavefronts that touch a y slab.
+// covers the interior only), and the C-PML terms of an axis are compiled in
+// only for wavefronts that touch a slab of that axis (elsewhere a = 0 and
+// K = 1 exactly, on both grids): eight variants. Most C-PML rows lie in the
+// slab of one axis only; one variant for x and z together had them divide by
+// K = 1 and test a = 0 along the other one (stress_bwd has 9, velocity_bwd 15
+// such divisions over the axes, about 11 instructions each): 160x240x240
+// cells velocity_bwd 360 -> 351 us and stress_bwd 372 -> 359 us, 84^3 cells
+// 32.3 -> 30.9 us and 29.9 -> 28.1 us.
 //
 // Fusion: the source injection is folded into the forward stress kernel; the
 // backward pass runs two kernels per step, {reverse velocity + density
@@ -53,6 +58,7 @@
 //           adjoint C-PML coefficients, Src/velocity_adj.cu:139,142).
 // FORM = 1: the same three places corrected.
 #include <algorithm>
+#include <type_traits>
 
 #include "efwi_common.h"
 #include "efwi_kernels.h"
@@ -380,17 +386,17 @@ __device__ __forceinline__ void velocity_fwd_cell(const Geom& G, const Acc& acc,
 // launch order does. The adjoint part reads the adjoint stress and the psi
 // arrays written by the adjoint stress step, and writes v-dagger and the psi
 // arrays the adjoint stress step reads.
-// RV: reverse part allowed; XZ: the row lies in the x or z C-PML; Y: the
+// RV: reverse part allowed; X, Z: the row lies in the x, z C-PML; Y: the
 // wavefront touches a y C-PML slab.
 // ---------------------------------------------------------------------------
-template <int FORM, bool RV, bool XZ, bool Y, class Acc>
+template <int FORM, bool RV, bool X, bool Z, bool Y, class Acc>
 __device__ __forceinline__ void velocity_bwd_cell(const Geom& G, const Acc& acc, const Prof& C, const Cell& c) {
   const int z = c.z, x = c.x, y = c.y, p = G.npml;
   const float dt = G.dt;
   const Dv D(G);
   const bool py = Y && in_pml(y, G.ny, p);
-  const bool px = XZ && in_pml(x, G.nx, p), pz = XZ && in_pml(z, G.nz, p);
-  const bool rev = RV && !XZ && !py;
+  const bool px = X && in_pml(x, G.nx, p), pz = Z && in_pml(z, G.nz, p);
+  const bool rev = RV && !X && !Z && !py;
   // ---- loads
   float r_sz = 0.0f, r_sx = 0.0f, r_sy = 0.0f, vz = 0.0f, vx = 0.0f, vy = 0.0f, grho = 0.0f;
   if (rev) {
@@ -403,30 +409,30 @@ __device__ __forceinline__ void velocity_bwd_cell(const Geom& G, const Acc& acc,
   }
   const float lambda = acc.own(GM, M_LAM), mu = acc.own(GM, M_MU), byc = acc.own(GM, M_BYC);
   const float avz = acc.own(GA, F_VZ), avx = acc.own(GA, F_VX), avy = acc.own(GA, F_VY);
-  const float ax = XZ ? pr(C, 1, R_A, x) : 0.0f, az = XZ ? pr(C, 0, R_A, z) : 0.0f;
-  const float axh = XZ ? pr(C, 1, R_AH, x) : 0.0f, azh = XZ ? pr(C, 0, R_AH, z) : 0.0f;
+  const float ax = X ? pr(C, 1, R_A, x) : 0.0f, az = Z ? pr(C, 0, R_A, z) : 0.0f;
+  const float axh = X ? pr(C, 1, R_AH, x) : 0.0f, azh = Z ? pr(C, 0, R_AH, z) : 0.0f;
   const float ay = Y ? pr(C, 2, R_A, y) : 0.0f, ayh = Y ? pr(C, 2, R_AH, y) : 0.0f;
-  const float Kx = XZ ? pr(C, 1, R_K, x) : 1.0f;
-  const float Kz = XZ ? pr(C, 0, R_K, z) : 1.0f;
-  const float Kxh = XZ ? pr(C, 1, R_KH, x) : 1.0f;
-  const float Kzh = XZ ? pr(C, 0, R_KH, z) : 1.0f;
+  const float Kx = X ? pr(C, 1, R_K, x) : 1.0f;
+  const float Kz = Z ? pr(C, 0, R_K, z) : 1.0f;
+  const float Kxh = X ? pr(C, 1, R_KH, x) : 1.0f;
+  const float Kzh = Z ? pr(C, 0, R_KH, z) : 1.0f;
   const float Ky = Y ? pr(C, 2, R_K, y) : 1.0f;
   const float Kyh = Y ? pr(C, 2, R_KH, y) : 1.0f;
   // vx-dagger terms
-  const float x1 = apsi_f<XZ>(acc, ax, P_VX_X, AX, G.dx);
+  const float x1 = apsi_f<X>(acc, ax, P_VX_X, AX, G.dx);
   const float x_szz = D.x(n_af(acc, GA, F_SZZ, AX));
   const float x_sxx = D.x(n_af(acc, GA, F_SXX, AX));
   const float x_syy = D.x(n_af(acc, GA, F_SYY, AX));
-  const float x6 = apsi_b<XZ>(acc, azh, P_VX_Z, AZ, G.dz);
+  const float x6 = apsi_b<Z>(acc, azh, P_VX_Z, AZ, G.dz);
   const float x_sxz = D.z(n_ab(acc, GA, F_SXZ, AZ));
   const float x8 = apsi_b<Y>(acc, ayh, P_VX_Y, AY, G.dy);
   const float x_sxy = D.y(n_ab(acc, GA, F_SXY, AY));
   // vz-dagger terms
-  const float z1 = apsi_f<XZ>(acc, az, P_VZ_Z, AZ, G.dz);
+  const float z1 = apsi_f<Z>(acc, az, P_VZ_Z, AZ, G.dz);
   const float z_szz = D.z(n_af(acc, GA, F_SZZ, AZ));
   const float z_sxx = D.z(n_af(acc, GA, F_SXX, AZ));
   const float z_syy = D.z(n_af(acc, GA, F_SYY, AZ));
-  const float z8 = apsi_b<XZ>(acc, axh, P_VZ_X, AX, G.dx);
+  const float z8 = apsi_b<X>(acc, axh, P_VZ_X, AX, G.dx);
   const float z_sxz = D.x(n_ab(acc, GA, F_SXZ, AX));
   const float z6 = apsi_b<Y>(acc, ayh, P_VZ_Y, AY, G.dy);
   const float z_syz = D.y(n_ab(acc, GA, F_SYZ, AY));
@@ -435,9 +441,9 @@ __device__ __forceinline__ void velocity_bwd_cell(const Geom& G, const Acc& acc,
   const float y_syy = D.y(n_af(acc, GA, F_SYY, AY));
   const float y_sxx = D.y(n_af(acc, GA, F_SXX, AY));
   const float y_szz = D.y(n_af(acc, GA, F_SZZ, AY));
-  const float y6 = apsi_b<XZ>(acc, axh, P_VY_X, AX, G.dx);
+  const float y6 = apsi_b<X>(acc, axh, P_VY_X, AX, G.dx);
   const float y_sxy = D.x(n_ab(acc, GA, F_SXY, AX));
-  const float y8 = apsi_b<XZ>(acc, azh, P_VY_Z, AZ, G.dz);
+  const float y8 = apsi_b<Z>(acc, azh, P_VY_Z, AZ, G.dz);
   const float y_syz = D.z(n_ab(acc, GA, F_SYZ, AZ));
   // psi values updated by this step
   float qx0 = 0, qx1 = 0, qx2 = 0, qz0 = 0, qz1 = 0, qz2 = 0, qy0 = 0, qy1 = 0, qy2 = 0;
@@ -446,15 +452,15 @@ __device__ __forceinline__ void velocity_bwd_cell(const Geom& G, const Acc& acc,
   if (py) { qy0 = acc.own(GP, P_SXY_Y); qy1 = acc.own(GP, P_SYZ_Y); qy2 = acc.own(GP, P_SYY_Y); }
   // ---- arithmetic
   const float l2m = lambda + 2.0f * mu;
-  const float nvx = avx + (x1 + kdiv<XZ>(l2m * x_sxx, Kx) * dt + kdiv<XZ>(lambda * x_szz, Kx) * dt +
-                           kdiv<XZ>(lambda * x_syy, Kx) * dt + kdiv<XZ>(mu, Kzh) * x_sxz * dt + x6 +
+  const float nvx = avx + (x1 + kdiv<X>(l2m * x_sxx, Kx) * dt + kdiv<X>(lambda * x_szz, Kx) * dt +
+                           kdiv<X>(lambda * x_syy, Kx) * dt + kdiv<Z>(mu, Kzh) * x_sxz * dt + x6 +
                            kdiv<Y>(mu, Kyh) * x_sxy * dt + x8);
-  const float nvz = avz + (z1 + kdiv<XZ>(l2m * z_szz, Kz) * dt + kdiv<XZ>(lambda * z_sxx, Kz) * dt +
-                           kdiv<XZ>(lambda * z_syy, Kz) * dt + kdiv<Y>(mu, Kyh) * z_syz * dt + z6 +
-                           kdiv<XZ>(mu, Kxh) * z_sxz * dt + z8);
+  const float nvz = avz + (z1 + kdiv<Z>(l2m * z_szz, Kz) * dt + kdiv<Z>(lambda * z_sxx, Kz) * dt +
+                           kdiv<Z>(lambda * z_syy, Kz) * dt + kdiv<Y>(mu, Kyh) * z_syz * dt + z6 +
+                           kdiv<X>(mu, Kxh) * z_sxz * dt + z8);
   const float nvy = avy + (y1 + kdiv<Y>(l2m * y_syy, Ky) * dt + kdiv<Y>(lambda * y_sxx, Ky) * dt +
-                           kdiv<Y>(lambda * y_szz, Ky) * dt + kdiv<XZ>(mu, Kxh) * y_sxy * dt + y6 +
-                           kdiv<XZ>(mu, Kzh) * y_syz * dt + y8);
+                           kdiv<Y>(lambda * y_szz, Ky) * dt + kdiv<X>(mu, Kxh) * y_sxy * dt + y6 +
+                           kdiv<Z>(mu, Kzh) * y_syz * dt + y8);
   // ---- stores
   if (rev) {
     acc.st(GW, F_VZ, vz - r_sz * byc * dt);
@@ -495,7 +501,7 @@ __device__ __forceinline__ void velocity_bwd_cell(const Geom& G, const Acc& acc,
 // [2, n-3] the adjoint stress (Src/stress_adj.cu:1-146). The imaging terms
 // read the adjoint stress before the adjoint part updates it.
 // ---------------------------------------------------------------------------
-template <bool RV, bool XZ, bool Y, class Acc>
+template <bool RV, bool X, bool Z, bool Y, class Acc>
 __device__ __forceinline__ void stress_bwd_cell(const Geom& G, const Acc& acc, const Prof& C, const Cell& c,
                                                 unsigned src_o, float amp) {
   const unsigned o = c.o;
@@ -503,8 +509,8 @@ __device__ __forceinline__ void stress_bwd_cell(const Geom& G, const Acc& acc, c
   const float dt = G.dt;
   const Dv D(G);
   const bool py = Y && in_pml(y, G.ny, p);
-  const bool px = XZ && in_pml(x, G.nx, p), pz = XZ && in_pml(z, G.nz, p);
-  const bool rev = RV && !XZ && !py;
+  const bool px = X && in_pml(x, G.nx, p), pz = Z && in_pml(z, G.nz, p);
+  const bool rev = RV && !X && !Z && !py;
   const float lambda = acc.own(GM, M_LAM), mu = acc.own(GM, M_MU), byc = acc.own(GM, M_BYC);
   // ---- loads of the reverse part
   float dvz_dz = 0, dvx_dx = 0, dvy_dy = 0, dvx_dz = 0, dvx_dy = 0, dvz_dx = 0, dvz_dy = 0, dvy_dx = 0, dvy_dz = 0;
@@ -526,30 +532,30 @@ __device__ __forceinline__ void stress_bwd_cell(const Geom& G, const Acc& acc, c
   // ---- loads of the adjoint part
   const float aszz = acc.own(GA, F_SZZ), asxx = acc.own(GA, F_SXX), asyy = acc.own(GA, F_SYY);
   const float asxz = acc.own(GA, F_SXZ), asxy = acc.own(GA, F_SXY), asyz = acc.own(GA, F_SYZ);
-  const float ax = XZ ? pr(C, 1, R_A, x) : 0.0f, az = XZ ? pr(C, 0, R_A, z) : 0.0f;
-  const float axh = XZ ? pr(C, 1, R_AH, x) : 0.0f, azh = XZ ? pr(C, 0, R_AH, z) : 0.0f;
+  const float ax = X ? pr(C, 1, R_A, x) : 0.0f, az = Z ? pr(C, 0, R_A, z) : 0.0f;
+  const float axh = X ? pr(C, 1, R_AH, x) : 0.0f, azh = Z ? pr(C, 0, R_AH, z) : 0.0f;
   const float ay = Y ? pr(C, 2, R_A, y) : 0.0f, ayh = Y ? pr(C, 2, R_AH, y) : 0.0f;
-  const float Kx = XZ ? pr(C, 1, R_K, x) : 1.0f;
-  const float Kz = XZ ? pr(C, 0, R_K, z) : 1.0f;
+  const float Kx = X ? pr(C, 1, R_K, x) : 1.0f;
+  const float Kz = Z ? pr(C, 0, R_K, z) : 1.0f;
   const float Ky = Y ? pr(C, 2, R_K, y) : 1.0f;
-  const float Kxh = XZ ? pr(C, 1, R_KH, x) : 1.0f;
-  const float Kzh = XZ ? pr(C, 0, R_KH, z) : 1.0f;
+  const float Kxh = X ? pr(C, 1, R_KH, x) : 1.0f;
+  const float Kzh = Z ? pr(C, 0, R_KH, z) : 1.0f;
   const float Kyh = Y ? pr(C, 2, R_KH, y) : 1.0f;
-  const float xz1 = apsi_f<XZ>(acc, ax, P_SXZ_X, AX, G.dx);
+  const float xz1 = apsi_f<X>(acc, ax, P_SXZ_X, AX, G.dx);
   const float xz_vz = D.x(n_af(acc, GA, F_VZ, AX));
-  const float xz3 = apsi_f<XZ>(acc, az, P_SXZ_Z, AZ, G.dz);
+  const float xz3 = apsi_f<Z>(acc, az, P_SXZ_Z, AZ, G.dz);
   const float xz_vx = D.z(n_af(acc, GA, F_VX, AZ));
-  const float xy1 = apsi_f<XZ>(acc, ax, P_SXY_X, AX, G.dx);
+  const float xy1 = apsi_f<X>(acc, ax, P_SXY_X, AX, G.dx);
   const float xy_vy = D.x(n_af(acc, GA, F_VY, AX));
   const float xy3 = apsi_f<Y>(acc, ay, P_SXY_Y, AY, G.dy);
   const float xy_vx = D.y(n_af(acc, GA, F_VX, AY));
   const float yz1 = apsi_f<Y>(acc, ay, P_SYZ_Y, AY, G.dy);
   const float yz_vz = D.y(n_af(acc, GA, F_VZ, AY));
-  const float yz3 = apsi_f<XZ>(acc, az, P_SYZ_Z, AZ, G.dz);
+  const float yz3 = apsi_f<Z>(acc, az, P_SYZ_Z, AZ, G.dz);
   const float yz_vy = D.z(n_af(acc, GA, F_VY, AZ));
-  const float txx = apsi_b<XZ>(acc, axh, P_SXX_X, AX, G.dx);
+  const float txx = apsi_b<X>(acc, axh, P_SXX_X, AX, G.dx);
   const float xx_vx = D.x(n_ab(acc, GA, F_VX, AX));
-  const float tzz = apsi_b<XZ>(acc, azh, P_SZZ_Z, AZ, G.dz);
+  const float tzz = apsi_b<Z>(acc, azh, P_SZZ_Z, AZ, G.dz);
   const float zz_vz = D.z(n_ab(acc, GA, F_VZ, AZ));
   const float tyy = apsi_b<Y>(acc, ayh, P_SYY_Y, AY, G.dy);
   const float yy_vy = D.y(n_ab(acc, GA, F_VY, AY));
@@ -561,13 +567,13 @@ __device__ __forceinline__ void stress_bwd_cell(const Geom& G, const Acc& acc, c
   // ---- arithmetic
   const float l2m = lambda + 2.0f * mu;
   const float nsxz =
-      asxz + (xz1 + kdiv<XZ>(xz_vz, Kx) * byc * dt + xz3 + kdiv<XZ>(xz_vx, Kz) * byc * dt);
+      asxz + (xz1 + kdiv<X>(xz_vz, Kx) * byc * dt + xz3 + kdiv<Z>(xz_vx, Kz) * byc * dt);
   const float nsxy =
-      asxy + (xy1 + kdiv<XZ>(xy_vy, Kx) * byc * dt + xy3 + kdiv<Y>(xy_vx, Ky) * byc * dt);
+      asxy + (xy1 + kdiv<X>(xy_vy, Kx) * byc * dt + xy3 + kdiv<Y>(xy_vx, Ky) * byc * dt);
   const float nsyz =
-      asyz + (yz1 + kdiv<Y>(yz_vz, Ky) * byc * dt + yz3 + kdiv<XZ>(yz_vy, Kz) * byc * dt);
-  const float nsxx = asxx + (txx + kdiv<XZ>(byc * xx_vx, Kxh) * dt);
-  const float nszz = aszz + (tzz + kdiv<XZ>(byc * zz_vz, Kzh) * dt);
+      asyz + (yz1 + kdiv<Y>(yz_vz, Ky) * byc * dt + yz3 + kdiv<Z>(yz_vy, Kz) * byc * dt);
+  const float nsxx = asxx + (txx + kdiv<X>(byc * xx_vx, Kxh) * dt);
+  const float nszz = aszz + (tzz + kdiv<Z>(byc * zz_vz, Kzh) * dt);
   const float nsyy = asyy + (tyy + kdiv<Y>(byc * yy_vy, Kyh) * dt);
   // ---- stores
   if (rev) {
@@ -610,13 +616,31 @@ __device__ __forceinline__ void stress_bwd_cell(const Geom& G, const Acc& acc, c
   }
 }
 
-// Per-wavefront dispatch of the backward cells on (XZ, Y).
-struct Flags {
-  bool xz, y;
-};
-__device__ __forceinline__ Flags flags_of(const Geom& G, const Cell& c) {
+// Per-wavefront dispatch of the backward cells: body gets the flags (X, Z, Y)
+// of the variant as compile-time constants.
+template <typename Body>
+__device__ __forceinline__ void by_slabs(const Geom& G, const Cell& c, Body&& body) {
+  using T = std::true_type;
+  using N = std::false_type;
   const int p = G.npml;
-  return Flags{in_pml(c.x, G.nx, p) || in_pml(c.z, G.nz, p), __any(in_pml(c.y, G.ny, p)) != 0};
+  const bool x = in_pml(c.x, G.nx, p), z = in_pml(c.z, G.nz, p), y = __any(in_pml(c.y, G.ny, p)) != 0;
+  if (y) {
+    if (x) {
+      if (z) body(T{}, T{}, T{});
+      else body(T{}, N{}, T{});
+    } else {
+      if (z) body(N{}, T{}, T{});
+      else body(N{}, N{}, T{});
+    }
+  } else {
+    if (x) {
+      if (z) body(T{}, T{}, N{});
+      else body(T{}, N{}, N{});
+    } else {
+      if (z) body(N{}, T{}, N{});
+      else body(N{}, N{}, N{});
+    }
+  }
 }
 
 // Source amplitude of step it at the source cell, 1500^2 * stf[it] * dt
@@ -723,15 +747,10 @@ template <int FORM, bool RV>
 __global__ __launch_bounds__(256) EFWI_BWD_ATTR void k_velocity_bwd(Sweep Sw, Geom G, Groups F, Prof C, RingFold Rf) {
   sweep(Sw, G, [&](const Cell& c) {
     const FlatAcc acc = flat_acc(G, F, c);
-    const Flags f = flags_of(G, c);
     const RingRestore<F_VZ, F_VY + 1> rr(RV ? Rf : RingFold{}, c);
-    if (f.xz) {
-      if (f.y) velocity_bwd_cell<FORM, RV, true, true>(G, acc, C, c);
-      else velocity_bwd_cell<FORM, RV, true, false>(G, acc, C, c);
-    } else {
-      if (f.y) velocity_bwd_cell<FORM, RV, false, true>(G, acc, C, c);
-      else velocity_bwd_cell<FORM, RV, false, false>(G, acc, C, c);
-    }
+    by_slabs(G, c, [&](auto X, auto Z, auto Y) {
+      velocity_bwd_cell<FORM, RV, decltype(X)::value, decltype(Z)::value, decltype(Y)::value>(G, acc, C, c);
+    });
     if (RV) rr.store(acc);
   });
 }
@@ -746,15 +765,10 @@ __global__ __launch_bounds__(256) EFWI_BWD_ATTR void k_stress_bwd(Sweep Sw, Geom
   const float amp = RV ? source_amp(S, G, it) : 0.0f;
   sweep(Sw, G, [&](const Cell& c) {
     const FlatAcc acc = flat_acc(G, F, c);
-    const Flags f = flags_of(G, c);
     const RingRestore<F_SZZ, F_WAVE_COUNT> rr(RV ? Rf : RingFold{}, c);
-    if (f.xz) {
-      if (f.y) stress_bwd_cell<RV, true, true>(G, acc, C, c, so, amp);
-      else stress_bwd_cell<RV, true, false>(G, acc, C, c, so, amp);
-    } else {
-      if (f.y) stress_bwd_cell<RV, false, true>(G, acc, C, c, so, amp);
-      else stress_bwd_cell<RV, false, false>(G, acc, C, c, so, amp);
-    }
+    by_slabs(G, c, [&](auto X, auto Z, auto Y) {
+      stress_bwd_cell<RV, decltype(X)::value, decltype(Z)::value, decltype(Y)::value>(G, acc, C, c, so, amp);
+    });
     if (RV) rr.store(acc);
   });
 }
@@ -766,7 +780,7 @@ __global__ __launch_bounds__(256) void k_velocity_bwd_in(Sweep Sw, Geom G, Group
   sweep(Sw, G, [&](const Cell& c) {
     const FlatAcc acc = flat_acc(G, F, c);
     const RingRestore<F_VZ, F_VY + 1> rr(Rf, c);
-    velocity_bwd_cell<FORM, true, false, false>(G, acc, C, c);
+    velocity_bwd_cell<FORM, true, false, false, false>(G, acc, C, c);
     rr.store(acc);
   });
 }
@@ -777,7 +791,7 @@ __global__ __launch_bounds__(256) void k_stress_bwd_in(Sweep Sw, Geom G, Groups 
   sweep(Sw, G, [&](const Cell& c) {
     const FlatAcc acc = flat_acc(G, F, c);
     const RingRestore<F_SZZ, F_WAVE_COUNT> rr(Rf, c);
-    stress_bwd_cell<true, false, false>(G, acc, C, c, so, amp);
+    stress_bwd_cell<true, false, false, false>(G, acc, C, c, so, amp);
     rr.store(acc);
   });
 }
@@ -966,14 +980,9 @@ __global__ __launch_bounds__(64 * R) void k_velocity_fwd_m(Sweep Sw, Geom G, Gro
 template <int FORM, int R>
 __global__ __launch_bounds__(64 * R) void k_velocity_bwd_m(Sweep Sw, Geom G, Groups F, Prof C) {
   march<VelocityBwdSlots, R>(Sw, G, F, [&](const Cell& c, const auto& acc) {
-    const Flags f = flags_of(G, c);
-    if (f.xz) {
-      if (f.y) velocity_bwd_cell<FORM, true, true, true>(G, acc, C, c);
-      else velocity_bwd_cell<FORM, true, true, false>(G, acc, C, c);
-    } else {
-      if (f.y) velocity_bwd_cell<FORM, true, false, true>(G, acc, C, c);
-      else velocity_bwd_cell<FORM, true, false, false>(G, acc, C, c);
-    }
+    by_slabs(G, c, [&](auto X, auto Z, auto Y) {
+      velocity_bwd_cell<FORM, true, decltype(X)::value, decltype(Z)::value, decltype(Y)::value>(G, acc, C, c);
+    });
   });
 }
 
@@ -982,14 +991,9 @@ __global__ __launch_bounds__(64 * R) void k_stress_bwd_m(Sweep Sw, Geom G, Group
   const unsigned so = source_off(S);
   const float amp = source_amp(S, G, it);
   march<StressBwdSlots, R>(Sw, G, F, [&](const Cell& c, const auto& acc) {
-    const Flags f = flags_of(G, c);
-    if (f.xz) {
-      if (f.y) stress_bwd_cell<true, true, true>(G, acc, C, c, so, amp);
-      else stress_bwd_cell<true, true, false>(G, acc, C, c, so, amp);
-    } else {
-      if (f.y) stress_bwd_cell<true, false, true>(G, acc, C, c, so, amp);
-      else stress_bwd_cell<true, false, false>(G, acc, C, c, so, amp);
-    }
+    by_slabs(G, c, [&](auto X, auto Z, auto Y) {
+      stress_bwd_cell<true, decltype(X)::value, decltype(Z)::value, decltype(Y)::value>(G, acc, C, c, so, amp);
+    });
   });
 }
 
@@ -1296,15 +1300,10 @@ __global__ __launch_bounds__(256) void k_batch(Sweep Sw, Geom G, Prof C, BatchLa
     } else if constexpr (KIND == 2) {
       sweep_block(Sw, G, b, [&](const Cell& c) {
         const FlatAcc acc = flat_acc(G, F, c);
-        const Flags f = flags_of(G, c);
         const RingRestore<F_VZ, F_VY + 1> rr(Rf, c);
-        if (f.xz) {
-          if (f.y) velocity_bwd_cell<FORM, true, true, true>(G, acc, C, c);
-          else velocity_bwd_cell<FORM, true, true, false>(G, acc, C, c);
-        } else {
-          if (f.y) velocity_bwd_cell<FORM, true, false, true>(G, acc, C, c);
-          else velocity_bwd_cell<FORM, true, false, false>(G, acc, C, c);
-        }
+        by_slabs(G, c, [&](auto X, auto Z, auto Y) {
+          velocity_bwd_cell<FORM, true, decltype(X)::value, decltype(Z)::value, decltype(Y)::value>(G, acc, C, c);
+        });
         rr.store(acc);
       });
     } else {
@@ -1312,15 +1311,10 @@ __global__ __launch_bounds__(256) void k_batch(Sweep Sw, Geom G, Prof C, BatchLa
       const float amp = source_amp(S, G, it);
       sweep_block(Sw, G, b, [&](const Cell& c) {
         const FlatAcc acc = flat_acc(G, F, c);
-        const Flags f = flags_of(G, c);
         const RingRestore<F_SZZ, F_WAVE_COUNT> rr(Rf, c);
-        if (f.xz) {
-          if (f.y) stress_bwd_cell<true, true, true>(G, acc, C, c, so, amp);
-          else stress_bwd_cell<true, true, false>(G, acc, C, c, so, amp);
-        } else {
-          if (f.y) stress_bwd_cell<true, false, true>(G, acc, C, c, so, amp);
-          else stress_bwd_cell<true, false, false>(G, acc, C, c, so, amp);
-        }
+        by_slabs(G, c, [&](auto X, auto Z, auto Y) {
+          stress_bwd_cell<true, decltype(X)::value, decltype(Z)::value, decltype(Y)::value>(G, acc, C, c, so, amp);
+        });
         rr.store(acc);
       });
     }
