@@ -33,7 +33,7 @@ int Ctx::batch_group_size(int n) const {
   if (batch.group > 0) return std::min(batch.group, n);
   if (batch.group < 0) return 0;
   const Tile t = tiles[K_STRESS_FWD].zdepth >= 16 ? Tile{4, 1} : tiles[K_STRESS_FWD];
-  const long per_shot = make_sweep(2, cfg.nz - 3, 2, cfg.nx - 3, 2, cfg.ny - 3, t).blocks;
+  const long per_shot = flat_blocks(G, t);
   const long want = (long)kBatchFill * std::max(batch.cus, 1);
   if (per_shot >= want) return 0;
   return (int)std::max(1L, std::min((long)n, (want + per_shot - 1) / std::max(per_shot, 1L)));

@@ -31,15 +31,17 @@ struct Tile {
 // the first rows_rem XCDs) x rows and walks it by chunks of Z planes.
 struct Sweep {
   int z0, nz, x0, rows_base, rows_rem, rg_max, y0, y1, yb0, nyb, R, Z, nzc;  // y segments yb0 .. yb0+nyb-1
+  int ly;    // lanes of a wavefront along y: 64 (one row) or 32 (two rows)
   int zrev;  // plane chunks last to first (consecutive kernels alternate, so that each starts where the
              // previous one ended, on data the Infinity Cache still holds)
   // cells the sweep leaves out (another launch covers them): planes
-  // [sk_z0, sk_z1] of rows [sk_x0, sk_x1] in y segments [sk_yb0, sk_yb1];
-  // empty when sk_z0 > sk_z1
-  int sk_z0, sk_z1, sk_x0, sk_x1, sk_yb0, sk_yb1;
+  // [sk_z0, sk_z1] of rows [sk_x0, sk_x1], y in [sk_y0, sk_y1]; empty when
+  // sk_z0 > sk_z1
+  int sk_z0, sk_z1, sk_x0, sk_x1, sk_y0, sk_y1;
   long blocks;
 };
-Sweep make_sweep(int z0, int z1, int x0, int x1, int y0, int y1, Tile t);
+// Workgroups of a flat forward launch of shape t on the grid's stencil box.
+long flat_blocks(const Geom& G, Tile t);
 
 // Fused forward step (stress + velocity of one time step in one launch):
 // workgroups of 64 x (R + 4) threads own R x rows of 60 y cells and Zc z

@@ -27,8 +27,8 @@
 // across a wavefront (a wavefront is one 64-cell segment of one x row) and
 // come through scalar loads.
 //
-// Work distribution ("sweep"): workgroups of 64 x R threads (R rows of 64
-// y-consecutive cells), numbered b = 0, 1, ...; workgroup b runs on XCD
+// Work distribution ("sweep"): workgroups of R wavefronts (each 64 consecutive
+// y cells of a row, or 32 of two rows), numbered b = 0, 1, ...; workgroup b runs on XCD
 // b % 8 (round-robin dispatch), and the kernels map b so that each XCD owns a
 // contiguous strip of x rows and walks it plane chunk by plane chunk in z.
 // The x and z neighbours a cell reads were then fetched into that XCD's L2 by
@@ -36,14 +36,9 @@
 //
 // Per-wavefront specialisation of the backward kernels: a wavefront whose
 // row lies in the x or z C-PML runs only the adjoint part (the reverse part
-// covers the interior only), and the C-PML terms of an axis are compiled in
-// only for wavefronts that touch a slab of that axis (elsewhere a = 0 and
-// K = 1 exactly, on both grids): eight variants. Most C-PML rows lie in the
-// slab of one axis only; one variant for x and z together had them divide by
-// K = 1 and test a = 0 along the other one (stress_bwd has 9, velocity_bwd 15
-// such divisions over the axes, about 11 instructions each): 160x240x240
-// cells velocity_bwd 360 -> 351 us and stress_bwd 372 -> 359 us, 84^3 cells
-// 32.3 -> 30.9 us and 29.9 -> 28.1 us.
+// covers the interior only), and one whose row is interior along x and z
+// drops every x/z C-PML term (there a = 0 and K = 1 exactly, on both grids);
+// the y C-PML terms are compiled in only for wavefronts that touch a y slab.
 //
 // Fusion: the source injection is folded into the forward stress kernel; the
 // backward pass runs two kernels per step, {reverse velocity + density
@@ -212,10 +207,11 @@ __device__ __forceinline__ Pv pv(const Prof& C, int ax, bool half, int i) {
               : Pv{pr(C, ax, R_B, i), pr(C, ax, R_A, i), pr(C, ax, R_K, i)};
 }
 
-// Workgroup b (64 x R threads: y lanes x rows) covers R rows of the strip of
-// XCD b % 8 and Z consecutive planes; the strip is walked plane chunk by
+// Workgroup b (R wavefronts of 64 / LY rows) covers R 64 / LY rows of the strip
+// of XCD b % 8 and Z consecutive planes; the strip is walked plane chunk by
 // plane chunk (z slowest), so each XCD's L2 sees a compact, z-ordered region.
-template <typename Body>
+// LY: lanes along y, 64 or 32 (the two halves of a wavefront on two rows).
+template <int LY, typename Body>
 __device__ __forceinline__ void sweep_block(const Sweep& S, const Geom& G, int b, Body&& body) {
   const int xcd = b & 7, j = b >> 3;
   const int per_plane = S.rg_max * S.nyb;
@@ -226,14 +222,16 @@ __device__ __forceinline__ void sweep_block(const Sweep& S, const Geom& G, int b
   const int yb = r - rg * S.nyb;
   const int rows = S.rows_base + (xcd < S.rows_rem ? 1 : 0);
   // blockDim.x == 64: threadIdx.y is uniform across a wavefront
-  const int row = __builtin_amdgcn_readfirstlane(rg * S.R + (int)threadIdx.y);
+  const int wrow = __builtin_amdgcn_readfirstlane(rg * S.R + (int)threadIdx.y);
+  const int row = LY == 64 ? wrow : 2 * wrow + ((int)threadIdx.x >> 5);
   if (row >= rows) return;
   Cell c;
   c.x = S.x0 + xcd * S.rows_base + min(xcd, S.rows_rem) + row;
-  c.y = (S.yb0 + yb) * 64 + (int)threadIdx.x;
+  const int ys = (S.yb0 + yb) * LY;
+  c.y = ys + (LY == 64 ? (int)threadIdx.x : (int)threadIdx.x & 31);
   if (c.y < S.y0 || c.y > S.y1) return;
-  // planes of this wavefront's row segment that another launch covers
-  const bool skip_col = c.x >= S.sk_x0 && c.x <= S.sk_x1 && S.yb0 + yb >= S.sk_yb0 && S.yb0 + yb <= S.sk_yb1;
+  // planes of this row segment that another launch covers
+  const bool skip_col = c.x >= S.sk_x0 && c.x <= S.sk_x1 && ys >= S.sk_y0 && ys <= S.sk_y1;
   const int skz0 = skip_col ? S.sk_z0 : 1, skz1 = skip_col ? S.sk_z1 : 0;
   const unsigned sx = 4u * (unsigned)G.py, sz = 4u * (unsigned)G.pxy;
   const int za = S.z0 + zc * S.Z;
@@ -258,9 +256,9 @@ __device__ __forceinline__ void sweep_block(const Sweep& S, const Geom& G, int b
     oy += sz;
   }
 }
-template <typename Body>
+template <int LY, typename Body>
 __device__ __forceinline__ void sweep(const Sweep& S, const Geom& G, Body&& body) {
-  sweep_block(S, G, (int)blockIdx.x, body);
+  sweep_block<LY>(S, G, (int)blockIdx.x, body);
 }
 
 // ---------------------------------------------------------------------------
@@ -386,7 +384,7 @@ __device__ __forceinline__ void velocity_fwd_cell(const Geom& G, const Acc& acc,
 // launch order does. The adjoint part reads the adjoint stress and the psi
 // arrays written by the adjoint stress step, and writes v-dagger and the psi
 // arrays the adjoint stress step reads.
-// RV: reverse part allowed; X, Z: the row lies in the x, z C-PML; Y: the
+// RV: reverse part allowed; XZ: the row lies in the x or z C-PML; Y: the
 // wavefront touches a y C-PML slab.
 // ---------------------------------------------------------------------------
 template <int FORM, bool RV, bool X, bool Z, bool Y, class Acc>
@@ -729,23 +727,24 @@ struct RingRestore {
   }
 };
 
+template <int LY>
 __global__ __launch_bounds__(256) EFWI_FWD_ATTR void k_stress_fwd(Sweep Sw, Geom G, Groups F, Prof C, Source S, int it,
                                                                   RingFold Rf) {
   const unsigned so = source_off(S);
   const float amp = source_amp(S, G, it);
-  sweep(Sw, G, [&](const Cell& c) { stress_fwd_cell(G, save_acc(G, F, Rf, c), C, c, so, amp); });
+  sweep<LY>(Sw, G, [&](const Cell& c) { stress_fwd_cell(G, save_acc(G, F, Rf, c), C, c, so, amp); });
 }
 
-template <int FORM>
+template <int FORM, int LY>
 __global__ __launch_bounds__(256) EFWI_FWD_ATTR void k_velocity_fwd(Sweep Sw, Geom G, Groups F, Prof C, RingFold Rf) {
-  sweep(Sw, G, [&](const Cell& c) { velocity_fwd_cell<FORM>(G, save_acc(G, F, Rf, c), C, c); });
+  sweep<LY>(Sw, G, [&](const Cell& c) { velocity_fwd_cell<FORM>(G, save_acc(G, F, Rf, c), C, c); });
 }
 
 // Backward velocity step (RV = true): reverse velocity + density imaging
 // (interior), then the adjoint velocity ([2, n-3]); RV = false: adjoint only.
-template <int FORM, bool RV>
+template <int FORM, bool RV, int LY>
 __global__ __launch_bounds__(256) EFWI_BWD_ATTR void k_velocity_bwd(Sweep Sw, Geom G, Groups F, Prof C, RingFold Rf) {
-  sweep(Sw, G, [&](const Cell& c) {
+  sweep<LY>(Sw, G, [&](const Cell& c) {
     const FlatAcc acc = flat_acc(G, F, c);
     const RingRestore<F_VZ, F_VY + 1> rr(RV ? Rf : RingFold{}, c);
     by_slabs(G, c, [&](auto X, auto Z, auto Y) {
@@ -758,12 +757,12 @@ __global__ __launch_bounds__(256) EFWI_BWD_ATTR void k_velocity_bwd(Sweep Sw, Ge
 // Backward stress step (RV = true): (source subtraction +) reverse stress +
 // lambda/mu imaging (interior), then the adjoint stress ([2, n-3]);
 // RV = false: adjoint only.
-template <bool RV>
+template <bool RV, int LY>
 __global__ __launch_bounds__(256) EFWI_BWD_ATTR void k_stress_bwd(Sweep Sw, Geom G, Groups F, Prof C, Source S, int it,
                                                                   RingFold Rf) {
   const unsigned so = RV ? source_off(S) : 0xFFFFFFFFu;
   const float amp = RV ? source_amp(S, G, it) : 0.0f;
-  sweep(Sw, G, [&](const Cell& c) {
+  sweep<LY>(Sw, G, [&](const Cell& c) {
     const FlatAcc acc = flat_acc(G, F, c);
     const RingRestore<F_SZZ, F_WAVE_COUNT> rr(RV ? Rf : RingFold{}, c);
     by_slabs(G, c, [&](auto X, auto Z, auto Y) {
@@ -777,7 +776,7 @@ __global__ __launch_bounds__(256) EFWI_BWD_ATTR void k_stress_bwd(Sweep Sw, Geom
 // (the interior launch of the split): one variant, no C-PML terms.
 template <int FORM>
 __global__ __launch_bounds__(256) void k_velocity_bwd_in(Sweep Sw, Geom G, Groups F, Prof C, RingFold Rf) {
-  sweep(Sw, G, [&](const Cell& c) {
+  sweep<64>(Sw, G, [&](const Cell& c) {
     const FlatAcc acc = flat_acc(G, F, c);
     const RingRestore<F_VZ, F_VY + 1> rr(Rf, c);
     velocity_bwd_cell<FORM, true, false, false, false>(G, acc, C, c);
@@ -788,7 +787,7 @@ __global__ __launch_bounds__(256) void k_stress_bwd_in(Sweep Sw, Geom G, Groups 
                                                        RingFold Rf) {
   const unsigned so = source_off(S);
   const float amp = source_amp(S, G, it);
-  sweep(Sw, G, [&](const Cell& c) {
+  sweep<64>(Sw, G, [&](const Cell& c) {
     const FlatAcc acc = flat_acc(G, F, c);
     const RingRestore<F_SZZ, F_WAVE_COUNT> rr(Rf, c);
     stress_bwd_cell<true, false, false, false>(G, acc, C, c, so, amp);
@@ -1268,7 +1267,7 @@ __device__ __forceinline__ long uniform_long(long x) {
 }
 
 // KIND: 0 stress_fwd, 1 velocity_fwd, 2 velocity_bwd, 3 stress_bwd
-template <int KIND, int FORM>
+template <int KIND, int FORM, int LY>
 __global__ __launch_bounds__(256) void k_batch(Sweep Sw, Geom G, Prof C, BatchLaunch L, int per_xcd, BatchRing R) {
   const int it = device_step(L.it);
   // ring slot of this step (the same index in every shot's ring), or none
@@ -1294,13 +1293,13 @@ __global__ __launch_bounds__(256) void k_batch(Sweep Sw, Geom G, Prof C, BatchLa
     if constexpr (KIND == 0) {
       const unsigned so = source_off(S);
       const float amp = source_amp(S, G, it);
-      sweep_block(Sw, G, b, [&](const Cell& c) { stress_fwd_cell(G, save_acc(G, F, Rf, c), C, c, so, amp); });
+      sweep_block<LY>(Sw, G, b, [&](const Cell& c) { stress_fwd_cell(G, save_acc(G, F, Rf, c), C, c, so, amp); });
     } else if constexpr (KIND == 1) {
-      sweep_block(Sw, G, b, [&](const Cell& c) { velocity_fwd_cell<FORM>(G, save_acc(G, F, Rf, c), C, c); });
+      sweep_block<LY>(Sw, G, b, [&](const Cell& c) { velocity_fwd_cell<FORM>(G, save_acc(G, F, Rf, c), C, c); });
     } else if constexpr (KIND == 2) {
-      sweep_block(Sw, G, b, [&](const Cell& c) {
+      sweep_block<LY>(Sw, G, b, [&](const Cell& c) {
         const FlatAcc acc = flat_acc(G, F, c);
-        const RingRestore<F_VZ, F_VY + 1> rr(Rf, c);
+            const RingRestore<F_VZ, F_VY + 1> rr(Rf, c);
         by_slabs(G, c, [&](auto X, auto Z, auto Y) {
           velocity_bwd_cell<FORM, true, decltype(X)::value, decltype(Z)::value, decltype(Y)::value>(G, acc, C, c);
         });
@@ -1309,9 +1308,9 @@ __global__ __launch_bounds__(256) void k_batch(Sweep Sw, Geom G, Prof C, BatchLa
     } else {
       const unsigned so = source_off(S);
       const float amp = source_amp(S, G, it);
-      sweep_block(Sw, G, b, [&](const Cell& c) {
+      sweep_block<LY>(Sw, G, b, [&](const Cell& c) {
         const FlatAcc acc = flat_acc(G, F, c);
-        const RingRestore<F_SZZ, F_WAVE_COUNT> rr(Rf, c);
+            const RingRestore<F_SZZ, F_WAVE_COUNT> rr(Rf, c);
         by_slabs(G, c, [&](auto X, auto Z, auto Y) {
           stress_bwd_cell<true, decltype(X)::value, decltype(Z)::value, decltype(Y)::value>(G, acc, C, c, so, amp);
         });
@@ -1326,7 +1325,8 @@ __global__ __launch_bounds__(256) void k_batch(Sweep Sw, Geom G, Prof C, BatchLa
 // ---------------------------------------------------------------------------
 // Launchers.
 // ---------------------------------------------------------------------------
-Sweep make_sweep(int z0, int z1, int x0, int x1, int y0, int y1, Tile t) {
+// ly: lanes of a wavefront along y (64 / ly rows).
+static Sweep make_sweep(int z0, int z1, int x0, int x1, int y0, int y1, Tile t, int ly) {
   Sweep S;
   S.R = t.rows < 1 ? 1 : (t.rows > 4 ? 4 : t.rows);
   S.Z = t.zdepth < 1 ? 1 : t.zdepth;
@@ -1335,19 +1335,39 @@ Sweep make_sweep(int z0, int z1, int x0, int x1, int y0, int y1, Tile t) {
   const int nxr = x1 - x0 + 1;
   S.rows_base = nxr / 8;
   S.rows_rem = nxr % 8;
-  const int rows_max = S.rows_base + (S.rows_rem ? 1 : 0);
-  S.rg_max = (rows_max + S.R - 1) / S.R;
+  const int rows_max = S.rows_base + (S.rows_rem ? 1 : 0), rw = 64 / ly;
+  S.rg_max = (rows_max + S.R * rw - 1) / (S.R * rw);
   S.y0 = y0; S.y1 = y1;
-  S.yb0 = y0 / 64;  // segments of 64 aligned at y = 0, from the one holding y0
-  S.nyb = y1 / 64 - S.yb0 + 1;
+  S.yb0 = y0 / ly;  // segments aligned at y = 0, from the one holding y0
+  S.nyb = y1 / ly - S.yb0 + 1;
   S.nzc = (S.nz + S.Z - 1) / S.Z;
+  S.ly = ly;
   S.zrev = 0;
-  S.sk_z0 = 1; S.sk_z1 = 0; S.sk_x0 = 1; S.sk_x1 = 0; S.sk_yb0 = 1; S.sk_yb1 = 0;
+  S.sk_z0 = 1; S.sk_z1 = 0; S.sk_x0 = 1; S.sk_x1 = 0; S.sk_y0 = 1; S.sk_y1 = 0;
   S.blocks = 8L * S.rg_max * S.nyb * S.nzc;
   return S;
 }
 
-static inline Sweep sweep_full(const Geom& G, Tile t) { return make_sweep(2, G.nz - 3, 2, G.nx - 3, 2, G.ny - 3, t); }
+static inline Sweep sweep_full(const Geom& G, Tile t, int ly) {
+  return make_sweep(2, G.nz - 3, 2, G.nx - 3, 2, G.ny - 3, t, ly);
+}
+// The flat sweep of a launch. A wavefront covers 64 y cells of one row, or 32
+// of two rows: the latter where it leaves at most 7/8 as many lanes per row
+// (fewer lanes past the row's end, and y C-PML terms in fewer wavefronts) and
+// the rows keep the device busy (at least 16 wavefronts per CU; on smaller
+// grids one wavefront's latency is what counts, and a wavefront with rows of
+// two kinds runs both variants). stress_fwd / velocity_fwd / velocity_bwd /
+// stress_bwd in us, 64 against 32 lanes: 84^3 cells (80 cells per row: 128 and
+// 96 lanes) 15.7 / 14.3 / 30.8 / 28.4 against 13.9 / 12.5 / 26.1 / 23.0;
+// 110x212x212 (256 and 224 lanes) 114 / 83 / 216 / 220 against 105 / 77 / 201 /
+// 183; 160x240x240 (256 lanes either way) 209 / 168 / 368 / 368 against 226 /
+// 185 / 396 / 345.
+static inline Sweep sweep_flat(const Geom& G, Tile t) {
+  const Sweep a = sweep_full(G, t, 64), b = sweep_full(G, t, 32);
+  const long waves = (long)(G.nz - 4) * (G.nx - 4) * a.nyb;
+  return 8 * 32 * b.nyb <= 7 * 64 * a.nyb && waves >= 16 * 256 ? b : a;
+}
+long flat_blocks(const Geom& G, Tile t) { return sweep_flat(G, t).blocks; }
 
 static inline dim3 grid_of(const Sweep& S) { return dim3((unsigned)S.blocks); }
 static inline dim3 block_of(const Sweep& S) { return dim3(64, S.R); }
@@ -1356,7 +1376,7 @@ static inline dim3 block_of(const Sweep& S) { return dim3(64, S.R); }
 // workgroup); smaller ones the flat sweep (rows 1, 2 or 4).
 static inline bool marching(Tile t) { return t.zdepth >= 16; }
 static inline Sweep sweep_march(const Geom& G, Tile t) {
-  Sweep S = sweep_full(G, Tile{1, t.zdepth});
+  Sweep S = sweep_full(G, Tile{1, t.zdepth}, 64);
   const int R = t.rows >= 8 ? 8 : 4;
   S.R = R;
   const int rows_max = S.rows_base + (S.rows_rem ? 1 : 0);
@@ -1364,6 +1384,13 @@ static inline Sweep sweep_march(const Geom& G, Tile t) {
   S.blocks = 8L * S.rg_max * S.nyb * S.nzc;
   return S;
 }
+// Launch of a flat kernel template over its last argument, the lanes per row.
+#define EFWI_FLAT(SW, KERNEL, ...)                                                                        \
+  do {                                                                                                    \
+    if ((SW).ly == 32) hipLaunchKernelGGL((KERNEL 32>), grid_of(SW), block_of(SW), 0, s, __VA_ARGS__);    \
+    else hipLaunchKernelGGL((KERNEL 64>), grid_of(SW), block_of(SW), 0, s, __VA_ARGS__);                  \
+  } while (0)
+#define EFWI_COMMA ,
 #define EFWI_MARCH(KERNEL, ZREV, ...)                                                             \
   do {                                                                                            \
     Sweep Sw = sweep_march(G, t);                                                                 \
@@ -1394,9 +1421,9 @@ bool launch_stress_fwd(Tile t, const Geom& G, const Groups& F, const Prof& C, co
     EFWI_MARCH(k_stress_fwd_m, 0, Sw, G, F, C, S, it);
     return false;
   }
-  const Sweep Sw = sweep_full(G, t);
+  const Sweep Sw = sweep_flat(G, t);
   const RingFold Rf = fold_for(G, ring);
-  hipLaunchKernelGGL(k_stress_fwd, grid_of(Sw), block_of(Sw), 0, s, Sw, G, F, C, S, it, Rf);
+  EFWI_FLAT(Sw, k_stress_fwd<, Sw, G, F, C, S, it, Rf);
   return Rf.slot != nullptr;
 }
 bool launch_velocity_fwd(Tile t, int form, const Geom& G, const Groups& F, const Prof& C, hipStream_t s,
@@ -1413,11 +1440,11 @@ bool launch_velocity_fwd(Tile t, int form, const Geom& G, const Groups& F, const
     }
     return false;
   }
-  Sweep Sw = sweep_full(G, t);
+  Sweep Sw = sweep_flat(G, t);
   Sw.zrev = 1;  // the stress kernel before it ran first to last
   const RingFold Rf = fold_for(G, ring);
-  if (form == 1) hipLaunchKernelGGL(k_velocity_fwd<1>, grid_of(Sw), block_of(Sw), 0, s, Sw, G, F, C, Rf);
-  else hipLaunchKernelGGL(k_velocity_fwd<0>, grid_of(Sw), block_of(Sw), 0, s, Sw, G, F, C, Rf);
+  if (form == 1) EFWI_FLAT(Sw, k_velocity_fwd<1 EFWI_COMMA, Sw, G, F, C, Rf);
+  else EFWI_FLAT(Sw, k_velocity_fwd<0 EFWI_COMMA, Sw, G, F, C, Rf);
   return Rf.slot != nullptr;
 }
 // y segments wholly inside the y interior [p, ny - 1 - p]: [lo, hi] (empty if lo > hi)
@@ -1436,11 +1463,11 @@ static inline Sweep split_sweeps(const Geom& G, Tile t, Sweep& rim) {
   int lo, hi;
   interior_segments(G, lo, hi);
   const int p = G.npml;
-  Sweep in = make_sweep(p, G.nz - 1 - p, p, G.nx - 1 - p, 64 * lo, 64 * hi + 63, t);
-  rim = make_sweep(2, G.nz - 3, 2, G.nx - 3, 2, G.ny - 3, t);
+  Sweep in = make_sweep(p, G.nz - 1 - p, p, G.nx - 1 - p, 64 * lo, 64 * hi + 63, t, 64);
+  rim = sweep_full(G, t, 64);
   rim.sk_z0 = p; rim.sk_z1 = G.nz - 1 - p;
   rim.sk_x0 = p; rim.sk_x1 = G.nx - 1 - p;
-  rim.sk_yb0 = lo; rim.sk_yb1 = hi;
+  rim.sk_y0 = 64 * lo; rim.sk_y1 = 64 * hi + 63;
   return in;
 }
 
@@ -1463,16 +1490,16 @@ bool launch_velocity_bwd(Tile t, int form, const Geom& G, const Groups& F, const
     const Sweep in = split_sweeps(G, t, rim);
     if (form == 1) {
       hipLaunchKernelGGL(k_velocity_bwd_in<1>, grid_of(in), block_of(in), 0, s, in, G, F, C, Rf);
-      hipLaunchKernelGGL((k_velocity_bwd<1, true>), grid_of(rim), block_of(rim), 0, s, rim, G, F, C, Rf);
+      hipLaunchKernelGGL((k_velocity_bwd<1, true, 64>), grid_of(rim), block_of(rim), 0, s, rim, G, F, C, Rf);
     } else {
       hipLaunchKernelGGL(k_velocity_bwd_in<0>, grid_of(in), block_of(in), 0, s, in, G, F, C, Rf);
-      hipLaunchKernelGGL((k_velocity_bwd<0, true>), grid_of(rim), block_of(rim), 0, s, rim, G, F, C, Rf);
+      hipLaunchKernelGGL((k_velocity_bwd<0, true, 64>), grid_of(rim), block_of(rim), 0, s, rim, G, F, C, Rf);
     }
     return Rf.slot != nullptr;
   }
-  const Sweep Sw = sweep_full(G, t);
-  if (form == 1) hipLaunchKernelGGL((k_velocity_bwd<1, true>), grid_of(Sw), block_of(Sw), 0, s, Sw, G, F, C, Rf);
-  else hipLaunchKernelGGL((k_velocity_bwd<0, true>), grid_of(Sw), block_of(Sw), 0, s, Sw, G, F, C, Rf);
+  const Sweep Sw = sweep_flat(G, t);
+  if (form == 1) EFWI_FLAT(Sw, k_velocity_bwd<1 EFWI_COMMA true EFWI_COMMA, Sw, G, F, C, Rf);
+  else EFWI_FLAT(Sw, k_velocity_bwd<0 EFWI_COMMA true EFWI_COMMA, Sw, G, F, C, Rf);
   return Rf.slot != nullptr;
 }
 bool launch_stress_bwd(Tile t, const Geom& G, const Groups& F, const Prof& C, const Source& S, int it,
@@ -1487,12 +1514,12 @@ bool launch_stress_bwd(Tile t, const Geom& G, const Groups& F, const Prof& C, co
     Sweep in = split_sweeps(G, t, rim);
     in.zrev = rim.zrev = 1;
     hipLaunchKernelGGL(k_stress_bwd_in, grid_of(in), block_of(in), 0, s, in, G, F, C, S, it, Rf);
-    hipLaunchKernelGGL(k_stress_bwd<true>, grid_of(rim), block_of(rim), 0, s, rim, G, F, C, S, it, Rf);
+    hipLaunchKernelGGL((k_stress_bwd<true, 64>), grid_of(rim), block_of(rim), 0, s, rim, G, F, C, S, it, Rf);
     return Rf.slot != nullptr;
   }
-  Sweep Sw = sweep_full(G, t);
+  Sweep Sw = sweep_flat(G, t);
   Sw.zrev = 1;  // the velocity kernel before it ran first to last
-  hipLaunchKernelGGL(k_stress_bwd<true>, grid_of(Sw), block_of(Sw), 0, s, Sw, G, F, C, S, it, Rf);
+  EFWI_FLAT(Sw, k_stress_bwd<true EFWI_COMMA, Sw, G, F, C, S, it, Rf);
   return Rf.slot != nullptr;
 }
 bool launch_fwd_fused(int R, int zc, int form, const Geom& G, const Groups& Fi, const Groups& Fo, const Prof& C,
@@ -1519,24 +1546,24 @@ bool launch_fwd_fused(int R, int zc, int form, const Geom& G, const Groups& Fi, 
 }
 
 void launch_velocity_adj(int form, const Geom& G, const Groups& F, const Prof& C, hipStream_t s) {
-  const Sweep Sw = sweep_full(G, Tile{1, 1});
+  const Sweep Sw = sweep_flat(G, Tile{1, 1});
   const RingFold none = fold_for(G, nullptr);
-  if (form == 1) hipLaunchKernelGGL((k_velocity_bwd<1, false>), grid_of(Sw), block_of(Sw), 0, s, Sw, G, F, C, none);
-  else hipLaunchKernelGGL((k_velocity_bwd<0, false>), grid_of(Sw), block_of(Sw), 0, s, Sw, G, F, C, none);
+  if (form == 1) EFWI_FLAT(Sw, k_velocity_bwd<1 EFWI_COMMA false EFWI_COMMA, Sw, G, F, C, none);
+  else EFWI_FLAT(Sw, k_velocity_bwd<0 EFWI_COMMA false EFWI_COMMA, Sw, G, F, C, none);
 }
 void launch_stress_adj(const Geom& G, const Groups& F, const Prof& C, hipStream_t s) {
-  const Sweep Sw = sweep_full(G, Tile{1, 1});
+  const Sweep Sw = sweep_flat(G, Tile{1, 1});
   Source none;
   none.cell = -1;
   none.stf = nullptr;
-  hipLaunchKernelGGL(k_stress_bwd<false>, grid_of(Sw), block_of(Sw), 0, s, Sw, G, F, C, none, 0, fold_for(G, nullptr));
+  EFWI_FLAT(Sw, k_stress_bwd<false EFWI_COMMA, Sw, G, F, C, none, 0, fold_for(G, nullptr));
 }
 
 // Batched launches (flat tiles only; a zdepth >= 16 shape falls back to its
 // flat counterpart rows x 1).
 static inline Sweep sweep_batch(const Geom& G, Tile t) {
   if (t.zdepth >= 16) t = Tile{t.rows >= 4 ? 4 : t.rows, 1};
-  return sweep_full(G, t);
+  return sweep_flat(G, t);
 }
 int device_cus(int device) {
   int cus = 256;
@@ -1568,18 +1595,25 @@ static inline dim3 batch_plan(const Sweep& Sw, BatchLaunch& L, int per_cu, int s
   L.take = (int)std::max(1L, std::min((long)L.take, rest / (wq * 2)));
   return dim3((unsigned)(8 * wq));
 }
-#define EFWI_BATCH(KERNEL)                                                                     \
-  do {                                                                                        \
-    static int occ_cache[8] = {0};                                                            \
-    Sweep Sw = sweep_batch(G, t);                                                             \
-    Sw.zrev = L.reverse; /* shots and planes last to first: start where the last launch ended */ \
-    const int per_xcd = (int)(Sw.blocks / 8);                                                 \
-    const dim3 blk = block_of(Sw);                                                            \
-    const int per_cu = resident_per_cu((KERNEL), (int)(blk.x * blk.y * blk.z), occ_cache);    \
-    BatchLaunch Lk = L;                                                                       \
-    const dim3 grid = batch_plan(Sw, Lk, per_cu, L.stat);                                             \
-    hipLaunchKernelGGL((KERNEL), grid, blk, 0, s, Sw, G, C, Lk, per_xcd, R);                  \
-  } while (0)
+template <class K>
+static void launch_batch(K kernel, int* occ_cache, const Sweep& Sw, const Geom& G, const Prof& C, const BatchLaunch& L,
+                         hipStream_t s, const BatchRing& R) {
+  const int per_xcd = (int)(Sw.blocks / 8);
+  const dim3 blk = block_of(Sw);
+  const int per_cu = resident_per_cu(kernel, (int)(blk.x * blk.y * blk.z), occ_cache);
+  BatchLaunch Lk = L;
+  const dim3 grid = batch_plan(Sw, Lk, per_cu, L.stat);
+  hipLaunchKernelGGL(kernel, grid, blk, 0, s, Sw, G, C, Lk, per_xcd, R);
+}
+template <int KIND, int FORM>
+static void launch_batch(Tile t, const Geom& G, const Prof& C, const BatchLaunch& L, hipStream_t s,
+                         const BatchRing& R) {
+  static int occ[2][8] = {{0}};
+  Sweep Sw = sweep_batch(G, t);
+  Sw.zrev = L.reverse;  // shots and planes last to first: start where the last launch ended
+  if (Sw.ly == 32) launch_batch(k_batch<KIND, FORM, 32>, occ[0], Sw, G, C, L, s, R);
+  else launch_batch(k_batch<KIND, FORM, 64>, occ[1], Sw, G, C, L, s, R);
+}
 // The caller's ring fold where it applies, else none.
 static inline BatchRing batch_ring(const Geom& G, const BatchRing* ring) {
   if (ring && ring->mode && ring_foldable(G, ring->B)) return *ring;
@@ -1590,24 +1624,24 @@ static inline BatchRing batch_ring(const Geom& G, const BatchRing* ring) {
 void launch_stress_fwd_batch(Tile t, const Geom& G, const Prof& C, const BatchLaunch& L, hipStream_t s,
                              const BatchRing* ring) {
   const BatchRing R = batch_ring(G, ring);
-  EFWI_BATCH((k_batch<0, 0>));
+  launch_batch<0, 0>(t, G, C, L, s, R);
 }
 void launch_velocity_fwd_batch(Tile t, int form, const Geom& G, const Prof& C, const BatchLaunch& L, hipStream_t s,
                                const BatchRing* ring) {
   const BatchRing R = batch_ring(G, ring);
-  if (form == 1) EFWI_BATCH((k_batch<1, 1>));
-  else EFWI_BATCH((k_batch<1, 0>));
+  if (form == 1) launch_batch<1, 1>(t, G, C, L, s, R);
+  else launch_batch<1, 0>(t, G, C, L, s, R);
 }
 void launch_velocity_bwd_batch(Tile t, int form, const Geom& G, const Prof& C, const BatchLaunch& L, hipStream_t s,
                                const BatchRing* ring) {
   const BatchRing R = batch_ring(G, ring);
-  if (form == 1) EFWI_BATCH((k_batch<2, 1>));
-  else EFWI_BATCH((k_batch<2, 0>));
+  if (form == 1) launch_batch<2, 1>(t, G, C, L, s, R);
+  else launch_batch<2, 0>(t, G, C, L, s, R);
 }
 void launch_stress_bwd_batch(Tile t, const Geom& G, const Prof& C, const BatchLaunch& L, hipStream_t s,
                              const BatchRing* ring) {
   const BatchRing R = batch_ring(G, ring);
-  EFWI_BATCH((k_batch<3, 0>));
+  launch_batch<3, 0>(t, G, C, L, s, R);
 }
 
 }  // namespace efwi

@@ -1,0 +1,52 @@
+"""The launch rules of the stencil kernels at the sizes where they change:
+each route against the oracle, bit for bit (no tolerance: the kernels evaluate
+the oracle's float expressions in its order)."""
+import numpy as np
+import pytest
+import torch
+
+from util import oracle_run
+
+pytestmark = pytest.mark.gpu
+
+
+def _gradient(w, obs, prepare=None):
+    """(syn, res, gradients) of every shot's run through one propagator."""
+    from efwi.propagator import Propagator
+    print(f"[gpu] grid={w.grid.shape} nt={w.grid.nt} form={w.grid.formulation} npml={w.grid.npml}", flush=True)
+    with Propagator(w.grid) as P:
+        if prepare:
+            prepare(P)
+        P.set_model(*(torch.from_numpy(a) for a in w.model))
+        P.zero_gradient()
+        syns, ress = [], []
+        for s, o in zip(w.shots, obs):
+            _, syn, res = P.run_shot(s, 1, torch.from_numpy(o), want_syn=True, want_res=True)
+            syns.append(syn.cpu().numpy())
+            ress.append(res.cpu().numpy())
+        return syns, ress, [g.cpu().numpy() for g in P.gradient()]
+
+
+def _check(orc, w, prepare=None):
+    obs = [s.astype(np.float32) for s in oracle_run(orc, w, model=w.true, calc_id=2).syn]
+    syns, ress, grads = _gradient(w, obs, prepare)
+    ref = oracle_run(orc, w, model=w.model, obs=obs, calc_id=1)
+    for k in range(len(w.shots)):
+        assert np.array_equal(syns[k], ref.syn[k].astype(np.float32))
+        assert np.array_equal(ress[k], ref.res[k].astype(np.float32))
+    for a, b in zip(grads, (ref.glam, ref.gmu, ref.grho)):
+        assert np.abs(b).max() > 0
+        assert np.array_equal(a, b.astype(np.float32))
+
+
+# padded y sizes: one 32-cell segment (2..31), a last segment of 4 cells, one
+# of 18, and one whole; 65 rows over 8 strips leave an odd row in every strip
+@pytest.mark.parametrize("ny,formulation", [(34, 0), (70, 1), (84, 0), (98, 0)])
+def test_two_rows_per_wavefront(orc, ny, formulation):
+    """Grids whose rows waste lanes of 64-cell segments run 32 lanes on each of
+    two rows per wavefront; rows of both halves differ in their C-PML slabs."""
+    from efwi import synth
+    npml = 6
+    w = synth.small(n=69 - 2 * npml, npml=npml, nt=24, ny=ny - 2 * npml, formulation=formulation)
+    assert w.grid.shape == (69, 69, ny)
+    _check(orc, w)
