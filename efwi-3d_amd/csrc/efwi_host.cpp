@@ -539,6 +539,41 @@ int Ctx::zero_gradient(hipStream_t s) {
   return EFWI_OK;
 }
 
+// The receivers of a shot by row (RecvFold), uploaded in one copy. They stay
+// with the gather and scatter launches where one lies outside the stencil box
+// (the velocity kernels never visit it) or the tables would be large
+// (receivers spread over many rows).
+int Ctx::map_receivers(const efwi_shot* sh, RecvMap& m) {
+  constexpr size_t kMaxTab = 1u << 20;
+  m.on = false;
+  const int n = sh->nrec;
+  if (n <= 0 || !recv_foldable(Tile{1, 1}, G, true)) return EFWI_OK;
+  const size_t nrows = (size_t)cfg.nz * cfg.nx, py = (size_t)G.py;
+  std::vector<int> host(nrows + n, -1);
+  size_t used = 0;
+  for (int r = 0; r < n; r++) {
+    const int z = sh->rec[3 * r], x = sh->rec[3 * r + 1], y = sh->rec[3 * r + 2];
+    if (z < 2 || z > cfg.nz - 3 || x < 2 || x > cfg.nx - 3 || y < 2 || y > cfg.ny - 3) return EFWI_OK;
+    int& k = host[(size_t)z * cfg.nx + x];
+    if (k < 0) k = (int)used++;
+    if (used * py > kMaxTab) return EFWI_OK;
+  }
+  m.next_off = nrows;
+  m.tab_off = nrows + n;
+  host.resize(m.tab_off + used * py, -1);
+  for (int r = n - 1; r >= 0; r--) {
+    const int z = sh->rec[3 * r], x = sh->rec[3 * r + 1], y = sh->rec[3 * r + 2];
+    int& first = host[m.tab_off + (size_t)host[(size_t)z * cfg.nx + x] * py + y];
+    host[m.next_off + r] = first;
+    first = r;
+  }
+  int rc;
+  if ((rc = grow(this, (void**)&m.dev, &m.cap, sizeof(int) * host.size()))) return rc;
+  HIP_TRY(hipMemcpy(m.dev, host.data(), sizeof(int) * host.size(), hipMemcpyHostToDevice));
+  m.on = true;
+  return EFWI_OK;
+}
+
 int Ctx::prepare_shot(const efwi_shot* sh, int calc_id) {
   const int nt = cfg.nt;
   if (!sh || !sh->stf) return fail(EFWI_ERR_ARG, "shot or its stf is NULL");
@@ -570,6 +605,7 @@ int Ctx::prepare_shot(const efwi_shot* sh, int calc_id) {
   int rc;
   if ((rc = grow(this, (void**)&rec_dev, &rec_cap, sizeof(long) * nrb))) return rc;
   if (nrec) HIP_TRY(hipMemcpy(rec_dev, cells.data(), sizeof(long) * nrec, hipMemcpyHostToDevice));
+  if ((rc = map_receivers(sh, recv))) return rc;
   const size_t seis = sizeof(float) * (size_t)nt * 3 * nrb;
   if ((rc = grow(this, (void**)&syn_t, &syn_cap, seis))) return rc;
   if (calc_id != EFWI_CALC_SYNTHETIC) {
@@ -605,8 +641,10 @@ void Ctx::forward_step(const Groups& Ff, const Wave& Wf, const Source& Sf, int i
   const bool fs = launch_stress_fwd(tiles[K_STRESS_FWD], G, Ff, C, Sf, it, s, src_stencil ? &rf : nullptr);
   prof.end(s);
   if (!src_stencil) launch_add_source(Wf.szz, Wf.sxx, Wf.syy, src_cell, stf_dev, it, G.dt, +1, s);
+  RecvFold rec = record && recv_foldable(tiles[K_VELOCITY_FWD], G, true) ? recv.fold(nrec) : RecvFold{};
+  if (rec.row) rec.out = syn_t + (size_t)(it + 1) * 3 * nrec;
   prof.begin(K_VELOCITY_FWD, s);
-  const bool fv = launch_velocity_fwd(tiles[K_VELOCITY_FWD], cfg.formulation, G, Ff, C, s, &rf);
+  const bool fv = launch_velocity_fwd(tiles[K_VELOCITY_FWD], cfg.formulation, G, Ff, C, s, &rf, &rec);
   prof.end(s);
   if (save >= 0 && !(fs && fv)) {
     Fields9 F9;
@@ -616,7 +654,7 @@ void Ctx::forward_step(const Groups& Ff, const Wave& Wf, const Source& Sf, int i
     if (!fs) launch_ring(B, G, F9, ring, save, F_SZZ, F_WAVE_COUNT, 0, s);
     prof.end(s);
   }
-  if (record) launch_record(Wf, rec_dev, nrec, it + 1, syn_t, s);
+  if (record && !rec.row) launch_record(Wf, rec_dev, nrec, it + 1, syn_t, s);
 }
 
 // The second set of wavefield and C-PML arrays of the fused steps, zeroed
@@ -766,12 +804,14 @@ int Ctx::run_shot(const efwi_shot* sh, int calc_id, const float* obs, float* syn
         RingFold rf{};
         rf.B = B;
         rf.slot = ring + slot * 9 * B.n;
+        RecvFold inj = split_bwd == 0 && recv_foldable(tiles[K_VELOCITY_BWD], G, false) ? recv.fold(nrec) : RecvFold{};
+        if (inj.row) inj.res = res_t + (size_t)it * 3 * nrec;
         prof.begin(K_VELOCITY_BWD, s);
-        const bool fv = launch_velocity_bwd(tiles[K_VELOCITY_BWD], form, G, F, C, s, &rf, split_bwd == 1);
+        const bool fv = launch_velocity_bwd(tiles[K_VELOCITY_BWD], form, G, F, C, s, &rf, split_bwd == 1, &inj);
         prof.end(s);
         if (!fv) launch_ring(B, G, F9, ring, slot, F_VZ, F_VY + 1, 1, s);
         if (!src_interior) launch_add_source(W.szz, W.sxx, W.syy, src_cell, stf_dev, it, G.dt, -1, s);
-        launch_inject(A, rec_dev, nrec, it, res_t, s);
+        if (!inj.row) launch_inject(A, rec_dev, nrec, it, res_t, s);
         prof.begin(K_STRESS_BWD, s);
         const bool fs = launch_stress_bwd(tiles[K_STRESS_BWD], G, F, C, S, it, s, &rf, split_bwd == 1);
         prof.end(s);

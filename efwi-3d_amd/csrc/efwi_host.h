@@ -43,6 +43,18 @@ struct Profiler {
   void release();
 };
 
+// The tables of a RecvFold in one device buffer: rows [nz * nx], then next
+// [nrec], then tab. `on`: the shot's receivers can be folded.
+struct RecvMap {
+  int* dev = nullptr;
+  size_t cap = 0;
+  bool on = false;
+  size_t next_off = 0, tab_off = 0;
+  RecvFold fold(int nrec) const {
+    return on ? RecvFold{dev, dev + tab_off, dev + next_off, nullptr, nullptr, nrec} : RecvFold{};
+  }
+};
+
 // Batched shots (efwi_run_batch): per-shot state, the device shot table, the
 // per-XCD queue heads, the device time step, a capture stream and the two
 // captured per-step graphs.
@@ -111,6 +123,7 @@ struct Ctx {
   float* w2_dev = nullptr;
   long* rec_dev = nullptr;
   size_t rec_cap = 0;
+  RecvMap recv;  // receivers by row, for the velocity kernels
   float* syn_t = nullptr;
   size_t syn_cap = 0;
   float* obs_t = nullptr;
@@ -151,6 +164,7 @@ struct Ctx {
   void fused_forward_step(const Source& Sf, int it, bool record, hipStream_t s, long save = -1);
   int set_model(const float* l, const float* m, const float* rho, int on_host, hipStream_t s);
   int zero_gradient(hipStream_t s);
+  int map_receivers(const efwi_shot* sh, RecvMap& m);
   int prepare_shot(const efwi_shot* sh, int calc_id);
   int run_shot(const efwi_shot* sh, int calc_id, const float* obs, float* syn, float* res,
                double* misfit, hipStream_t s);

@@ -66,17 +66,31 @@ struct RingFold {
   float* slot;  // ring + slot index * 9 * B.n, or null: no ring traffic
 };
 bool ring_foldable(const Geom& G, const Band& B);
+// Receivers folded into the velocity kernels: the cell of a receiver writes
+// its new velocity to the seismograms (forward), or adds the residuals to its
+// adjoint velocity (backward). row[z * nx + x]: the row's index in tab, or -1;
+// tab[index * py + y]: the cell's first receiver, or -1; next[r]: the
+// receiver after r in the same cell, or -1. Callers pass one only where
+// recv_foldable holds (and no split for velocity_bwd); nothing is then left
+// for launch_record / launch_inject.
+struct RecvFold {
+  const int *row, *tab, *next;  // row null: no receivers folded
+  float* out;                   // forward: the recorded step's [3][nrec] (x, y, z)
+  const float* res;             // backward: the injected step's [3][nrec]
+  int nrec;
+};
+bool recv_foldable(Tile t, const Geom& G, bool forward);
 bool launch_stress_fwd(Tile t, const Geom& G, const Groups& F, const Prof& C, const Source& S, int it,
                        hipStream_t s, const RingFold* ring = nullptr);
 bool launch_velocity_fwd(Tile t, int form, const Geom& G, const Groups& F, const Prof& C, hipStream_t s,
-                         const RingFold* ring = nullptr);
+                         const RingFold* ring = nullptr, const RecvFold* recv = nullptr);
 // split: the wavefronts clear of every C-PML slab (rows inside the x and z
 // interior, 64-cell y segments inside the y interior) run as a launch of
 // their own on a kernel without the C-PML terms (fewer registers, more
 // wavefronts per SIMD), the rest as the general kernel's launch that skips
 // them. Flat sweeps only; results do not depend on it.
 bool launch_velocity_bwd(Tile t, int form, const Geom& G, const Groups& F, const Prof& C, hipStream_t s,
-                         const RingFold* ring = nullptr, bool split = false);
+                         const RingFold* ring = nullptr, bool split = false, const RecvFold* recv = nullptr);
 bool launch_stress_bwd(Tile t, const Geom& G, const Groups& F, const Prof& C, const Source& S, int it,
                        hipStream_t s, const RingFold* ring = nullptr, bool split = false);
 // whether the grid has wavefronts clear of every C-PML slab

@@ -124,6 +124,9 @@ struct FlatAcc {
     return ld(g(gi), k, d == 0 ? o : d == -2 ? b.m2 : d == -1 ? b.m1 : d == 1 ? b.p1 : b.p2);
   }
   __device__ __forceinline__ void st(int gi, int k, float v) const { efwi::st(g(gi), k, o, v); }
+  // the new velocity of the cell; the adjoint velocity before it is stored
+  __device__ __forceinline__ void record(float, float, float) const {}
+  __device__ __forceinline__ void inject(float&, float&, float&) const {}
 };
 
 // Difference numerators of the 4th-order staggered operators along axis ax;
@@ -368,9 +371,13 @@ __device__ __forceinline__ void velocity_fwd_cell(const Geom& G, const Acc& acc,
     dsxy_dy = cpml(i.b, i.a, i.K, qy1, dsxy_dy);
     dsyy_dy = cpml(h.b, h.a, h.K, qy2, dsyy_dy);
   }
-  acc.st(GW, F_VZ, vz + (dszz_dz + dsxz_dx + dsyz_dy) * byc * dt);
-  acc.st(GW, F_VX, vx + (dsxz_dz + dsxx_dx + dsxy_dy) * byc * dt);
-  acc.st(GW, F_VY, vy + (dsyz_dz + dsxy_dx + dsyy_dy) * byc * dt);
+  const float nvz = vz + (dszz_dz + dsxz_dx + dsyz_dy) * byc * dt;
+  const float nvx = vx + (dsxz_dz + dsxx_dx + dsxy_dy) * byc * dt;
+  const float nvy = vy + (dsyz_dz + dsxy_dx + dsyy_dy) * byc * dt;
+  acc.st(GW, F_VZ, nvz);
+  acc.st(GW, F_VX, nvx);
+  acc.st(GW, F_VY, nvy);
+  acc.record(nvx, nvy, nvz);
   if (pz) { acc.st(GP, P_SZZ_Z, qz0); acc.st(GP, P_SXZ_Z, qz1); acc.st(GP, P_SYZ_Z, qz2); }
   if (px) { acc.st(GP, P_SXZ_X, qx0); acc.st(GP, P_SXX_X, qx1); acc.st(GP, P_SXY_X, qx2); }
   if (py) { acc.st(GP, P_SYZ_Y, qy0); acc.st(GP, P_SXY_Y, qy1); acc.st(GP, P_SYY_Y, qy2); }
@@ -467,9 +474,11 @@ __device__ __forceinline__ void velocity_bwd_cell(const Geom& G, const Acc& acc,
     const float nb2 = -(byc * byc);
     acc.st(GM, M_GRHO, grho + -(avz * r_sz * dt * nb2 + avx * r_sx * dt * nb2 + avy * r_sy * dt * nb2));
   }
-  acc.st(GA, F_VX, nvx);
-  acc.st(GA, F_VZ, nvz);
-  acc.st(GA, F_VY, nvy);
+  float jvx = nvx, jvy = nvy, jvz = nvz;  // the psi below are fed before the injection
+  acc.inject(jvx, jvy, jvz);
+  acc.st(GA, F_VX, jvx);
+  acc.st(GA, F_VZ, jvz);
+  acc.st(GA, F_VY, jvy);
   if (px) {
     const float b = pr(C, 1, R_B, x), bh = pr(C, 1, R_BH, x);
     acc.st(GP, P_SXX_X, bh * qx0 + byc * nvx * dt);
@@ -688,21 +697,69 @@ __device__ __forceinline__ int ring_index(const RingFold& R, const Cell& c) {
   return R.slot ? band_index(R.B, c.z, c.x, c.y) : -1;
 }
 
+// First receiver of the cell, or -1. Only rows that hold receivers (one load
+// per wavefront) look the cell up.
+__device__ __forceinline__ int first_receiver(const RecvFold& V, const Geom& G, const Cell& c) {
+  if (!V.row) return -1;
+  const int k = V.row[c.z * G.nx + c.x];
+  return k >= 0 ? V.tab[(long)k * G.py + c.y] : -1;
+}
+
 // Accessor of the forward kernels: a band cell's new wavefield values also go
 // to the ring slot (rk: the cell's index in a slot's field, or -1), so the
 // boundary save needs no pass of its own. The ring's field order is the
-// WaveField order.
+// WaveField order. A receiver cell's new velocity goes to the seismograms
+// (Src/utilities.cu:481-495): a gather launch of its own took 4.6 us per step
+// (its two dependent loads), a tenth of a step at 84^3 cells.
 struct SaveAcc : FlatAcc {
   float* rs;
   long rn;
   int rk;
+  RecvFold V;
+  int r0;
+  __device__ __forceinline__ void record(float vx, float vy, float vz) const {
+    for (int r = r0; r >= 0; r = V.next[r]) {
+      V.out[r] = vx;
+      V.out[V.nrec + r] = vy;
+      V.out[2 * V.nrec + r] = vz;
+    }
+  }
   __device__ __forceinline__ void st(int gi, int k, float v) const {
     FlatAcc::st(gi, k, v);
     if (gi == GW && rk >= 0) rs[(long)k * rn + rk] = v;
   }
 };
-__device__ __forceinline__ SaveAcc save_acc(const Geom& G, const Groups& F, const RingFold& R, const Cell& c) {
-  return SaveAcc{flat_acc(G, F, c), R.slot, R.B.n, ring_index(R, c)};
+__device__ __forceinline__ SaveAcc save_acc(const Geom& G, const Groups& F, const RingFold& R, const Cell& c,
+                                            const RecvFold& V = RecvFold{}) {
+  return SaveAcc{flat_acc(G, F, c), R.slot, R.B.n, ring_index(R, c), V, first_receiver(V, G, c)};
+}
+
+// Accessor of the backward velocity kernel: the residuals of the cell's
+// receivers are added to the adjoint velocity (Src/utilities.cu:497-507), one
+// after another; those of the first receiver are loaded with the cell.
+struct InjectAcc : FlatAcc {
+  RecvFold V;
+  int r0;
+  float q[3];
+  __device__ __forceinline__ void inject(float& vx, float& vy, float& vz) const {
+    if (r0 < 0) return;
+    vx += q[0];
+    vy += q[1];
+    vz += q[2];
+    for (int r = V.next[r0]; r >= 0; r = V.next[r]) {
+      vx += V.res[r];
+      vy += V.res[V.nrec + r];
+      vz += V.res[2 * V.nrec + r];
+    }
+  }
+};
+__device__ __forceinline__ InjectAcc inject_acc(const Geom& G, const Groups& F, const Cell& c, const RecvFold& V) {
+  InjectAcc a{flat_acc(G, F, c), V, first_receiver(V, G, c), {0.0f, 0.0f, 0.0f}};
+  if (a.r0 >= 0) {
+#pragma unroll
+    for (int i = 0; i < 3; i++) a.q[i] = V.res[i * V.nrec + a.r0];
+  }
+  return a;
 }
 
 // Restore folded into a backward kernel: a band cell loads the slot's values
@@ -735,17 +792,21 @@ __global__ __launch_bounds__(256) EFWI_FWD_ATTR void k_stress_fwd(Sweep Sw, Geom
   sweep<LY>(Sw, G, [&](const Cell& c) { stress_fwd_cell(G, save_acc(G, F, Rf, c), C, c, so, amp); });
 }
 
-template <int FORM, int LY>
-__global__ __launch_bounds__(256) EFWI_FWD_ATTR void k_velocity_fwd(Sweep Sw, Geom G, Groups F, Prof C, RingFold Rf) {
-  sweep<LY>(Sw, G, [&](const Cell& c) { velocity_fwd_cell<FORM>(G, save_acc(G, F, Rf, c), C, c); });
+template <int FORM, bool REC, int LY>
+__global__ __launch_bounds__(256) EFWI_FWD_ATTR void k_velocity_fwd(Sweep Sw, Geom G, Groups F, Prof C, RingFold Rf,
+                                                                    RecvFold V) {
+  sweep<LY>(Sw, G, [&](const Cell& c) {
+    velocity_fwd_cell<FORM>(G, save_acc(G, F, Rf, c, REC ? V : RecvFold{}), C, c);
+  });
 }
 
 // Backward velocity step (RV = true): reverse velocity + density imaging
 // (interior), then the adjoint velocity ([2, n-3]); RV = false: adjoint only.
-template <int FORM, bool RV, int LY>
-__global__ __launch_bounds__(256) EFWI_BWD_ATTR void k_velocity_bwd(Sweep Sw, Geom G, Groups F, Prof C, RingFold Rf) {
+template <int FORM, bool RV, bool REC, int LY>
+__global__ __launch_bounds__(256) EFWI_BWD_ATTR void k_velocity_bwd(Sweep Sw, Geom G, Groups F, Prof C, RingFold Rf,
+                                                                    RecvFold V) {
   sweep<LY>(Sw, G, [&](const Cell& c) {
-    const FlatAcc acc = flat_acc(G, F, c);
+    const InjectAcc acc = inject_acc(G, F, c, REC ? V : RecvFold{});
     const RingRestore<F_VZ, F_VY + 1> rr(RV ? Rf : RingFold{}, c);
     by_slabs(G, c, [&](auto X, auto Z, auto Y) {
       velocity_bwd_cell<FORM, RV, decltype(X)::value, decltype(Z)::value, decltype(Y)::value>(G, acc, C, c);
@@ -867,6 +928,8 @@ struct MarchAcc {
     return ax == AX ? p[d * kTileW] : ax == AY ? p[d] : p[0];
   }
   __device__ __forceinline__ void st(int g, int k, float v) const { f.st(g, k, v); }
+  __device__ __forceinline__ void record(float, float, float) const {}
+  __device__ __forceinline__ void inject(float&, float&, float&) const {}
 };
 
 template <class S, int R, typename Body>
@@ -1067,6 +1130,8 @@ struct FusedVAcc {
       efwi::st(po, k, f.o, v);
     }
   }
+  __device__ __forceinline__ void record(float, float, float) const {}
+  __device__ __forceinline__ void inject(float&, float&, float&) const {}
 };
 
 template <int FORM, int R>
@@ -1426,8 +1491,20 @@ bool launch_stress_fwd(Tile t, const Geom& G, const Groups& F, const Prof& C, co
   EFWI_FLAT(Sw, k_stress_fwd<, Sw, G, F, C, S, it, Rf);
   return Rf.slot != nullptr;
 }
+// Receivers are folded up to 256 (forward) and 128 (backward) wavefronts per
+// CU: on larger grids the kernels lose more to the folded form's registers
+// (velocity_bwd 117 -> 123) than the launches cost. A gradient of 44^3 cells
+// 4.29 -> 3.88 ms for 119 steps, of 84^3 cells 45.1 -> 43.7 ms for 499; the
+// forward pass of 84x180x180 cells 37.2 -> 36.9 ms for 499; a gradient of 160x240x240
+// cells would go from 162 to 165 ms for 149.
+bool recv_foldable(Tile t, const Geom& G, bool forward) {
+  const long waves = (long)(G.nz - 4) * (G.nx - 4) * ((G.ny - 3) / 64 + 1);
+  return !marching(t) && waves <= (forward ? 256 : 128) * 256;
+}
+static inline RecvFold recv_for(const RecvFold* v) { return v ? *v : RecvFold{}; }
+
 bool launch_velocity_fwd(Tile t, int form, const Geom& G, const Groups& F, const Prof& C, hipStream_t s,
-                         const RingFold* ring) {
+                         const RingFold* ring, const RecvFold* recv) {
   if (marching(t)) {
     Sweep Sw = sweep_march(G, t);
     Sw.zrev = 1;
@@ -1443,8 +1520,14 @@ bool launch_velocity_fwd(Tile t, int form, const Geom& G, const Groups& F, const
   Sweep Sw = sweep_flat(G, t);
   Sw.zrev = 1;  // the stress kernel before it ran first to last
   const RingFold Rf = fold_for(G, ring);
-  if (form == 1) EFWI_FLAT(Sw, k_velocity_fwd<1 EFWI_COMMA, Sw, G, F, C, Rf);
-  else EFWI_FLAT(Sw, k_velocity_fwd<0 EFWI_COMMA, Sw, G, F, C, Rf);
+  const RecvFold V = recv_for(recv);
+  if (V.row) {
+    if (form == 1) EFWI_FLAT(Sw, k_velocity_fwd<1 EFWI_COMMA true EFWI_COMMA, Sw, G, F, C, Rf, V);
+    else EFWI_FLAT(Sw, k_velocity_fwd<0 EFWI_COMMA true EFWI_COMMA, Sw, G, F, C, Rf, V);
+  } else {
+    if (form == 1) EFWI_FLAT(Sw, k_velocity_fwd<1 EFWI_COMMA false EFWI_COMMA, Sw, G, F, C, Rf, V);
+    else EFWI_FLAT(Sw, k_velocity_fwd<0 EFWI_COMMA false EFWI_COMMA, Sw, G, F, C, Rf, V);
+  }
   return Rf.slot != nullptr;
 }
 // y segments wholly inside the y interior [p, ny - 1 - p]: [lo, hi] (empty if lo > hi)
@@ -1472,7 +1555,7 @@ static inline Sweep split_sweeps(const Geom& G, Tile t, Sweep& rim) {
 }
 
 bool launch_velocity_bwd(Tile t, int form, const Geom& G, const Groups& F, const Prof& C, hipStream_t s,
-                         const RingFold* ring, bool split) {
+                         const RingFold* ring, bool split, const RecvFold* recv) {
   if (marching(t)) {
     const Sweep Sw = sweep_march(G, t);
     if (form == 1) {
@@ -1485,21 +1568,27 @@ bool launch_velocity_bwd(Tile t, int form, const Geom& G, const Groups& F, const
     return false;
   }
   const RingFold Rf = fold_for(G, ring);
+  const RecvFold V = recv_for(recv);
   if (split && has_interior_segments(G)) {
     Sweep rim;
     const Sweep in = split_sweeps(G, t, rim);
     if (form == 1) {
       hipLaunchKernelGGL(k_velocity_bwd_in<1>, grid_of(in), block_of(in), 0, s, in, G, F, C, Rf);
-      hipLaunchKernelGGL((k_velocity_bwd<1, true, 64>), grid_of(rim), block_of(rim), 0, s, rim, G, F, C, Rf);
+      hipLaunchKernelGGL((k_velocity_bwd<1, true, false, 64>), grid_of(rim), block_of(rim), 0, s, rim, G, F, C, Rf, RecvFold{});
     } else {
       hipLaunchKernelGGL(k_velocity_bwd_in<0>, grid_of(in), block_of(in), 0, s, in, G, F, C, Rf);
-      hipLaunchKernelGGL((k_velocity_bwd<0, true, 64>), grid_of(rim), block_of(rim), 0, s, rim, G, F, C, Rf);
+      hipLaunchKernelGGL((k_velocity_bwd<0, true, false, 64>), grid_of(rim), block_of(rim), 0, s, rim, G, F, C, Rf, RecvFold{});
     }
     return Rf.slot != nullptr;
   }
   const Sweep Sw = sweep_flat(G, t);
-  if (form == 1) EFWI_FLAT(Sw, k_velocity_bwd<1 EFWI_COMMA true EFWI_COMMA, Sw, G, F, C, Rf);
-  else EFWI_FLAT(Sw, k_velocity_bwd<0 EFWI_COMMA true EFWI_COMMA, Sw, G, F, C, Rf);
+  if (V.row) {
+    if (form == 1) EFWI_FLAT(Sw, k_velocity_bwd<1 EFWI_COMMA true EFWI_COMMA true EFWI_COMMA, Sw, G, F, C, Rf, V);
+    else EFWI_FLAT(Sw, k_velocity_bwd<0 EFWI_COMMA true EFWI_COMMA true EFWI_COMMA, Sw, G, F, C, Rf, V);
+  } else {
+    if (form == 1) EFWI_FLAT(Sw, k_velocity_bwd<1 EFWI_COMMA true EFWI_COMMA false EFWI_COMMA, Sw, G, F, C, Rf, V);
+    else EFWI_FLAT(Sw, k_velocity_bwd<0 EFWI_COMMA true EFWI_COMMA false EFWI_COMMA, Sw, G, F, C, Rf, V);
+  }
   return Rf.slot != nullptr;
 }
 bool launch_stress_bwd(Tile t, const Geom& G, const Groups& F, const Prof& C, const Source& S, int it,
@@ -1548,8 +1637,8 @@ bool launch_fwd_fused(int R, int zc, int form, const Geom& G, const Groups& Fi, 
 void launch_velocity_adj(int form, const Geom& G, const Groups& F, const Prof& C, hipStream_t s) {
   const Sweep Sw = sweep_flat(G, Tile{1, 1});
   const RingFold none = fold_for(G, nullptr);
-  if (form == 1) EFWI_FLAT(Sw, k_velocity_bwd<1 EFWI_COMMA false EFWI_COMMA, Sw, G, F, C, none);
-  else EFWI_FLAT(Sw, k_velocity_bwd<0 EFWI_COMMA false EFWI_COMMA, Sw, G, F, C, none);
+  if (form == 1) EFWI_FLAT(Sw, k_velocity_bwd<1 EFWI_COMMA false EFWI_COMMA false EFWI_COMMA, Sw, G, F, C, none, RecvFold{});
+  else EFWI_FLAT(Sw, k_velocity_bwd<0 EFWI_COMMA false EFWI_COMMA false EFWI_COMMA, Sw, G, F, C, none, RecvFold{});
 }
 void launch_stress_adj(const Geom& G, const Groups& F, const Prof& C, hipStream_t s) {
   const Sweep Sw = sweep_flat(G, Tile{1, 1});

@@ -50,3 +50,25 @@ def test_two_rows_per_wavefront(orc, ny, formulation):
     w = synth.small(n=69 - 2 * npml, npml=npml, nt=24, ny=ny - 2 * npml, formulation=formulation)
     assert w.grid.shape == (69, 69, ny)
     _check(orc, w)
+
+
+def test_folded_receivers(orc):
+    """Receivers in the velocity kernels: several in one cell, in the C-PML, on
+    the first and last cells of the stencil box, at 64-cell segment edges."""
+    from efwi import synth
+    w = synth.small(n=24, npml=6, nt=60, ny=68)
+    nz, nx, ny = w.grid.shape
+    assert ny == 80
+    rec = [(8, 8, y) for y in (2, 5, 31, 32, 63, 64, ny - 3)] + [(2, 2, 2), (nz - 3, nx - 3, ny - 3), (2, nx - 3, 40)]
+    rec += [(9, 10, 40)] * 3 + [(8, 8, 63)]
+    w.shots[0].rec = np.array(rec, np.int32)
+    _check(orc, w)
+
+
+def test_receivers_outside_the_stencil_box(orc):
+    """One receiver on the outermost cells sends the shot's receivers to the gather and scatter launches."""
+    from efwi import synth
+    w = synth.small(n=24, npml=6, nt=60)
+    nz, nx, ny = w.grid.shape
+    w.shots[0].rec = np.array([(8, 8, 8), (10, 12, 20), (1, 8, 8), (8, nx - 2, 8), (8, 8, ny - 1)], np.int32)
+    _check(orc, w)
