@@ -1,9 +1,10 @@
 // Batched shots: several shots of one grid and model advanced together. Every
-// stencil step of all shots is one persistent launch over a (shot, tile) work
-// queue (efwi_stencil.hip), the receiver, ring and injection work of all
-// shots one launch each, and each time step's launch sequence is captured
-// once in a hipGraph and replayed nt - 1 times with the time step kept in
-// device memory. Per shot the arithmetic is that of efwi_run_shot in the
+// stencil step of a group of shots is one launch over their (shot, tile) items
+// (efwi_stencil.hip: a workgroup each, or persistent workgroups on a work queue
+// with efwi_batch_config), the ring, and where the velocity kernels do not take
+// them the receiver and injection work, of all shots one launch each, and
+// kGraphSteps time steps are captured once in a hipGraph and replayed with the
+// time step kept in device memory. Per shot the arithmetic is that of efwi_run_shot in the
 // reverse-reconstruction mode (memory_mode 0), so each shot's seismograms,
 // misfit and gradient equal a single-shot run's bit for bit.
 #include <algorithm>
@@ -14,6 +15,8 @@
 
 namespace efwi {
 
+static constexpr int kGraphSteps = 16;  // time steps per captured graph
+
 void Ctx::release_batch() {
   if (batch.gf) hipGraphExecDestroy(batch.gf);
   if (batch.gb) hipGraphExecDestroy(batch.gb);
@@ -22,21 +25,30 @@ void Ctx::release_batch() {
   batch.cs = nullptr;
 }
 
-// Shots per persistent launch, or 0: one shot after another through the
-// single-shot kernels. The persistent launches pay for their work queue (an
-// atomic claim per few tiles) and, over many shots, lose the Infinity Cache
-// reuse between consecutive kernels that a single shot has; they win where a
-// shot alone leaves the device idle. Automatic (group = 0): where one shot
-// already gives kBatchFill workgroup tiles per compute unit, the single-shot
-// kernels; otherwise groups of enough shots to reach that many tiles.
-int Ctx::batch_group_size(int n) const {
+// Shots per launch, or 0: one shot after another through the single-shot
+// kernels. Automatic (group = 0): a launch over several shots fills the device
+// where one shot alone does not, until the group's state (kStateFields arrays
+// per shot) no longer stays in the 256 MB Infinity Cache between consecutive
+// kernels: groups of as many shots as kGroupBytes of state, evenly split, and
+// the single-shot kernels where that is one. Gradients of n shots by group size, ms:
+// 44^3 cells (21 MB a shot, n = 12): single 43.9, 3: 27.0, 6: 22.6, 12: 19.9;
+// 72^3 (84 MB, n = 8): single 55.5, 2: 48.9, 4: 46.2, 8: 52.5; 84^3 (114 MB, n = 8):
+// single 67.2, 2: 60.3, 3: 60.1, 4: 64.8; 84x104x104 (188 MB, n = 6): single
+// 44.0, 2: 42.7, 3: 49.4; 84x140x140 (277 MB, n = 4): single 31.2, 2: 36.1. The
+// boundary rings of a group (one per shot) take at most half of the free memory.
+int Ctx::batch_group_size(int n, bool grad) const {
   if (batch.group > 0) return std::min(batch.group, n);
   if (batch.group < 0) return 0;
-  const Tile t = tiles[K_STRESS_FWD].zdepth >= 16 ? Tile{4, 1} : tiles[K_STRESS_FWD];
-  const long per_shot = flat_blocks(G, t);
-  const long want = (long)kBatchFill * std::max(batch.cus, 1);
-  if (per_shot >= want) return 0;
-  return (int)std::max(1L, std::min((long)n, (want + per_shot - 1) / std::max(per_shot, 1L)));
+  long fit = (long)(kGroupBytes / ((double)G.fs * kStateFields));
+  if (grad && fit > 1) {
+    size_t free_b = 0, total_b = 0;
+    const double ring_b = (double)B.n * 9 * (cfg.nt - 1) * sizeof(float);
+    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) free_b = 0;
+    fit = std::min(fit, (long)std::max((double)batch.ring.size(), 0.5 * (double)free_b / ring_b));
+  }
+  if (fit < 2) return 0;
+  const int groups = (int)((n + fit - 1) / fit);
+  return (n + groups - 1) / groups;
 }
 
 // Point the context's state (wavefields, C-PML arrays, model and gradients)
@@ -82,6 +94,7 @@ int Ctx::ensure_batch(int n, int nring) {
     batch.obs_t.push_back(nullptr);
     batch.res_t.push_back(nullptr);
     batch.rec.push_back(nullptr);
+    batch.recv.push_back(RecvMap{});
     batch.seis_cap.push_back(0);
     batch.rec_cap.push_back(0);
     batch.nrec.push_back(0);
@@ -105,7 +118,7 @@ int Ctx::run_batch(const efwi_shot* shots, int n, int calc_id, const float* cons
     int rc0 = ensure_batch(0, 0);
     if (rc0) return rc0;
   }
-  const int gsz0 = batch_group_size(n);
+  const int gsz0 = batch_group_size(n, calc_id == EFWI_CALC_GRADIENT);
   const int gsz = gsz0 > 0 ? gsz0 : 1;
   int rc = ensure_batch(n, calc_id == EFWI_CALC_GRADIENT && gsz0 > 0 ? gsz : 0);
   if (rc) return rc;
@@ -140,6 +153,8 @@ int Ctx::run_batch(const efwi_shot* shots, int n, int calc_id, const float* cons
     const size_t nrb = (size_t)std::max(nrec_k, 1);
     if ((rc = grow(this, (void**)&batch.rec[k], &batch.rec_cap[k], sizeof(long) * nrb))) return rc;
     if (nrec_k) HIP_TRY(hipMemcpy(batch.rec[k], cells.data(), sizeof(long) * nrec_k, hipMemcpyHostToDevice));
+    batch.recv[k].on = false;
+    if (gsz0 > 0 && (rc = map_receivers(sh, batch.recv[k]))) return rc;
     const size_t seis = sizeof(float) * (size_t)nt * 3 * nrb;
     if (batch.seis_cap[k] < seis) {
       size_t c1 = batch.seis_cap[k], c2 = batch.seis_cap[k], c3 = batch.seis_cap[k];
@@ -161,6 +176,15 @@ int Ctx::run_batch(const efwi_shot* shots, int n, int calc_id, const float* cons
     d.syn_t = batch.syn_t[k];
     d.res_t = batch.res_t[k];
     d.ring = calc_id == EFWI_CALC_GRADIENT && gsz0 > 0 ? batch.ring[k % gsz] : nullptr;
+  }
+  // receivers in the velocity kernels where every shot's can be
+  bool fold_rec = recv_foldable(Tile{1, 1}, G, true) && (!grad || recv_foldable(Tile{1, 1}, G, false));
+  for (int k = 0; k < n; k++) fold_rec = fold_rec && (batch.recv[k].on || batch.nrec[k] == 0);
+  for (int k = 0; k < n; k++) {
+    const RecvFold v = fold_rec ? batch.recv[k].fold(batch.nrec[k]) : RecvFold{};
+    tab[k].rrow = v.row;
+    tab[k].rtab = v.tab;
+    tab[k].rnext = v.next;
   }
   HIP_TRY(hipMemcpy(batch.shots_dev, tab.data(), sizeof(ShotDev) * n, hipMemcpyHostToDevice));
   // ---- state: the model into every shot's model group, zero wavefields and gradients
@@ -200,17 +224,26 @@ int Ctx::run_batch(const efwi_shot* shots, int n, int calc_id, const float* cons
   const int gn = std::min(gsz, n - g0);
   int gmax_nrec = 0;
   for (int k = g0; k < g0 + gn; k++) gmax_nrec = std::max(gmax_nrec, batch.nrec[k]);
-  BatchLaunch L0{batch.shots_dev + g0, gn, batch.counters, batch.it_dev, batch.cus, batch.take, batch.static_pct, 0};
+  const bool queue = batch.static_pct >= 0;
+  BatchLaunch L0{batch.shots_dev + g0, gn, batch.counters, nullptr, 0, batch.cus, batch.take, batch.static_pct, 0};
   BatchLaunch L1 = L0;
   L1.counters = batch.counters + 8 * kQueueStride;
   L1.reverse = 1;
+  auto at = [](BatchLaunch L, const int* itp, int off) {
+    L.it = itp;
+    L.off = off;
+    return L;
+  };
+  auto clear = [&](const BatchLaunch& L, hipStream_t st) {
+    if (queue) launch_fill(reinterpret_cast<float*>(L.counters), 8 * kQueueStride, 0.0f, st);
+  };
   const std::string tiles_key = std::to_string(tiles[K_STRESS_FWD].rows) + "x" + std::to_string(tiles[K_STRESS_FWD].zdepth) +
                                 "," + std::to_string(tiles[K_VELOCITY_FWD].rows) + "x" + std::to_string(tiles[K_VELOCITY_FWD].zdepth) +
                                 "," + std::to_string(tiles[K_VELOCITY_BWD].rows) + "x" + std::to_string(tiles[K_VELOCITY_BWD].zdepth) +
                                 "," + std::to_string(tiles[K_STRESS_BWD].rows) + "x" + std::to_string(tiles[K_STRESS_BWD].zdepth);
   const std::string key = std::to_string(n) + "|" + std::to_string(g0) + "+" + std::to_string(gn) + "|" +
                           std::to_string(gmax_nrec) + "|" + tiles_key + "|" +
-                          std::to_string(batch.take) + "|" + std::to_string(batch.static_pct) + "|";
+                          std::to_string(batch.take) + "|" + std::to_string(batch.static_pct) + (fold_rec ? "|r" : "|");
   // ---- forward loop (Src/libCUFD.cu:312-354 per shot): ring save of the
   // state before step it, stress + source, velocity, record of step it + 1.
   // With the ring folded, the stencil kernels of step it save the state they
@@ -222,40 +255,44 @@ int Ctx::run_batch(const efwi_shot* shots, int n, int calc_id, const float* cons
   save.last = nt - 2;
   BatchRing restore = save;
   restore.mode = 2;
-  auto fwd_step = [&](hipStream_t st) {
-    if (grad && !fold) launch_ring_batch(B, G, batch.shots_dev + g0, gn, batch.it_dev, 0, 9, 0, st);
-    launch_fill(reinterpret_cast<float*>(batch.counters), 8 * kQueueStride, 0.0f, st);
-    launch_stress_fwd_batch(tiles[K_STRESS_FWD], G, C, L0, st, fold ? &save : nullptr);
-    launch_fill(reinterpret_cast<float*>(batch.counters + 8 * kQueueStride), 8 * kQueueStride, 0.0f, st);
-    launch_velocity_fwd_batch(tiles[K_VELOCITY_FWD], form, G, C, L1, st, fold ? &save : nullptr);
-    launch_record_batch(batch.shots_dev + g0, gn, gmax_nrec, batch.it_dev, 1, st);
-    launch_step_add(batch.it_dev, 1, st);
+  // one forward step: time step (itp ? *itp : 0) + off
+  auto fwd_step = [&](hipStream_t st, const int* itp, int off) {
+    if (grad && !fold) launch_ring_batch(B, G, batch.shots_dev + g0, gn, itp, off, 0, 9, 0, st);
+    clear(L0, st);
+    launch_stress_fwd_batch(tiles[K_STRESS_FWD], G, C, at(L0, itp, off), st, fold ? &save : nullptr);
+    clear(L1, st);
+    launch_velocity_fwd_batch(tiles[K_VELOCITY_FWD], form, G, C, at(L1, itp, off), st, fold ? &save : nullptr);
+    if (!fold_rec) launch_record_batch(batch.shots_dev + g0, gn, gmax_nrec, itp, off + 1, st);
   };
-  auto run_steps = [&](hipGraphExec_t* exec, std::string* have, const std::string& want, int count,
+  // `count` steps from time step `start`, `dir` apart: kGraphSteps at a time
+  // as a captured graph (its nodes take the step from a device counter, which
+  // the last one advances), the rest launched directly
+  auto run_steps = [&](hipGraphExec_t* exec, std::string* have, const std::string& want, int start, int dir, int count,
                        auto&& step) -> int {
-    if (!use_graph) {
-      for (int i = 0; i < count; i++) step(q);
-      return EFWI_OK;
+    constexpr int U = kGraphSteps;
+    const int replays = use_graph ? count / U : 0;
+    if (replays > 0) {
+      if (*exec == nullptr || *have != want) {
+        if (*exec) HIP_TRY(hipGraphExecDestroy(*exec));
+        *exec = nullptr;
+        hipGraph_t g = nullptr;
+        HIP_TRY(hipStreamBeginCapture(q, hipStreamCaptureModeThreadLocal));
+        for (int i = 0; i < U; i++) step(q, batch.it_dev, dir * i);
+        launch_step_add(batch.it_dev, dir * U, q);
+        HIP_TRY(hipStreamEndCapture(q, &g));
+        hipError_t e = hipGraphInstantiate(exec, g, nullptr, nullptr, 0);
+        hipGraphDestroy(g);
+        if (e != hipSuccess) return fail(EFWI_ERR_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
+        *have = want;
+      }
+      HIP_TRY(hipMemcpyAsync(batch.it_dev, &start, sizeof(int), hipMemcpyHostToDevice, q));
+      for (int i = 0; i < replays; i++) HIP_TRY(hipGraphLaunch(*exec, q));
     }
-    if (*exec == nullptr || *have != want) {
-      if (*exec) HIP_TRY(hipGraphExecDestroy(*exec));
-      *exec = nullptr;
-      hipGraph_t g = nullptr;
-      HIP_TRY(hipStreamBeginCapture(q, hipStreamCaptureModeThreadLocal));
-      step(q);
-      HIP_TRY(hipStreamEndCapture(q, &g));
-      hipError_t e = hipGraphInstantiate(exec, g, nullptr, nullptr, 0);
-      hipGraphDestroy(g);
-      if (e != hipSuccess) return fail(EFWI_ERR_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
-      *have = want;
-    }
-    for (int i = 0; i < count; i++) HIP_TRY(hipGraphLaunch(*exec, q));
+    for (int i = replays * U; i < count; i++) step(q, nullptr, start + dir * i);
     return EFWI_OK;
   };
-  const int zero = 0;
-  HIP_TRY(hipMemcpyAsync(batch.it_dev, &zero, sizeof(int), hipMemcpyHostToDevice, q));
-  if (fold) launch_ring_batch(B, G, batch.shots_dev + g0, gn, batch.it_dev, 0, 9, 0, q);
-  if ((rc = run_steps(&batch.gf, &batch.key_f, key + (grad ? "g" : "f"), nt - 1, fwd_step))) return rc;
+  if (fold) launch_ring_batch(B, G, batch.shots_dev + g0, gn, nullptr, 0, 0, 9, 0, q);
+  if ((rc = run_steps(&batch.gf, &batch.key_f, key + (grad ? "g" : "f"), 0, 1, nt - 1, fwd_step))) return rc;
   HIP_TRY(hipGetLastError());
   for (int k = g0; k < g0 + gn; k++)
     if (syn && syn[k] && batch.nrec[k] > 0) launch_from_time_major(batch.syn_t[k], syn[k], batch.nrec[k], nt, q);
@@ -286,19 +323,16 @@ int Ctx::run_batch(const efwi_shot* shots, int n, int calc_id, const float* cons
       launch_inject(Ak, batch.rec[k], batch.nrec[k], nt - 1, batch.res_t[k], q);
       launch_stress_adj(G, g, C, q);
     }
-    auto bwd_step = [&](hipStream_t st) {
-      launch_fill(reinterpret_cast<float*>(batch.counters), 8 * kQueueStride, 0.0f, st);
-      launch_velocity_bwd_batch(tiles[K_VELOCITY_BWD], form, G, C, L0, st, fold ? &restore : nullptr);
-      if (!fold) launch_ring_batch(B, G, batch.shots_dev + g0, gn, batch.it_dev, 0, 3, 1, st);
-      launch_inject_batch(batch.shots_dev + g0, gn, gmax_nrec, batch.it_dev, st);
-      launch_fill(reinterpret_cast<float*>(batch.counters + 8 * kQueueStride), 8 * kQueueStride, 0.0f, st);
-      launch_stress_bwd_batch(tiles[K_STRESS_BWD], G, C, L1, st, fold ? &restore : nullptr);
-      if (!fold) launch_ring_batch(B, G, batch.shots_dev + g0, gn, batch.it_dev, 3, 9, 1, st);
-      launch_step_add(batch.it_dev, -1, st);
+    auto bwd_step = [&](hipStream_t st, const int* itp, int off) {
+      clear(L0, st);
+      launch_velocity_bwd_batch(tiles[K_VELOCITY_BWD], form, G, C, at(L0, itp, off), st, fold ? &restore : nullptr);
+      if (!fold) launch_ring_batch(B, G, batch.shots_dev + g0, gn, itp, off, 0, 3, 1, st);
+      if (!fold_rec) launch_inject_batch(batch.shots_dev + g0, gn, gmax_nrec, itp, off, st);
+      clear(L1, st);
+      launch_stress_bwd_batch(tiles[K_STRESS_BWD], G, C, at(L1, itp, off), st, fold ? &restore : nullptr);
+      if (!fold) launch_ring_batch(B, G, batch.shots_dev + g0, gn, itp, off, 3, 9, 1, st);
     };
-    const int start = nt - 2;
-    HIP_TRY(hipMemcpyAsync(batch.it_dev, &start, sizeof(int), hipMemcpyHostToDevice, q));
-    if ((rc = run_steps(&batch.gb, &batch.key_b, key + "b", nt - 1, bwd_step))) return rc;
+    if ((rc = run_steps(&batch.gb, &batch.key_b, key + "b", nt - 2, -1, nt - 1, bwd_step))) return rc;
     HIP_TRY(hipGetLastError());
   }
   }  // groups of shots

@@ -63,6 +63,7 @@ struct BatchState {
   std::vector<Groups> F;
   std::vector<float*> ring, stf, syn_t, obs_t, res_t;
   std::vector<long*> rec;
+  std::vector<RecvMap> recv;
   std::vector<size_t> seis_cap, rec_cap;
   std::vector<int> nrec;
   ShotDev* shots_dev = nullptr;
@@ -73,7 +74,7 @@ struct BatchState {
   std::string key_f, key_b;
   int cus = 0;
   int take = 2;        // queue items per atomic (efwi_batch_config)
-  int static_pct = 0;  // static share of the queues, percent
+  int static_pct = -1;  // static share of the queues, percent; -1: no queue, one workgroup per tile
   int group = 0;       // shots per persistent launch (efwi_batch_group), 0 = automatic
 };
 
@@ -172,8 +173,10 @@ struct Ctx {
   int autotune(int reps, hipStream_t s, double* report);
   // batched shots (efwi_batch.cpp)
   BatchState batch;
-  static constexpr int kBatchFill = 16;  // automatic groups: workgroup tiles per CU and launch
-  int batch_group_size(int n) const;
+  // automatic groups: state bytes of a launch's shots, arrays per shot
+  static constexpr double kGroupBytes = 384e6;
+  static constexpr int kStateFields = 2 * F_WAVE_COUNT + P_PSI_COUNT + M_COUNT;
+  int batch_group_size(int n, bool grad) const;
   void bind_state(const Groups& g);
   int ensure_batch(int n, int nring);
   int run_batch(const efwi_shot* shots, int n, int calc_id, const float* const* obs, float* const* syn,

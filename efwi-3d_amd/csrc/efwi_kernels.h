@@ -40,8 +40,6 @@ struct Sweep {
   int sk_z0, sk_z1, sk_x0, sk_x1, sk_y0, sk_y1;
   long blocks;
 };
-// Workgroups of a flat forward launch of shape t on the grid's stencil box.
-long flat_blocks(const Geom& G, Tile t);
 
 // Fused forward step (stress + velocity of one time step in one launch):
 // workgroups of 64 x (R + 4) threads own R x rows of 60 y cells and Zc z
@@ -104,10 +102,11 @@ bool launch_fwd_fused(int R, int zc, int form, const Geom& G, const Groups& Fi, 
 void launch_velocity_adj(int form, const Geom& G, const Groups& F, const Prof& C, hipStream_t s);
 void launch_stress_adj(const Geom& G, const Groups& F, const Prof& C, hipStream_t s);
 
-// batched persistent stencil kernels: one launch covers the (shot, tile) items
-// of all shots of L, with the flat sweep's tiles (t.zdepth < 16).
+// batched stencil kernels: one launch covers the (shot, tile) items of all
+// shots of L, with the flat sweep's tiles (t.zdepth < 16), one workgroup per
+// item or (L.stat >= 0) persistent workgroups on a work queue.
 // A BatchRing folds each shot's boundary ring (ShotDev::ring) into them, the
-// slot following the launch's device step it: mode 1 (forward kernels) saves
+// slot following the launch's step it: mode 1 (forward kernels) saves
 // the state they produce into slot it + 1 while it + 1 <= last, mode 2
 // (backward kernels) restores slot it. Callers pass one only where
 // ring_foldable holds.
@@ -153,10 +152,10 @@ void launch_vp2max(const Geom& G, const float* lam, const float* mu, const float
 // FP64 dot product of float vectors; returns the number of partials written.
 int launch_dot64(const float* a, const float* b, long n, double* partials, int max_blocks, hipStream_t s);
 // batched per-step aux kernels of the shot table (time step read on the device)
-void launch_record_batch(const ShotDev* shots, int nshots, int max_nrec, const int* it, int it_offset,
-                         hipStream_t s);
-void launch_inject_batch(const ShotDev* shots, int nshots, int max_nrec, const int* it, hipStream_t s);
-void launch_ring_batch(const Band& B, const Geom& G, const ShotDev* shots, int nshots, const int* it, int k0,
+// (step = (it ? *it : 0) + off)
+void launch_record_batch(const ShotDev* shots, int nshots, int max_nrec, const int* it, int off, hipStream_t s);
+void launch_inject_batch(const ShotDev* shots, int nshots, int max_nrec, const int* it, int off, hipStream_t s);
+void launch_ring_batch(const Band& B, const Geom& G, const ShotDev* shots, int nshots, const int* it, int off, int k0,
                        int k1, int restore, hipStream_t s);
 void launch_step_add(int* it, int delta, hipStream_t s);
 // [3][nrec][nt] <-> [nt][3][nrec]

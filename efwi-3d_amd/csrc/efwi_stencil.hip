@@ -1243,13 +1243,14 @@ __global__ __launch_bounds__(64 * (R + 4)) void k_fwd_fused(FusedSweep S, Geom G
 }
 
 // ---------------------------------------------------------------------------
-// Batched shots: one persistent launch per stencil step covers every (shot,
-// tile) item of the batch. Items are the flat sweep's workgroup tiles; those of
-// XCD strip q (tile index b with b % 8 == q) of every shot form queue q. A
-// workgroup drains the queue of the XCD it runs on (hardware register
-// XCC_ID), taking `take` consecutive items per atomic, then steals from the
-// other queues, so every item is processed once whatever the placement. The time step is
-// read from device memory, so a captured step replays unchanged.
+// Batched shots: one launch per stencil step covers every (shot, tile) item of
+// a group of shots. Items are the flat sweep's workgroup tiles; captured steps
+// read the time step from device memory, so that they replay unchanged. In the
+// work-queue form (efwi_batch_config) the items of XCD strip q (tile index b
+// with b % 8 == q) of every shot form queue q. A persistent workgroup drains the
+// queue of the XCD it runs on (hardware register XCC_ID), taking `take`
+// consecutive items per atomic, then steals from the other queues, so every
+// item is processed once whatever the placement.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ int xcc_id() {
   // s_getreg_b32 hwreg(HW_REG_XCC_ID, 0, 4): bits [3:0] hold the XCC of the wave
@@ -1312,8 +1313,9 @@ __device__ __forceinline__ void persistent_items(const BatchLaunch& L, int per_x
   }
 }
 
-__device__ __forceinline__ int device_step(const int* it) {
-  return __builtin_amdgcn_readfirstlane(__hip_atomic_load(it, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+__device__ __forceinline__ int device_step(const BatchLaunch& L) {
+  if (!L.it) return L.off;
+  return __builtin_amdgcn_readfirstlane(__hip_atomic_load(L.it, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) + L.off;
 }
 
 // The shot table is read with vector loads (the compiler cannot prove that the
@@ -1331,58 +1333,105 @@ __device__ __forceinline__ long uniform_long(long x) {
   return (long)(unsigned long long)uniform_ptr((char*)x);
 }
 
-// KIND: 0 stress_fwd, 1 velocity_fwd, 2 velocity_bwd, 3 stress_bwd
-template <int KIND, int FORM, int LY>
-__global__ __launch_bounds__(256) void k_batch(Sweep Sw, Geom G, Prof C, BatchLaunch L, int per_xcd, BatchRing R) {
-  const int it = device_step(L.it);
+// What a batched kernel needs of one shot. KIND: 0 stress_fwd, 1 velocity_fwd,
+// 2 velocity_bwd, 3 stress_bwd.
+struct ShotItem {
+  Groups F;
+  Source S;
+  RingFold Rf;
+  RecvFold V;
+};
+template <int KIND>
+__device__ __forceinline__ ShotItem shot_item(const ShotDev& sd, int it, const BatchRing& R) {
+  ShotItem q{};
+  q.F.w = uniform_ptr(sd.F.w);
+  q.F.a = uniform_ptr(sd.F.a);
+  q.F.p = uniform_ptr(sd.F.p);
+  q.F.m = uniform_ptr(sd.F.m);
+  if (KIND == 0 || KIND == 3) {
+    q.S.cell = uniform_long(sd.cell);
+    q.S.stf = uniform_ptr(sd.stf);
+  }
   // ring slot of this step (the same index in every shot's ring), or none
   const int slot = R.mode == 1 ? it + 1 : it;
   const bool ring_on = R.mode == 2 || (R.mode == 1 && slot <= R.last);
+  q.Rf.B = R.B;
+  q.Rf.slot = ring_on ? uniform_ptr(sd.ring) + (long)slot * 9 * R.B.n : nullptr;
+  if (KIND == 1 || KIND == 2) {
+    q.V.row = uniform_ptr(sd.rrow);
+    if (q.V.row) {
+      q.V.tab = uniform_ptr(sd.rtab);
+      q.V.next = uniform_ptr(sd.rnext);
+      q.V.nrec = __builtin_amdgcn_readfirstlane(sd.nrec);
+      const long o = 3L * q.V.nrec;
+      q.V.out = uniform_ptr(sd.syn_t) + (it + 1) * o;
+      q.V.res = uniform_ptr(sd.res_t) + it * o;
+    }
+  }
+  return q;
+}
+// Workgroup tile b of one shot.
+template <int KIND, int FORM, int LY>
+__device__ __forceinline__ void batch_tile(const Sweep& Sw, const Geom& G, const Prof& C, const ShotItem& q, int it,
+                                           int b) {
+  if constexpr (KIND == 0) {
+    const unsigned so = source_off(q.S);
+    const float amp = source_amp(q.S, G, it);
+    sweep_block<LY>(Sw, G, b, [&](const Cell& c) { stress_fwd_cell(G, save_acc(G, q.F, q.Rf, c), C, c, so, amp); });
+  } else if constexpr (KIND == 1) {
+    sweep_block<LY>(Sw, G, b, [&](const Cell& c) { velocity_fwd_cell<FORM>(G, save_acc(G, q.F, q.Rf, c, q.V), C, c); });
+  } else if constexpr (KIND == 2) {
+    sweep_block<LY>(Sw, G, b, [&](const Cell& c) {
+      const InjectAcc acc = inject_acc(G, q.F, c, q.V);
+      const RingRestore<F_VZ, F_VY + 1> rr(q.Rf, c);
+      by_slabs(G, c, [&](auto X, auto Z, auto Y) {
+        velocity_bwd_cell<FORM, true, decltype(X)::value, decltype(Z)::value, decltype(Y)::value>(G, acc, C, c);
+      });
+      rr.store(acc);
+    });
+  } else {
+    const unsigned so = source_off(q.S);
+    const float amp = source_amp(q.S, G, it);
+    sweep_block<LY>(Sw, G, b, [&](const Cell& c) {
+      const FlatAcc acc = flat_acc(G, q.F, c);
+      const RingRestore<F_SZZ, F_WAVE_COUNT> rr(q.Rf, c);
+      by_slabs(G, c, [&](auto X, auto Z, auto Y) {
+        stress_bwd_cell<true, decltype(X)::value, decltype(Z)::value, decltype(Y)::value>(G, acc, C, c, so, amp);
+      });
+      rr.store(acc);
+    });
+  }
+}
+
+// Work queue: persistent workgroups claim (shot, tile) items.
+template <int KIND, int FORM, int LY>
+__global__ __launch_bounds__(256) void k_batch(Sweep Sw, Geom G, Prof C, BatchLaunch L, int per_xcd, BatchRing R) {
+  const int it = device_step(L);
   int have = -1;
-  Groups F{};
-  Source S{};
-  RingFold Rf{};
-  Rf.B = R.B;
+  ShotItem q{};
   persistent_items(L, per_xcd, [&](int shot, int b) {
     if (shot != have) {  // consecutive items mostly belong to one shot
-      const ShotDev& sd = L.shots[shot];
-      F.w = uniform_ptr(sd.F.w);
-      F.a = uniform_ptr(sd.F.a);
-      F.p = uniform_ptr(sd.F.p);
-      F.m = uniform_ptr(sd.F.m);
-      S.cell = uniform_long(sd.cell);
-      S.stf = uniform_ptr(sd.stf);
-      Rf.slot = ring_on ? uniform_ptr(sd.ring) + (long)slot * 9 * R.B.n : nullptr;
+      q = shot_item<KIND>(L.shots[shot], it, R);
       have = shot;
     }
-    if constexpr (KIND == 0) {
-      const unsigned so = source_off(S);
-      const float amp = source_amp(S, G, it);
-      sweep_block<LY>(Sw, G, b, [&](const Cell& c) { stress_fwd_cell(G, save_acc(G, F, Rf, c), C, c, so, amp); });
-    } else if constexpr (KIND == 1) {
-      sweep_block<LY>(Sw, G, b, [&](const Cell& c) { velocity_fwd_cell<FORM>(G, save_acc(G, F, Rf, c), C, c); });
-    } else if constexpr (KIND == 2) {
-      sweep_block<LY>(Sw, G, b, [&](const Cell& c) {
-        const FlatAcc acc = flat_acc(G, F, c);
-            const RingRestore<F_VZ, F_VY + 1> rr(Rf, c);
-        by_slabs(G, c, [&](auto X, auto Z, auto Y) {
-          velocity_bwd_cell<FORM, true, decltype(X)::value, decltype(Z)::value, decltype(Y)::value>(G, acc, C, c);
-        });
-        rr.store(acc);
-      });
-    } else {
-      const unsigned so = source_off(S);
-      const float amp = source_amp(S, G, it);
-      sweep_block<LY>(Sw, G, b, [&](const Cell& c) {
-        const FlatAcc acc = flat_acc(G, F, c);
-            const RingRestore<F_SZZ, F_WAVE_COUNT> rr(Rf, c);
-        by_slabs(G, c, [&](auto X, auto Z, auto Y) {
-          stress_bwd_cell<true, decltype(X)::value, decltype(Z)::value, decltype(Y)::value>(G, acc, C, c, so, amp);
-        });
-        rr.store(acc);
-      });
-    }
+    batch_tile<KIND, FORM, LY>(Sw, G, C, q, it, b);
   });
+}
+
+// One workgroup per (tile, shot): blockIdx.x is the tile (a multiple of 8 of
+// them, so that a tile stays on the XCD of its strip), blockIdx.y the shot.
+// The tiles are alike, so the hardware's dispatch balances them as well as a
+// queue does and without its costs (two fills, an atomic claim and a look at
+// the other seven XCDs' heads, one after another, per workgroup: 35-42 us per
+// launch of 4800 tiles of 44^3 cells where the tiles take 15). 12 shots of
+// 44^3 cells, 119 steps: 89 ms in the queue's former groups of 3, 42 ms in one
+// group of 12, and 20 ms here.
+template <int KIND, int FORM, int LY>
+__global__ __launch_bounds__(256) void k_batch_flat(Sweep Sw, Geom G, Prof C, BatchLaunch L, BatchRing R) {
+  const int it = device_step(L);
+  const int k = (int)blockIdx.y;
+  const ShotItem q = shot_item<KIND>(L.shots[L.reverse ? L.nshots - 1 - k : k], it, R);
+  batch_tile<KIND, FORM, LY>(Sw, G, C, q, it, (int)blockIdx.x);
 }
 
 }  // namespace
@@ -1432,7 +1481,6 @@ static inline Sweep sweep_flat(const Geom& G, Tile t) {
   const long waves = (long)(G.nz - 4) * (G.nx - 4) * a.nyb;
   return 8 * 32 * b.nyb <= 7 * 64 * a.nyb && waves >= 16 * 256 ? b : a;
 }
-long flat_blocks(const Geom& G, Tile t) { return sweep_flat(G, t).blocks; }
 
 static inline dim3 grid_of(const Sweep& S) { return dim3((unsigned)S.blocks); }
 static inline dim3 block_of(const Sweep& S) { return dim3(64, S.R); }
@@ -1700,8 +1748,15 @@ static void launch_batch(Tile t, const Geom& G, const Prof& C, const BatchLaunch
   static int occ[2][8] = {{0}};
   Sweep Sw = sweep_batch(G, t);
   Sw.zrev = L.reverse;  // shots and planes last to first: start where the last launch ended
-  if (Sw.ly == 32) launch_batch(k_batch<KIND, FORM, 32>, occ[0], Sw, G, C, L, s, R);
-  else launch_batch(k_batch<KIND, FORM, 64>, occ[1], Sw, G, C, L, s, R);
+  if (L.stat < 0) {
+    const dim3 grid((unsigned)Sw.blocks, (unsigned)L.nshots);
+    if (Sw.ly == 32) hipLaunchKernelGGL((k_batch_flat<KIND, FORM, 32>), grid, block_of(Sw), 0, s, Sw, G, C, L, R);
+    else hipLaunchKernelGGL((k_batch_flat<KIND, FORM, 64>), grid, block_of(Sw), 0, s, Sw, G, C, L, R);
+  } else if (Sw.ly == 32) {
+    launch_batch(k_batch<KIND, FORM, 32>, occ[0], Sw, G, C, L, s, R);
+  } else {
+    launch_batch(k_batch<KIND, FORM, 64>, occ[1], Sw, G, C, L, s, R);
+  }
 }
 // The caller's ring fold where it applies, else none.
 static inline BatchRing batch_ring(const Geom& G, const BatchRing* ring) {

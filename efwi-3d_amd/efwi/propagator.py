@@ -256,9 +256,9 @@ class Propagator:
         return (None if calc_id == N.CALC_SYNTHETIC else j.value), syn, res
 
     def run_batch(self, shots, calc_id: int, obs=None, want_syn=False, use_graph=True):
-        """All `shots` together: one persistent launch per stencil step over
-        every (shot, tile) item, each time step replayed from a captured
-        hipGraph (use_graph). Returns (misfits, syns): a list of FP64 misfits
+        """All `shots` together: one launch per stencil step over every
+        (shot, tile) item of a group of shots, the time steps replayed from a
+        captured hipGraph (use_graph). Returns (misfits, syns): a list of FP64 misfits
         (None for calc_id 2) and, when requested, [3][nrec][nt] CUDA tensors.
         calc_id 1 keeps one gradient per shot (batch_gradient)."""
         g = self.grid
@@ -294,16 +294,17 @@ class Propagator:
         return misfits, (syns if (want_syn or calc_id == N.CALC_SYNTHETIC) else None)
 
     def batch_group(self, shots_per_launch: int = 0):
-        """How run_batch runs: groups of this many shots per persistent launch,
-        -1 for one shot after another on the single-shot kernels, 0 for the
-        automatic choice (single-shot kernels where one shot fills the
-        device). Results do not depend on it."""
+        """How run_batch runs: groups of this many shots per launch, -1 for one
+        shot after another on the single-shot kernels, 0 for the automatic
+        choice (as many shots as stay near the Infinity Cache's size). Results
+        do not depend on it."""
         N.check(N.lib().efwi_batch_group(self._h, int(shots_per_launch)), "efwi_batch_group")
 
     def batch_config(self, take: int = 2, static_pct: int = 0):
-        """Work distribution of the batched launches: each persistent workgroup
-        runs static_pct percent of an even share of its XCD's queue, then
-        claims the rest `take` tiles per atomic."""
+        """Run the batched launches from a work queue (without this call every
+        tile is a workgroup of its own): each persistent workgroup runs
+        static_pct percent of an even share of its XCD's queue, then claims
+        the rest `take` tiles per atomic. Results do not depend on it."""
         N.check(N.lib().efwi_batch_config(self._h, int(take), int(static_pct)), "efwi_batch_config")
 
     def batch_gradient(self, shot: int):

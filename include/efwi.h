@@ -182,11 +182,11 @@ int efwi_get_resident_segments(const efwi_ctx* ctx, int* segments, int* total);
 int efwi_set_fusion(efwi_ctx* ctx, int pass, int rows, int zchunk);
 
 /* Batched shots: run `nshots` shots of this grid and model together. Each
- * stencil step of all shots is one persistent launch over a (shot, tile) work
- * queue (per-XCD queues with stealing), the ring, receiver and injection work
- * of all shots one launch each, and with use_graph != 0 each time step's
- * launch sequence is captured once in a hipGraph and replayed (the time step
- * lives in device memory). obs[k] / syn[k] are device arrays [3][nrec_k][nt]
+ * stencil step of a group of shots is one launch over their (shot, tile)
+ * items, the receiver and injection work part of the velocity kernels (or of
+ * all shots one launch each), and with use_graph != 0 sixteen time steps'
+ * launches are captured once in a hipGraph and replayed (the time step lives in
+ * device memory). obs[k] / syn[k] are device arrays [3][nrec_k][nt]
  * (syn may be NULL or hold NULLs); misfits[k] receives shot k's misfit.
  * calc_id 1 keeps a separate gradient per shot (efwi_batch_gradient) and
  * needs the full ring (memory_mode 0 or automatic) for every shot; sources
@@ -196,22 +196,22 @@ int efwi_set_fusion(efwi_ctx* ctx, int pass, int rows, int zchunk);
  * another, Src/libCUFD.cu:237-620). */
 int efwi_run_batch(efwi_ctx* ctx, const efwi_shot* shots, int nshots, int calc_id, const float* const* obs,
                    float* const* syn, double* misfits, int use_graph, void* stream);
-/* Work distribution of the batched stencil launches. Each persistent
- * workgroup first runs a static share of its XCD's queue, static_pct percent
- * (0..100) of an even split, and then claims the rest of the queues, at most
- * `take` tiles per atomic (1..4096; lowered for small batches). Defaults:
- * take 2, static_pct 0. Results do not depend on either. */
+/* Work queue for the batched stencil launches. Without a call, every
+ * (shot, tile) item is a workgroup of its own, which is faster. After it,
+ * persistent workgroups on per-XCD queues with stealing: each first runs a
+ * static share of its XCD's queue, static_pct percent (0..100) of an even
+ * split, and then claims the rest of the queues, at most `take` tiles per
+ * atomic (1..4096; lowered for small batches). Results do not depend on it. */
 int efwi_batch_config(efwi_ctx* ctx, int take, int static_pct);
 /* How efwi_run_batch runs its shots. shots_per_launch > 0: groups of that
- * many shots, one group after another, each group one persistent launch per
- * stencil step over its (shot, tile) queue with its own captured graphs
- * (gradient batches keep a boundary ring per shot of a group only); -1: one
- * shot after another through the single-shot kernels (each shot on its own
- * state, as efwi_run_shot runs it); 0 (default): automatic, the single-shot
- * kernels where one shot already gives 16 workgroup tiles per compute unit
- * (the persistent queue's claims and the lost cache reuse between kernels
- * make it slower there), else groups of enough shots to reach that. Results
- * do not depend on it. */
+ * many shots, one group after another, each group one launch per stencil step
+ * over its (shot, tile) items with its own captured graphs (gradient batches
+ * keep a boundary ring per shot of a group only); -1: one shot after another
+ * through the single-shot kernels (each shot on its own state, as
+ * efwi_run_shot runs it); 0 (default): automatic, groups of as many shots as
+ * keep their state within about 1.5 times the Infinity Cache and their rings
+ * within half of the free memory, the single-shot kernels where that is one.
+ * Results do not depend on it. */
 int efwi_batch_group(efwi_ctx* ctx, int shots_per_launch);
 /* Gradient (lambda, mu, rho) of shot `shot` of the last efwi_run_batch. */
 int efwi_batch_gradient(efwi_ctx* ctx, int shot, float* g_lambda, float* g_mu, float* g_rho, int on_host,

@@ -72,3 +72,31 @@ def test_receivers_outside_the_stencil_box(orc):
     nz, nx, ny = w.grid.shape
     w.shots[0].rec = np.array([(8, 8, 8), (10, 12, 20), (1, 8, 8), (8, nx - 2, 8), (8, 8, ny - 1)], np.int32)
     _check(orc, w)
+
+
+@pytest.mark.parametrize("nt", [18, 33, 40])
+def test_batch_steps_replayed_and_launched(nt):
+    """A batch replays captured graphs of sixteen time steps and launches the
+    rest directly: nt - 1 = one graph and one step, two graphs, two graphs and
+    seven steps, on narrow rows (two per wavefront); equal to single shots."""
+    from efwi import synth
+    from efwi.propagator import Propagator, ShotSpec
+    w = synth.small(n=69 - 12, npml=6, nt=nt, ny=70 - 12)
+    base = w.shots[0]
+    rec = np.array([[9, 20, 30], [9, 20, 30], [10, 2, 2]], np.int32)
+    shots = [base, ShotSpec((12, 30, 40), base.stf, rec), ShotSpec((20, 10, 12), base.stf, rec[:1])]
+    print(f"[gpu] batch grid={w.grid.shape} nt={nt}", flush=True)
+    with Propagator(w.grid) as P:
+        P.set_model(*(torch.from_numpy(a) for a in w.true))
+        obs = [P.run_shot(s, 2)[1] for s in shots]
+        P.set_model(*(torch.from_numpy(a) for a in w.model))
+        mis, syns = P.run_batch(shots, 1, obs, want_syn=True)
+        grads = [P.batch_gradient(k) for k in range(len(shots))]
+        again, _ = P.run_batch(shots, 1, obs)
+        for k, s in enumerate(shots):
+            P.zero_gradient()
+            j, syn, _ = P.run_shot(s, 1, obs[k], want_syn=True)
+            assert mis[k] == j and again[k] == j
+            assert torch.equal(syns[k], syn)
+            for a, b, c in zip(grads[k], P.gradient(), P.batch_gradient(k)):
+                assert torch.equal(a, b) and torch.equal(c, b)
