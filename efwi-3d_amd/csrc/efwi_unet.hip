@@ -386,56 +386,81 @@ __global__ void k_flip_many(FlipSet S) {
   }
 }
 
-// Weight gradient partials on v_mfma_f32_16x16x32_bf16: K = voxels. A block
-// of four wavefronts takes `per` bricks of 2 (z) x 2 (x) rows of TY voxels
-// along y, consecutive along z (bricks are numbered z fastest), one 16-channel
-// block of m and one of n. Per brick it copies into LDS, channel-major (y
-// contiguous, rows padded to TY + 8 so that each 8-lane phase of a fragment
-// read hits distinct banks; 8-byte stores of 4 voxels per channel): dpre of the
-// brick (zero outside the volume) and the brick's src halo (4 planes x 4 rows
-// of TY + 2 voxels) in a ring of four plane slots (plane z in slot z mod 4):
-// a brick that follows its z neighbour in the same block keeps that
-// neighbour's last two halo planes and copies only two new ones. Wavefront w takes output row w and every tap: per 32 voxels it
-// reads one A fragment (A[m][k] = dpre[voxel k][m]) and, per (dz, dx), two
-// 16-byte granules of the halo row from which the three dy shifts of the B
-// fragment (B[k][n] = src[voxel k + d_t][n]) follow by dword selection and
-// byte alignment. The four wavefronts' sums meet in LDS, and the block writes
-// part[chunk][t][m][n] for its m and n blocks. With db, the blocks of the first
-// n block also sum the A fragments they read (dpre over their voxels: the bias
-// gradient of their m block) into part[chunk][27 mc kc + m]; a chunk's
+// Weight gradient partials on v_mfma_f32_16x16x32_bf16: K = voxels. A block of
+// four wavefronts takes `per` bricks of 2 (z) x 2 (x) rows of TY voxels along
+// y, consecutive along x (bricks are numbered x fastest), one 16-channel block
+// of m and one of n. A brick owns its src rows; a src row is multiplied with the
+// 9 dpre rows around it, so the block keeps the dpre rows x0 - 1 .. x0 + 2 of
+// the planes z0 - 1 .. z0 + 2 in an LDS ring of three row pairs (one new pair
+// per brick; the first pair of a column is a step without products) and the
+// brick's four src rows (TY + 2 voxels) in one of two buffers, zero outside the
+// volume. The rows of the next two steps are in flight in registers during a
+// step's products, with one barrier per step. LDS holds the voxels as they are
+// in memory (16 channels, 32 bytes); fragments (8 voxels of one channel per
+// lane) are read with the transposing LDS load: 16 lanes read 4 voxels x 16
+// channels and each gets its channel's 4 values, so lane group g holds voxels
+// 4 g .. 4 g + 3 and 16 + 4 g .. 16 + 4 g + 3 of 32, for dpre and src alike, and
+// a tap's dy is an offset of one voxel. Per src row and 32 voxels a wavefront
+// reads 3 src fragments (dy) and 9 dpre fragments (dz, dx) for 27 products:
+// 12 KB of LDS reads per 432 matrix-core cycles. Wavefront w takes plane
+// z0 + w / 2 and, of its rows, voxels 32 (w % 2) .. + 31 (TY = 64) or row
+// x0 + w % 2 (TY = 32). The four wavefronts' sums meet in LDS, and the block
+// writes part[chunk][t][m][n] for its m and n blocks. With db, the blocks of the
+// first n block also sum the centre dpre fragments they read (each voxel once:
+// the bias gradient of their m block) into part[chunk][27 mc kc + m]; a chunk's
 // partials are 27 mc kc + mc floats.
-// Transposed store of 4 voxels x 8 channels (q[k] = channels of voxel k):
-// channel j's four values at dst[j * pitch .. + 3], one 8-byte store each.
-__device__ __forceinline__ void store_quads(uint16_t* dst, int pitch, const uint4 (&q)[4]) {
-  const unsigned* d[4] = {&q[0].x, &q[1].x, &q[2].x, &q[3].x};
-#pragma unroll
-  for (int j = 0; j < 8; j++) {
-    const int h = j >> 1, sh = (j & 1) * 16;
-    const unsigned lo = ((d[0][h] >> sh) & 0xFFFFu) | (((d[1][h] >> sh) & 0xFFFFu) << 16);
-    const unsigned hi = ((d[2][h] >> sh) & 0xFFFFu) | (((d[3][h] >> sh) & 0xFFFFu) << 16);
-    *reinterpret_cast<uint2*>(dst + j * pitch) = uint2{lo, hi};
-  }
+//
+// Bound by the instructions of a step (54 products, 48 LDS reads and about 180
+// scalar and 60 vector instructions that fetch and store the next rows, at two
+// wavefronts per SIMD: 27 accumulators and two steps' rows take 210 registers)
+// and, at 16x16 channels, by the fixed cost of a block (ring start, sums of the
+// wavefronts, partials). Before, operands were transposed by shifts and 8-byte
+// LDS stores, a wavefront read 19 KB of LDS per 432 matrix-core cycles, and
+// every load had its own bounds branches. With k_sum_chunks, at 12 bricks per
+// block: 96x128x128 voxels 16x16 channels 83 -> 37 us, 75x101x131 84 -> 35;
+// 16x48 at 24 bricks 172 -> 80. With the ring but loads behind bounds branches
+// 40 us; one step in flight instead of two changes nothing then. Blocks of a
+// chunk on different XCDs (n block slowest): 16x48 122 us, 32x96 at 48x64x64
+// 96 against 48.
+typedef __attribute__((address_space(3))) unsigned char lds_u8;
+__device__ __forceinline__ bf8 tr_fragment(const lds_u8* p) {
+  struct {
+    s4 lo, hi;
+  } q = {__builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4*)p),
+         __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4*)(p + 512))};
+  return __builtin_bit_cast(bf8, q);
+}
+// 16 bytes at `off` of the `bytes` at row (row and bytes: one value per wavefront); zero past them
+__device__ __forceinline__ uint4 ld_row(const uint16_t* row, int bytes, int off) {
+  const unsigned long p = (unsigned long)row;
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)p), hi = __builtin_amdgcn_readfirstlane((unsigned)(p >> 32));
+  void* const base = reinterpret_cast<void*>((unsigned long)hi << 32 | lo);
+  return __builtin_bit_cast(
+      uint4, __builtin_amdgcn_raw_buffer_load_b128(
+                 __builtin_amdgcn_make_buffer_rsrc(base, (short)0, __builtin_amdgcn_readfirstlane(bytes), 0x00020000),
+                 off, 0, 0));
 }
 
 template <int TY>
-__global__ __launch_bounds__(256) void k_wgrad(const uint16_t* __restrict__ dpre, int ldp, int mc,
-                                               const uint16_t* __restrict__ src, int lds, int kc,
-                                               float* __restrict__ part, float* __restrict__ dw,
-                                               float* __restrict__ db, Vol V, int ntz, int ntx, int nty, int per,
-                                               const uint16_t* __restrict__ src2, int lds2, int kc1, int up1) {
-  constexpr int HW = TY + 2, P = TY + 8, NK = TY / 32;
-  constexpr int A_BYTES = 4 * 16 * P * 2, B_BYTES = 16 * 16 * P * 2, R_BYTES = 9 * 4 * 256 * 4;
-  constexpr int S_BYTES = A_BYTES + (B_BYTES > R_BYTES ? B_BYTES : R_BYTES);
+__global__ __launch_bounds__(256, 2) void k_wgrad(const uint16_t* __restrict__ dpre, int ldp, int mc,
+                                                  const uint16_t* __restrict__ src, int lds, int kc,
+                                                  float* __restrict__ part, float* __restrict__ dw,
+                                                  float* __restrict__ db, Vol V, int ntz, int ntx, int nty, int per,
+                                                  const uint16_t* __restrict__ src2, int lds2, int kc1, int up1) {
+  constexpr int A_ROW = TY * 32, A_SLOT = 8 * A_ROW, B_ROW = (TY + 2) * 32, B_BUF = 4 * B_ROW;
+  constexpr int A_BYTES = 3 * A_SLOT, R_BYTES = 9 * 4 * 256 * 4;
+  constexpr int S_BYTES = A_BYTES + 2 * B_BUF > R_BYTES ? A_BYTES + 2 * B_BUF : R_BYTES;
+  constexpr int NA = 8 * TY * 2 / 256, NB = (2 * (TY + 2) + 63) / 64;  // 16-byte loads per thread
   __shared__ __align__(16) unsigned char smem[S_BYTES];
-  uint16_t* Ah = reinterpret_cast<uint16_t*>(smem);            // [row][m][y]
-  uint16_t* Bh = reinterpret_cast<uint16_t*>(smem + A_BYTES);  // [halo row][n][hv]
-  float* red = reinterpret_cast<float*>(smem + A_BYTES);       // after the last brick
-  const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
-  const int i = lane & 15, g = lane >> 4;
-  const int wz = wv >> 1, wx = wv & 1;
-  const int mb = blockIdx.y, nb = blockIdx.z;
+  float* red = reinterpret_cast<float*>(smem);  // after the last brick
+  const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  // the channel blocks of a chunk go to one XCD (blocks are dealt to the 8 XCDs in turn), one after the other
+  const int nblocks = (mc / 16) * (kc / 16), turn = (int)(blockIdx.x / 8), cb = turn % nblocks;
+  const int mb = cb / (kc / 16), nb = cb % (kc / 16);
+  const int chunk = turn / nblocks * 8 + (int)(blockIdx.x % 8);
   const long nbricks = (long)ntz * ntx * nty;
-  const long b0 = (long)blockIdx.x * per, b1 = std::min(nbricks, b0 + per);
+  const long b0 = (long)chunk * per, b1 = std::min(nbricks, b0 + per);
+  if (b0 >= nbricks) return;
   const bool bias = db != nullptr && nb == 0;
   // this block's 16 src channels: from src below kc1, else from src2
   const bool second = nb * 16 >= kc1;
@@ -448,90 +473,109 @@ __global__ __launch_bounds__(256) void k_wgrad(const uint16_t* __restrict__ dpre
   f4 acc[27];
 #pragma unroll
   for (int t = 0; t < 27; t++) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
-  for (long brick = b0; brick < b1; brick++) {
-    const int zt = (int)(brick % ntz);
-    const long r2 = brick / ntz;
-    const int xt = (int)(r2 % ntx), yt = (int)(r2 / ntx);
-    const int z0 = 2 * zt, x0 = 2 * xt, y0 = yt * TY;
-    // planes z0 - 1 and z0 are in the ring when this block's previous brick
-    // was the one below in the same column
-    const int hz0 = brick > b0 && zt > 0 ? 2 : 0;
-    // channel-major copies, 4 voxels along y per item: each channel's 4 values
-    // go out as one 8-byte LDS store (consecutive lanes take consecutive
-    // voxel quads of one channel row). Threads keep their (granule, quad,
-    // row) for the brick; in a brick clear of the volume faces no voxel needs
-    // a bounds check.
-    const bool interior = z0 >= 1 && z0 + 2 < V.nz && x0 >= 1 && x0 + 2 < V.nx && y0 >= 1 && y0 + TY + 2 < V.ny;
-    if (tid < 4 * (TY / 4) * 2) {
-      const int y4 = tid % (TY / 4), rem = tid / (TY / 4);
-      const int gr = rem & 1, row = rem >> 1;
-      const int z = z0 + (row >> 1), x = x0 + (row & 1), y = y0 + 4 * y4;
-      const bool zx_ok = z < V.nz && x < V.nx;
-      const uint16_t* p = dpre + V.vox(zx_ok ? z : 0, zx_ok ? x : 0, y) * ldp + mb * 16 + 8 * gr;
-      uint4 q[4];
+  // Pair p of column (zt, yt): dpre rows 2 p - 1, 2 p of the planes 2 zt - 1 .. 2 zt + 2
+  // and, per wavefront, one of the src rows 2 p - 2, 2 p - 1 of the planes 2 zt, 2 zt + 1,
+  // voxels y0 - 1 .. y0 + TY. Every load instruction stays in one row, whose bounds are those of
+  // a buffer descriptor in scalar registers (empty outside the volume and past the last step):
+  // what is out of range reads as zero without a branch or an address per lane.
+  int fp = __builtin_amdgcn_readfirstlane((int)(b0 % ntx)), fz = __builtin_amdgcn_readfirstlane((int)(b0 / ntx % ntz)),
+      fy = __builtin_amdgcn_readfirstlane((int)(b0 / ((long)ntx * ntz)));
+  const int gr2 = (tid & 1) * 16;
+  const int a_off = (lane >> 1) * ldp * 2 + gr2;  // voxel lane / 2 of the row's 32 of this instruction
+  int b_off[NB];                                  // from the voxel before the row's first
 #pragma unroll
-      for (int k = 0; k < 4; k++) {
-        q[k] = uint4{0u, 0u, 0u, 0u};
-        if (interior || (zx_ok && y + k < V.ny)) q[k] = ld16(p + (long)k * ldp);
-      }
-      store_quads(Ah + (row * 16 + 8 * gr) * P + 4 * y4, P, q);
+  for (int u = 0; u < NB; u++) b_off[u] = (((((lane + 64 * u) >> 1) - 1) >> (int)up) + 1) * (int)sl * 2 + gr2;
+  const int a_row = TY == 64 ? wv >> 1 : wv & 1, a_half = TY == 64 ? 32 * (wv & 1) : 0, a_plane = TY == 64 ? 0 : wv >> 1;
+  const int ush = (int)up, unx = V.nx >> ush, uny = V.ny >> ush;
+  auto fetch = [&](bool live, uint4 (&qa)[NA], uint4 (&qb)[NB]) {
+    const int y0 = fy * TY, ya = y0 + a_half, xa = 2 * fp - 1 + a_row;
+    const int na = V.ny - ya < 32 ? V.ny - ya : 32;
+    const int a_bytes = live && na > 0 && (unsigned)xa < (unsigned)V.nx ? na * ldp * 2 : 0;
+#pragma unroll
+    for (int u = 0; u < NA; u++) {
+      const int z = 2 * fz - 1 + (TY == 64 ? u : 2 * u + a_plane);
+      qa[u] = ld_row(dpre + V.vox(z, xa, ya) * ldp + mb * 16, (unsigned)z < (unsigned)V.nz ? a_bytes : 0, a_off);
     }
-    constexpr int HW4 = (HW + 3) / 4;
-    // halo: thread = (granule, quad, hx) walks hz = 0..3 (uniform plane offsets)
-    if (tid < 2 * HW4 * 4) {
-      const int y4 = tid % HW4, rem = tid / HW4;
-      const int gr = rem & 1, hx = rem >> 1;
-      const int xs = x0 - 1 + hx, ys = y0 - 1 + 4 * y4;
-      const bool x_ok = xs >= 0 && xs < V.nx;
-      const long v0 = V.vox(z0 - 1, x_ok ? xs : 0, ys);
-      const long plane = (long)V.nx * V.ny;
+    const int z = 2 * fz + (wv >> 1), x = 2 * fp - 2 + (wv & 1);
+    const int nv = ((V.ny - y0) >> ush) + 1 < TY + 2 ? ((V.ny - y0) >> ush) + 1 : TY + 2;
+    const int b_bytes = live && (unsigned)z < (unsigned)V.nz && (unsigned)x < (unsigned)V.nx ? nv * (int)sl * 2 : 0;
+    const uint16_t* const row = sb + (((long)(z >> ush) * unx + (x >> ush)) * uny + (y0 >> ush) - 1) * sl + scol;
 #pragma unroll
-      for (int hz = 0; hz < 4; hz++) {
-        if (hz < hz0) continue;
-        const int zs = z0 - 1 + hz;
-        const bool zx_ok = x_ok && zs >= 0 && zs < V.nz;
-        const uint16_t* p = sb + (v0 + hz * plane) * sl + scol + 8 * gr;
-        // coarse row of (zs, xs) when up (read only where zx_ok)
-        const uint16_t* pc =
-            sb + (((long)(zs >> 1) * (V.nx >> 1) + (xs >> 1)) * (V.ny >> 1)) * sl + scol + 8 * gr;
-        uint4 q[4];
+    for (int u = 0; u < NB; u++)
+      qb[u] = ld_row(row, b_bytes, u == 0 && fy == 0 && lane < 2 ? (int)0x80000000 : b_off[u]);  // y = -1
+    if (++fp > ntx) {
+      fp = 0;
+      if (++fz == ntz) {
+        fz = 0;
+        fy++;
+      }
+    }
+  };
+  auto put = [&](int slot, int par, const uint4 (&qa)[NA], const uint4 (&qb)[NB]) {
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-          q[k] = uint4{0u, 0u, 0u, 0u};
-          if (interior || (zx_ok && ys + k >= 0 && ys + k < V.ny))
-            q[k] = up ? ld16(pc + (long)((ys + k) >> 1) * sl) : ld16(p + (long)k * sl);
+    for (int u = 0; u < NA; u++) st16(smem + slot * A_SLOT + (tid + 256 * u) * 16, qa[u]);
+#pragma unroll
+    for (int u = 0; u < NB; u++)
+      if (lane + 64 * u < 2 * (TY + 2)) st16(smem + A_BYTES + par * B_BUF + wv * B_ROW + (lane + 64 * u) * 16, qb[u]);
+  };
+  const lds_u8* const l0 = (const lds_u8*)smem + 8 * lane;
+  const int zp = wv >> 1, sub = wv & 1;
+  // the brick between the pairs in slots `prev` and `cur`
+  auto products = [&](int prev, int cur, int par) {
+#pragma unroll
+    for (int rr = 0; rr < (TY == 64 ? 2 : 1); rr++) {
+      const int xr = TY == 64 ? rr : sub, c = TY == 64 ? sub : 0;
+      const lds_u8* const bp = l0 + A_BYTES + par * B_BUF + (zp * 2 + xr) * B_ROW + c * 1024;
+      bf8 b[3];
+#pragma unroll
+      for (int d = 0; d < 3; d++) b[d] = tr_fragment(bp + 32 * d);
+#pragma unroll
+      for (int dxi = 0; dxi < 3; dxi++) {
+        // the dpre row of tap dx = dxi - 1: x0 + xr - dx, of the four from x0 - 1
+        const int r = xr + 2 - dxi;
+        const lds_u8* const ap = l0 + (r < 2 ? prev : cur) * A_SLOT + (2 * zp + (r & 1)) * A_ROW + c * 1024;
+#pragma unroll
+        for (int dzi = 0; dzi < 3; dzi++) {
+          const bf8 a = tr_fragment(ap + 2 * (2 - dzi) * A_ROW);
+          if (bias && dxi == 1 && dzi == 1) {
+            const uint4 q = __builtin_bit_cast(uint4, a);
+            const unsigned u[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+            for (int k = 0; k < 4; k++) bsum += __uint_as_float(u[k] << 16) + __uint_as_float(u[k] & 0xFFFF0000u);
+          }
+#pragma unroll
+          for (int d = 0; d < 3; d++) {
+            const int t = 9 * dzi + 3 * dxi + d;
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[d], acc[t], 0, 0, 0);
+          }
         }
-        store_quads(Bh + (((zs & 3) * 4 + hx) * 16 + 8 * gr) * P + 4 * y4, P, q);
       }
     }
+  };
+  // one step per pair; the first of a column only brings its rows
+  const int steps = (int)(b1 - b0 + (b1 - 1) / ntx - b0 / ntx + 1);
+  int pc = fp;               // pair of the current step
+  bool first = true;         // no pair of this column before it
+  int prev = 2, cur = 0;     // ring slots of the previous and the current pair
+  uint4 qa0[NA], qb0[NB], qa1[NA], qb1[NB];
+  auto step = [&](int s, uint4 (&qa)[NA], uint4 (&qb)[NB], const uint4 (&na)[NA], const uint4 (&nbq)[NB]) {
+    fetch(s + 2 < steps, qa, qb);
+    if (!first) products(prev, cur, s & 1);
+    first = pc == ntx;
+    pc = first ? 0 : pc + 1;
+    prev = cur;
+    cur = cur == 2 ? 0 : cur + 1;
+    if (s + 1 < steps) put(cur, (s + 1) & 1, na, nbq);
     __syncthreads();
+  };
+  fetch(true, qa0, qb0);
+  fetch(true, qa1, qb1);  // a block has at least one brick, so at least two steps
+  put(0, 0, qa0, qb0);
+  __syncthreads();
 #pragma unroll 1
-    for (int c = 0; c < NK; c++) {
-      const uint4 a = *reinterpret_cast<const uint4*>(&Ah[(wv * 16 + i) * P + 32 * c + 8 * g]);
-      if (bias) {
-        const unsigned u[4] = {a.x, a.y, a.z, a.w};
-#pragma unroll
-        for (int j = 0; j < 4; j++) bsum += __uint_as_float(u[j] << 16) + __uint_as_float(u[j] & 0xFFFF0000u);
-      }
-#pragma unroll
-      for (int dzdx = 0; dzdx < 9; dzdx++) {
-        const int hr = ((z0 - 1 + wz + dzdx / 3) & 3) * 4 + (wx + dzdx % 3);
-        const uint16_t* bp = &Bh[(hr * 16 + i) * P + 32 * c + 8 * g];
-        const uint4 g0 = *reinterpret_cast<const uint4*>(bp);
-        const uint4 g1 = *reinterpret_cast<const uint4*>(bp + 8);
-        // halo voxels 32c + 8g + (dy + 1) + j, j = 0..7
-        const uint4 s1 = {__builtin_amdgcn_alignbyte(g0.y, g0.x, 2), __builtin_amdgcn_alignbyte(g0.z, g0.y, 2),
-                          __builtin_amdgcn_alignbyte(g0.w, g0.z, 2), __builtin_amdgcn_alignbyte(g1.x, g0.w, 2)};
-        const uint4 s2 = {g0.y, g0.z, g0.w, g1.x};
-        const bf8 av = __builtin_bit_cast(bf8, a);
-        acc[3 * dzdx] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, __builtin_bit_cast(bf8, g0), acc[3 * dzdx], 0, 0, 0);
-        acc[3 * dzdx + 1] =
-            __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, __builtin_bit_cast(bf8, s1), acc[3 * dzdx + 1], 0, 0, 0);
-        acc[3 * dzdx + 2] =
-            __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, __builtin_bit_cast(bf8, s2), acc[3 * dzdx + 2], 0, 0, 0);
-      }
-    }
-    __syncthreads();
+  for (int s = 0; s < steps; s += 2) {
+    step(s, qa0, qb0, qa1, qb1);
+    if (s + 1 < steps) step(s + 1, qa1, qb1, qa0, qb0);
   }
   // sum of the four wavefronts, 9 taps at a time; lane (i, g) holds
   // D[m = 4 g + j][n = i] of each tap
@@ -549,10 +593,10 @@ __global__ __launch_bounds__(256) void k_wgrad(const uint16_t* __restrict__ dpre
     for (int tt = 0; tt < 9; tt++) {
       const float s = red[(tt * 4 + 0) * 256 + tid] + red[(tt * 4 + 1) * 256 + tid] + red[(tt * 4 + 2) * 256 + tid] +
                       red[(tt * 4 + 3) * 256 + tid];
-      part[(long)blockIdx.x * stride + ((long)(9 * p + tt) * mc + m) * kc + n] = s;
+      part[(long)chunk * stride + ((long)(9 * p + tt) * mc + m) * kc + n] = s;
       // dw is summed from the partials by atomics after this kernel: the
       // first chunk's blocks clear it
-      if (blockIdx.x == 0) dw[((long)(9 * p + tt) * mc + m) * kc + n] = 0.f;
+      if (chunk == 0) dw[((long)(9 * p + tt) * mc + m) * kc + n] = 0.f;
     }
     __syncthreads();
   }
@@ -563,8 +607,8 @@ __global__ __launch_bounds__(256) void k_wgrad(const uint16_t* __restrict__ dpre
       float s = 0.f;
 #pragma unroll
       for (int q = 0; q < 16; q++) s += red[16 * q + tid];
-      part[(long)blockIdx.x * stride + W + mb * 16 + tid] = s;
-      if (blockIdx.x == 0) db[mb * 16 + tid] = 0.f;
+      part[(long)chunk * stride + W + mb * 16 + tid] = s;
+      if (chunk == 0) db[mb * 16 + tid] = 0.f;
     }
   }
 }
@@ -1363,7 +1407,7 @@ static int wgrad_launch(const uint16_t* dpre, int ldp, int mc, const uint16_t* s
   const int ty = wgrad_ty(ny);
   const int ntz = (nz + 1) / 2, ntx = (nx + 1) / 2, nty = (ny + ty - 1) / ty;
   const int chunks = (int)((wgrad_bricks(nz, nx, ny) + per - 1) / per);
-  const dim3 grid((unsigned)chunks, (unsigned)(mc / 16), (unsigned)(kc / 16));
+  const dim3 grid((unsigned)((chunks + 7) / 8 * 8 * (mc / 16) * (kc / 16)));
   if (ty == 64)
     hipLaunchKernelGGL((k_wgrad<64>), grid, dim3(256), 0, s, dpre, ldp, mc, src, lds, kc, scratch, dw, db, V, ntz, ntx,
                        nty, per, src2, lds2, kc1, up1);

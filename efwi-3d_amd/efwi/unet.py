@@ -45,7 +45,7 @@ LAYERS = [
     ("dec1a", 48, 16, 1), ("dec1b", 16, 16, 1),
 ]
 IN_CHANNELS = 2       # raw gradient, log illumination
-WGRAD_WORKGROUPS = 768   # weight gradient: about three resident workgroups per CU
+WGRAD_PER_XCD = 64    # weight gradient: resident workgroups per XCD (two per CU)
 
 
 def nn_check(rc: int, what: str):
@@ -215,16 +215,18 @@ class UNet3D:
         nn_check(rc, f"dgrad {name}")
 
     def _wgrad_per(self, cout, cin, dims):
-        """Bricks per weight-gradient workgroup: enough workgroups to fill the
-        GPU (about WGRAD_WORKGROUPS over the (m, n) channel blocks), between 2
-        and 24 bricks each (fewer bricks per workgroup multiply the FP32
-        partials that are written and summed, more keep more halo planes in
-        the workgroup's z ring; measured on MI355X at the U-Net's shapes:
-        48->16 at 96x128x128 per 8 205 us, per 24 172 us; 96->32 at 48x64x64
-        per 8 112 us, per 12 96 us)."""
+        """Bricks per weight-gradient workgroup: all workgroups resident at once
+        where that takes 6 to 24 bricks each. A chunk's (m, n) channel blocks
+        run on one XCD, which holds WGRAD_PER_XCD workgroups. Fewer bricks
+        multiply the FP32 partials that are written and summed (64x64 at
+        24x32x32: per 2 37 us, 6 23, 12 20; 64x32: per 3 20, 6 17), a few
+        workgroups beyond the resident ones cost a second pass (32x96 at
+        48x64x64: per 18 63 us, 20 48; 16x16 at 96x128x128: per 10 46, 12 37),
+        and more than 24 gain nothing (16x48: per 24 80, 40 80)."""
         bricks = int(self.lib.efwi_nn_wgrad_scratch(cout, cin, *dims, 1)) // (27 * cout * cin + cout)
         blocks = (cout // 16) * (cin // 16)
-        return int(min(24, max(2, bricks * blocks // WGRAD_WORKGROUPS)))
+        chunks = 8 * max(1, WGRAD_PER_XCD // blocks)
+        return int(min(24, max(6, -(-bricks // chunks))))
 
     def _wgrad(self, name, gpre, ldg, src, lds, dims, src2=None):
         """Weight and bias gradients of layer `name`; with src2, its input is
