@@ -77,6 +77,26 @@ __device__ __forceinline__ void tap(int t, int& dz, int& dx, int& dy) {
   dy = t % 3 - 1;
 }
 
+// A buffer descriptor of the `bytes` at row (both one value per wavefront):
+// loads past them return zero, stores past them are dropped, without a branch
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t row_rsrc(const void* row, int bytes) {
+  const unsigned long p = (unsigned long)row;
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)p), hi = __builtin_amdgcn_readfirstlane((unsigned)(p >> 32));
+  return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>((unsigned long)hi << 32 | lo), (short)0,
+                                           __builtin_amdgcn_readfirstlane(bytes), 0x00020000);
+}
+constexpr int kPastRow = (int)0x80000000;  // a byte offset past every row
+__device__ __forceinline__ uint4 ld_row(const void* row, int bytes, int off) {
+  return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(row_rsrc(row, bytes), off, 0, 0));
+}
+__device__ __forceinline__ uint2 ld_row8(const void* row, int bytes, int off) {
+  return __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(row_rsrc(row, bytes), off, 0, 0));
+}
+__device__ __forceinline__ void st_row8(void* row, int bytes, int off, const uint2& q) {
+  typedef unsigned u2 __attribute__((ext_vector_type(2)));
+  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, q), row_rsrc(row, bytes), off, 0, 0);
+}
+
 // 3x3x3 convolution as implicit GEMM on v_mfma_f32_16x16x32_bf16, the input
 // staged through LDS. A workgroup of 2 TZ wavefronts owns a brick of TZ (z) x
 // 2 (x) rows of TY = 16 MB voxels along y and NB blocks of 16 output
@@ -354,6 +374,253 @@ __global__ __launch_bounds__(512) void k_conv3(const uint16_t* __restrict__ src,
   }
 }
 
+
+// The convolution (mode 0) of rows of 64 voxels or more with the loads of the
+// next input chunk in flight over this one's products. A block of eight
+// wavefronts owns bricks as k_conv3's (4 z, 2 x, 64 voxels) and walks every
+// (gridDim.x / 8)-th brick of its XCD's contiguous run, 16 input channels of a
+// brick at a step; the halo is double buffered, one barrier per step.
+//  - Each load instruction stays in one halo row, whose bounds are those of a
+//    descriptor in scalar registers (empty outside the volume and past the last
+//    step): no branch and no address per lane. The last 2 of a row's 66 voxels
+//    take one more load for all of a wavefront's rows.
+//  - The weights lie in LDS, or with 16 input channels and one output block in
+//    registers. The fragments of two tap pairs ahead are read over a pair's products.
+//  - D is computed transposed (weights x voxels): a lane holds 4 channels of a
+//    voxel and stores (and masks) them as 8 bytes; a wavefront's store is 512
+//    contiguous bytes.
+// The products and their order are k_conv3's, so the results are too.
+//
+// Bound by LDS reads (14 fragments of 1 KB per 16 voxels and 14 NB products;
+// 2.9 of the 6.4 us that the 16->16 step of eight wavefronts takes at 128 bytes a
+// clock) and by the wavefronts' scalar and address work, during which the LDS
+// idles: without the loads 31 of 34 us, with one of the 14 products 24. One block
+// per CU at 170 to 255 registers; two with single buffers and 128 registers spill
+// and were slower (51 us); keeping the rows in an LDS ring along x (halo rows per
+// output row 1.5 instead of 3) changed nothing at 96x128x128. Measured, k_conv3 against this:
+// 16->16 at 96x128x128 45 -> 34 us, at 120x200x200 163 -> 112; 16->48 100 -> 66;
+// 32->32 at 60x100x100 70 -> 47, 96->32 180 -> 120; 48->16 at 120x200x200 337 -> 316.
+template <int NB, bool ONE>
+__global__ __launch_bounds__(512, 2) void k_conv_pipe(
+    const uint16_t* __restrict__ src, int lds, int kc, const uint16_t* __restrict__ w, const float* __restrict__ bias,
+    uint16_t* __restrict__ dst, int ldd, int nc, const uint16_t* __restrict__ mask, int ldm, Vol V, int relu,
+    int ntx, int nty, int nbricks, int per_xcd, int vec_out, const uint16_t* __restrict__ src2, int lds2, int kc1,
+    uint16_t* __restrict__ dst2, int ldd2, int nc1, int up1) {
+  constexpr int MB = 4, TY = 16 * MB, HW = TY + 2, VB = 32, NBC = 16 * NB;
+  constexpr int TZ = conv_tz(MB), NT = 128 * TZ, HR = (TZ + 2) * 4;  // halo rows
+  constexpr int RPW = HR / (NT / 64);               // halo rows per wavefront
+  constexpr int WU = (27 * NBC * 2 + NT - 1) / NT;  // weight granules per thread
+  constexpr int HB = HR * HW * VB, WB = 27 * NBC * VB;
+  constexpr bool WR = ONE && NB == 1;  // weights in registers
+  constexpr int WBUF = ONE ? 1 : 2, WL = 2 * HB, ZERO = WL + WBUF * WB;
+  // halo buffers, weight buffers, zeros (the 28th tap's inputs and weights)
+  __shared__ __align__(16) unsigned char smem[ZERO + MB * 512];
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wz = wv >> 1, wx = wv & 1;
+  const int i = lane & 15, g = lane >> 4, hi = g >> 1, grl = g & 1;
+  const int nb0 = blockIdx.y * NB;
+  // LDS byte offset of the lane's granule of the halo voxel (wz, wx, i) for
+  // each kind of tap pair, relative to the lower tap's row: dy (0, 1), (1, 2),
+  // (2, 0 of the next row), (2, 0 of the next plane's first row)
+  auto granule = [&](int d) { return (i + d) * VB + 16 * (grl ^ granule_swizzle<16>(i + d)); };
+  const int corner = (wz * 4 + wx) * HW * VB;
+  const int pair01 = corner + (hi ? granule(1) : granule(0)), pair12 = corner + (hi ? granule(2) : granule(1));
+  const int pair20 = corner + (hi ? granule(0) + HW * VB : granule(2));
+  const int pair20z = corner + (hi ? granule(0) + 2 * HW * VB : granule(2));
+  const int last2 = corner + granule(2), zero_in = ZERO + 32 * i - (2 * 4 + 2) * HW * VB;
+  const int wbase = WL + i * VB + 16 * (grl ^ granule_swizzle<16>(i)) + hi * NBC * VB;
+  const int w27 = hi ? ZERO + 32 * i : wbase + 26 * NBC * VB;
+  // this block's bricks: every (gridDim.x / 8)-th of its XCD's contiguous run
+  const int step = gridDim.x >> 3, end = std::min(nbricks, ((int)(blockIdx.x & 7) + 1) * per_xcd);
+  int next = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+  if (next >= end) return;  // whole block
+  // the coordinates of the next brick, and those of a step
+  int yt = next % nty, xt = next / nty % ntx, zt = next / nty / ntx;
+  const int sy = step % nty, sx = step / nty % ntx, sz = step / nty / ntx;
+  uint4 hq[RPW * 2], tq, wq[WU];  // halo rows, their last voxels, weights
+  bool tok = false;
+  const int gr16 = 16 * (lane & 1);
+  // the row and voxel of the lane's granule of the last two voxels
+  const int trow = wv * RPW + (lane >> 2), tvox = 64 + ((lane >> 1) & 1);
+  auto fetch = [&](bool live, int c0) {
+    const int z0 = TZ * zt - 1, x0 = 2 * xt - 1, y0 = yt * TY;
+    const bool second = !ONE && c0 >= kc1;
+    const unsigned char* const sb = reinterpret_cast<const unsigned char*>((second ? src2 : src) + (second ? c0 - kc1 : c0));
+    const unsigned sl2 = 2 * (second ? lds2 : lds);
+    const int ush = up1 && !second ? 1 : 0, unx = V.nx >> ush, uny = V.ny >> ush;
+    const unsigned rb = uny * sl2;
+    // z0 and x0 are odd: halves of z0 + hz are (z0 - 1) / 2 + (hz + 1) / 2
+    const unsigned char* const base =
+        sb + ((long)((z0 >> ush) * unx + (x0 >> ush)) * rb + (long)((y0 >> ush) - 1) * (long)sl2);
+    const int nv = ((V.ny - y0) >> ush) + 1 < HW ? ((V.ny - y0) >> ush) + 1 : HW;
+    const int bytes = live ? nv * (int)sl2 : 0;
+    const int voff = (((lane >> 1) - 1 >> ush) + 1) * sl2 + gr16, voff0 = y0 == 0 && lane < 2 ? kPastRow : voff;
+#pragma unroll
+    for (int u = 0; u < RPW; u++) {
+      const int r = wv * RPW + u, hz = r >> 2, hx = r & 3;
+      const bool in = (unsigned)(z0 + hz) < (unsigned)V.nz && (unsigned)(x0 + hx) < (unsigned)V.nx;
+      const unsigned char* const row = base + (unsigned long)(unsigned)(((hz + ush) >> ush) * unx + ((hx + ush) >> ush)) * rb;
+      hq[2 * u] = ld_row(row, in ? bytes : 0, voff0);
+      hq[2 * u + 1] = ld_row(row, in ? bytes : 0, voff + (32 >> ush) * (int)sl2);
+    }
+    const int hz = trow >> 2, hx = trow & 3;
+    tok = live && lane < 4 * RPW && (unsigned)(z0 + hz) < (unsigned)V.nz && (unsigned)(x0 + hx) < (unsigned)V.nx &&
+          y0 - 1 + tvox < V.ny;
+    const unsigned long off = (unsigned long)(unsigned)(((hz + ush) >> ush) * unx + ((hx + ush) >> ush)) * rb +
+                              (((tvox - 1) >> ush) + 1) * sl2 + gr16;
+    tq = ld16(tok ? base + off : sb);
+  };
+  auto fetch_w = [&](int c0) {
+    // granule tid + NT u: (tap, n, granule), the granule fastest; zero past tap 26
+#pragma unroll
+    for (int u = 0; u < WU; u++) {
+      const int item = tid + NT * u, t = item / (2 * NBC), n = nb0 * 16 + (item >> 1) % NBC, gr = item & 1;
+      wq[u] = ld_row(w + c0, 27 * nc * kc * 2 - c0 * 2, ((t * nc + n) * kc + 8 * gr) * 2);
+    }
+  };
+  auto put = [&](int buf) {
+    // (voxels 32 apart have the same swizzle)
+    const int v = lane >> 1;
+    unsigned char* const p = smem + buf * HB + (wv * RPW * HW + v) * VB + 16 * ((lane & 1) ^ granule_swizzle<16>(v));
+#pragma unroll
+    for (int u = 0; u < RPW; u++)
+#pragma unroll
+      for (int m = 0; m < 2; m++) st16(p + (u * HW + 32 * m) * VB, hq[2 * u + m]);
+    if (lane < 4 * RPW)
+      st16(smem + buf * HB + (trow * HW + tvox) * VB + 16 * ((lane & 1) ^ granule_swizzle<16>(tvox)),
+           tok ? tq : uint4{0u, 0u, 0u, 0u});
+  };
+  auto put_w = [&](int buf) {
+#pragma unroll
+    for (int u = 0; u < WU; u++) {
+      const int item = tid + NT * u, n = (item >> 1) % NBC;
+      if (item < 27 * NBC * 2)
+        st16(smem + WL + buf * WB + (item >> 1) * VB + 16 * ((item & 1) ^ granule_swizzle<16>(n & 15)), wq[u]);
+    }
+  };
+  f4 acc[MB][NB], bn[NB];
+#pragma unroll
+  for (int c = 0; c < NB; c++) {
+    const int n = (nb0 + c) * 16 + 4 * g;
+    bn[c] = bias ? f4{bias[n], bias[n + 1], bias[n + 2], bias[n + 3]} : f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int m = 0; m < MB; m++) acc[m][c] = f4{0.f, 0.f, 0.f, 0.f};
+  }
+  int c0 = 0;
+  fetch(true, 0);
+  fetch_w(0);
+  if (tid < MB * 32) st16(smem + ZERO + 16 * tid, uint4{0u, 0u, 0u, 0u});
+  put(0);
+  put_w(0);
+  __syncthreads();
+  uint4 wr[WR ? 14 : 1];
+  if (WR)
+#pragma unroll
+    for (int q = 0; q < 14; q++) wr[q] = lds_read16(smem, q == 13 ? w27 : wbase + 2 * q * NBC * VB);
+  int buf = 0;
+  for (;;) {
+    const bool last = ONE || c0 + 16 >= kc;
+    // this brick's output row
+    const int z = TZ * zt + wz, x = 2 * xt + wx, y0 = yt * TY;
+    const long vrow = V.vox(z, x, y0);
+    const int nrow = last && z < V.nz && x < V.nx ? (V.ny - y0 < TY ? V.ny - y0 : TY) : 0;
+    // its mask
+    uint2 mk[MB][NB];
+    if (mask && vec_out) {
+#pragma unroll
+      for (int m = 0; m < MB; m++)
+#pragma unroll
+        for (int c = 0; c < NB; c++)
+          mk[m][c] = ld_row8(mask + vrow * ldm + (nb0 + c) * 16, nrow * ldm * 2, ((16 * m + i) * ldm + 4 * g) * 2);
+    }
+    if (last) {
+      next += step;
+      yt += sy;
+      xt += sx;
+      zt += sz;
+      if (yt >= nty) yt -= nty, xt++;
+      if (xt >= ntx) xt -= ntx, zt++;
+    }
+    const int nc0 = last ? 0 : c0 + 16;
+    const bool more = next < end;
+    fetch(more, nc0);
+    if (!ONE) fetch_w(nc0);
+    // fragments of the pair (2 q, 2 q + 1), read D pairs ahead of their products
+    constexpr int D = NB > 2 ? 1 : 2;
+    uint4 a[D + 1][MB], bw[D + 1][NB];
+    auto read = [&](int q) {
+      const int tl = 2 * q, dy = tl % 3, row = tl / 9 * 4 + tl / 3 % 3;
+      const int pair = dy == 0 ? pair01 : dy == 1 ? pair12 : row % 4 == 2 ? pair20z : pair20;
+      const int ao = q < 13 ? pair + buf * HB : hi ? zero_in : last2 + buf * HB;
+#pragma unroll
+      for (int m = 0; m < MB; m++) a[q % (D + 1)][m] = lds_read16(smem, ao + row * HW * VB + 16 * m * VB);
+      if (!WR) {
+        const int wb = WBUF > 1 ? buf * WB : 0;
+#pragma unroll
+        for (int c = 0; c < NB; c++)
+          bw[q % (D + 1)][c] = lds_read16(smem, q == 13 && hi ? w27 : wb + wbase + (tl * NBC + 16 * c) * VB);
+      }
+    };
+#pragma unroll
+    for (int q = 0; q < D; q++) read(q);
+#pragma unroll
+    for (int q = 0; q < 14; q++) {
+      if (q + D < 14) read(q + D);
+#pragma unroll
+      for (int m = 0; m < MB; m++) {
+#pragma unroll
+        for (int c = 0; c < NB; c++)
+          acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              __builtin_bit_cast(bf8, WR ? wr[WR ? q : 0] : bw[q % (D + 1)][c]), __builtin_bit_cast(bf8, a[q % (D + 1)][m]),
+              ONE && q == 0 ? f4{0.f, 0.f, 0.f, 0.f} : acc[m][c], 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (last) {
+      // D[channel 4 g + j][voxel i] of each (row block, column block)
+#pragma unroll
+      for (int c = 0; c < NB; c++) {
+        const int n0 = (nb0 + c) * 16, n = n0 + 4 * g;
+        const int od = n0 < nc1 ? ldd : ldd2;
+        uint16_t* const out = n0 < nc1 ? dst + vrow * ldd + n0 : dst2 + vrow * ldd2 + (n0 - nc1);
+#pragma unroll
+        for (int m = 0; m < MB; m++) {
+          const int v = 16 * m + i;
+          f4 r = acc[m][c] + bn[c];
+          if (relu)
+#pragma unroll
+            for (int jj = 0; jj < 4; jj++) r[jj] = fmaxf(r[jj], 0.f);
+          if (vec_out) {
+            if (mask) {
+              if (!(__uint_as_float(mk[m][c].x << 16) > 0.f)) r[0] = 0.f;
+              if (!(__uint_as_float(mk[m][c].x & 0xFFFF0000u) > 0.f)) r[1] = 0.f;
+              if (!(__uint_as_float(mk[m][c].y << 16) > 0.f)) r[2] = 0.f;
+              if (!(__uint_as_float(mk[m][c].y & 0xFFFF0000u) > 0.f)) r[3] = 0.f;
+            }
+            typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
+            st_row8(out, nrow * od * 2, (v * od + 4 * g) * 2, __builtin_bit_cast(uint2, __builtin_convertvector(r, bf4)));
+          } else if (v < nrow) {
+#pragma unroll
+            for (int jj = 0; jj < 4; jj++)
+              out[(long)v * od + 4 * g + jj] = f2bf(mask && !(bf2f(mask[(vrow + v) * ldm + n + jj]) > 0.f) ? 0.f : r[jj]);
+          }
+        }
+      }
+      if (!ONE)
+#pragma unroll
+        for (int m = 0; m < MB; m++)
+#pragma unroll
+          for (int c = 0; c < NB; c++) acc[m][c] = f4{0.f, 0.f, 0.f, 0.f};
+    }
+    if (!more) break;
+    buf ^= 1;
+    put(buf);
+    if (!ONE) put_w(buf);
+    c0 = nc0;
+    __syncthreads();
+  }
+}
+
 // wt[t][k][n] = w[26 - t][n][k]: the weights of a layer's input gradient as a
 // forward convolution (taps mirrored, channels transposed)
 __global__ void k_flip_weights(const uint16_t* __restrict__ w, int kc, int nc, uint16_t* __restrict__ wt) {
@@ -430,17 +697,6 @@ __device__ __forceinline__ bf8 tr_fragment(const lds_u8* p) {
          __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4*)(p + 512))};
   return __builtin_bit_cast(bf8, q);
 }
-// 16 bytes at `off` of the `bytes` at row (row and bytes: one value per wavefront); zero past them
-__device__ __forceinline__ uint4 ld_row(const uint16_t* row, int bytes, int off) {
-  const unsigned long p = (unsigned long)row;
-  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)p), hi = __builtin_amdgcn_readfirstlane((unsigned)(p >> 32));
-  void* const base = reinterpret_cast<void*>((unsigned long)hi << 32 | lo);
-  return __builtin_bit_cast(
-      uint4, __builtin_amdgcn_raw_buffer_load_b128(
-                 __builtin_amdgcn_make_buffer_rsrc(base, (short)0, __builtin_amdgcn_readfirstlane(bytes), 0x00020000),
-                 off, 0, 0));
-}
-
 template <int TY>
 __global__ __launch_bounds__(256, 2) void k_wgrad(const uint16_t* __restrict__ dpre, int ldp, int mc,
                                                   const uint16_t* __restrict__ src, int lds, int kc,
@@ -1248,22 +1504,46 @@ int efwi_nn_conv3_cat(const uint16_t* src, int lds, int kc1, int up1, const uint
   const int TZ = conv_tz(MB);
   const int ntz = (nz + TZ - 1) / TZ, ntx = (nx + 1) / 2, nty = (ny + 16 * MB - 1) / (16 * MB);
   const long bricks = (long)ntz * ntx * nty;
+  const int per_xcd = (int)((bricks + 7) / 8);
+  // outputs (and mask) as 8- and 16-byte granules where the pointers allow
+  const int vec_out = (uintptr_t)dst % 16 == 0 && (uintptr_t)dst2 % 16 == 0 && (!mask || (uintptr_t)mask % 16 == 0);
+  // Rows of 64 voxels or more in mode 0: the pipelined kernel, one block per CU,
+  // with the most output blocks that still give every CU three bricks or more
+  // (a last round of few bricks costs as much as a full one: 32->16 at 48x64x64,
+  // 384 bricks, 13.3 us against k_conv3's 12.7; 16->32, 384 bricks at two blocks
+  // 12.5 us, 768 at one 11.6 against 14.5). Three blocks' weights fit LDS only
+  // with one chunk of input channels.
+  if (MB == 4 && mode == 0 && bricks <= INT_MAX - 8L * device_cus()) {
+    const int most = kc == 16 ? 3 : 2;
+    for (int nb = most; nb >= 1; nb--) {
+      if (nbt % nb || bricks * (nbt / nb) < (nb > 1 ? 3L : 2L) * device_cus()) continue;
+      const dim3 pgrid(8u * std::max(1, std::min(per_xcd, device_cus() / 8 / (nbt / nb))), (unsigned)(nbt / nb));
+#define EFWI_NN_CONV_PIPE(B, ONE)                                                                               \
+  hipLaunchKernelGGL((k_conv_pipe<B, ONE>), pgrid, dim3(512), 0, s, src, lds, kc, w, bias, dst, ldd, nc, mask, ldm, \
+                     V, relu, ntx, nty, (int)bricks, per_xcd, vec_out, src2, lds2, kc1, dst2, ldd2, nc1, up1 ? 1 : 0)
+      if (nb == 3) EFWI_NN_CONV_PIPE(3, true);
+      else if (nb == 2 && kc == 16) EFWI_NN_CONV_PIPE(2, true);
+      else if (nb == 2) EFWI_NN_CONV_PIPE(2, false);
+      else if (kc == 16) EFWI_NN_CONV_PIPE(1, true);
+      else EFWI_NN_CONV_PIPE(1, false);
+#undef EFWI_NN_CONV_PIPE
+      return nn_check(s);
+    }
+  }
   // where the bricks times the output-block groups would give fewer than four
   // workgroups per CU (the coarser levels), one block per workgroup: more
   // workgroups, whose wavefronts hide each other's load latency (48x64x64
   // voxels: 32->32 27.7 -> 22.5 us, 96->32 82 -> 75 us)
   int NB = nbt % 4 == 0 ? 4 : nbt % 3 == 0 ? 3 : nbt % 2 == 0 ? 2 : 1;
   if (bricks * (nbt / NB) < 4L * device_cus()) NB = 1;
-  const int per_xcd = (int)((bricks + 7) / 8);
   const dim3 grid((unsigned)(8L * per_xcd), (unsigned)(nbt / NB));
-  // outputs (and mask) as 16-byte granules where the pointers allow
-  const int vec_out = (uintptr_t)dst % 16 == 0 && (uintptr_t)dst2 % 16 == 0 && (!mask || (uintptr_t)mask % 16 == 0);
 #define EFWI_NN_CONV_LAUNCH(CK, M, B, MODE)                                                                       \
   hipLaunchKernelGGL((k_conv3<CK, M, B, MODE>), grid, dim3(128 * conv_tz(M)), 0, s, src, lds, kc, w, bias, dst,  \
                      ldd, nc, mask, ldm, V, relu, ntz, ntx, nty, per_xcd, vec_out, src2, lds2, kc1, dst2, ldd2,   \
                      nc1, up1 ? 1 : 0)
-#define EFWI_NN_CONV_MODE(CK, M, B)                         \
-  if (mode == 0) { EFWI_NN_CONV_LAUNCH(CK, M, B, 0); }    \
+  // (rows of 64 voxels that are left to k_conv3 in mode 0 are too few for NB > 1)
+#define EFWI_NN_CONV_MODE(CK, M, B)                                      \
+  if (mode == 0) { EFWI_NN_CONV_LAUNCH(CK, M, (M == 4 ? 1 : B), 0); }  \
   else { EFWI_NN_CONV_LAUNCH(CK, M, B, 1); }
 #define EFWI_NN_CONV_NB(CK, M)                              \
   if (NB == 4) { EFWI_NN_CONV_MODE(CK, M, 4) }             \
