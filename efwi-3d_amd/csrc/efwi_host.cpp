@@ -235,6 +235,7 @@ int Ctx::init() {
   G.pxy = (long)c.nx * G.py;
   G.dz = c.dz; G.dx = c.dx; G.dy = c.dy; G.dt = c.dt;
   N = (long)c.nz * G.pxy;
+  tiles[K_VELOCITY_BWD] = tiles[K_STRESS_BWD] = default_bwd_tile(G);
   // field groups: fields fs bytes apart (256-byte aligned), each group below 4 GiB
   const size_t fs = ((size_t)N * sizeof(float) + 255) / 256 * 256;
   if (fs * P_PSI_COUNT > 0xFFFFFFFFull)

@@ -78,6 +78,8 @@ struct RecvFold {
   int nrec;
 };
 bool recv_foldable(Tile t, const Geom& G, bool forward);
+// launch shape of the two backward kernels before a caller or the autotuner sets one
+Tile default_bwd_tile(const Geom& G);
 bool launch_stress_fwd(Tile t, const Geom& G, const Groups& F, const Prof& C, const Source& S, int it,
                        hipStream_t s, const RingFold* ring = nullptr);
 bool launch_velocity_fwd(Tile t, int form, const Geom& G, const Groups& F, const Prof& C, hipStream_t s,

@@ -1539,6 +1539,15 @@ bool launch_stress_fwd(Tile t, const Geom& G, const Groups& F, const Prof& C, co
   EFWI_FLAT(Sw, k_stress_fwd<, Sw, G, F, C, S, it, Rf);
   return Rf.slot != nullptr;
 }
+// The backward kernels of large grids read more planes of z neighbours than
+// stay in the L2s between two z planes of a launch: from 256 wavefronts of 64
+// cells per CU on, two z planes per workgroup re-read them sooner. 160x240x240
+// cells velocity 367 -> 351 us, stress 368 -> 359; 200x360x360 876 -> 860 and
+// 917 -> 917; below, and for the two-row wavefronts, one plane is as fast or faster.
+Tile default_bwd_tile(const Geom& G) {
+  const Sweep S = sweep_flat(G, Tile{1, 1});
+  return S.ly == 64 && (long)(G.nz - 4) * (G.nx - 4) * S.nyb >= 256L * 256 ? Tile{1, 2} : Tile{1, 1};
+}
 // Receivers are folded up to 256 (forward) and 128 (backward) wavefronts per
 // CU: on larger grids the kernels lose more to the folded form's registers
 // (velocity_bwd 117 -> 123) than the launches cost. A gradient of 44^3 cells

@@ -100,3 +100,30 @@ def test_batch_steps_replayed_and_launched(nt):
             assert torch.equal(syns[k], syn)
             for a, b, c in zip(grads[k], P.gradient(), P.batch_gradient(k)):
                 assert torch.equal(a, b) and torch.equal(c, b)
+
+
+@pytest.mark.parametrize("ny,depth", [(61 * 64, 2), (60 * 64, 1)])
+def test_backward_shape_of_large_grids(ny, depth):
+    """From 256 wavefronts per CU on, the backward kernels take two z planes per
+    workgroup (an odd number of planes here); results are those of one."""
+    from efwi import synth
+    npml = 4
+    w = synth.small(n=37 - 2 * npml, npml=npml, nt=40, ny=ny - 2 * npml)
+    nz, nx, _ = w.grid.shape
+    z, x, y = w.shots[0].src
+    w.shots[0].rec = np.array([(z + 1, x, y), (z + 2, x + 1, y - 2)], np.int32)
+    assert ((nz - 4) * (nx - 4) * ((ny - 3) // 64 + 1) >= 65536) == (depth == 2)
+    shapes = []
+
+    def one_plane(P):
+        for k in ("velocity_bwd", "stress_bwd"):
+            shapes.append(P.tiles()[k])
+            P.set_tile(k, 1, 1)
+
+    rng = np.random.default_rng(1)
+    obs = [rng.standard_normal((3, len(s.rec), w.grid.nt)).astype(np.float32) for s in w.shots]
+    a = _gradient(w, obs)
+    b = _gradient(w, obs, one_plane)
+    assert shapes == [(1, depth)] * 2
+    for x, y in zip(a[2], b[2]):
+        assert np.abs(x).max() > 0 and np.array_equal(x, y)
