@@ -375,44 +375,46 @@ __global__ __launch_bounds__(512) void k_conv3(const uint16_t* __restrict__ src,
 }
 
 
-// The convolution (mode 0) of rows of 64 voxels or more with the loads of the
-// next input chunk in flight over this one's products. A block of eight
-// wavefronts owns bricks as k_conv3's (4 z, 2 x, 64 voxels) and walks every
+// The convolution (mode 0, aligned rows) of rows of 64 voxels or more with the
+// loads of the next input chunk in flight over this one's products. A block of
+// eight wavefronts owns bricks as k_conv3's (4 z, 2 x, 64 voxels) and walks every
 // (gridDim.x / 8)-th brick of its XCD's contiguous run, 16 input channels of a
-// brick at a step; the halo is double buffered, one barrier per step.
+// brick at a step.
 //  - Each load instruction stays in one halo row, whose bounds are those of a
 //    descriptor in scalar registers (empty outside the volume and past the last
 //    step): no branch and no address per lane. The last 2 of a row's 66 voxels
 //    take one more load for all of a wavefront's rows.
-//  - The weights lie in LDS, or with 16 input channels and one output block in
-//    registers. The fragments of two tap pairs ahead are read over a pair's products.
+//  - The weights lie in LDS. The fragments of the next tap pairs are read over a
+//    pair's products.
 //  - D is computed transposed (weights x voxels): a lane holds 4 channels of a
 //    voxel and stores (and masks) them as 8 bytes; a wavefront's store is 512
 //    contiguous bytes.
+//  - One output block: a single halo buffer and 128 registers, so that two blocks
+//    share a CU and each fills the other's phases; two or three: the halo (and the
+//    chunk's weights) double buffered, one block per CU.
 // The products and their order are k_conv3's, so the results are too.
 //
-// Bound by LDS reads (14 fragments of 1 KB per 16 voxels and 14 NB products;
-// 2.9 of the 6.4 us that the 16->16 step of eight wavefronts takes at 128 bytes a
-// clock) and by the wavefronts' scalar and address work, during which the LDS
-// idles: without the loads 31 of 34 us, with one of the 14 products 24. One block
-// per CU at 170 to 255 registers; two with single buffers and 128 registers spill
-// and were slower (51 us); keeping the rows in an LDS ring along x (halo rows per
-// output row 1.5 instead of 3) changed nothing at 96x128x128. Measured, k_conv3 against this:
-// 16->16 at 96x128x128 45 -> 34 us, at 120x200x200 163 -> 112; 16->48 100 -> 66;
-// 32->32 at 60x100x100 70 -> 47, 96->32 180 -> 120; 48->16 at 120x200x200 337 -> 316.
+// Bound by LDS reads (14 fragments of 1 KB per 16 voxels and 14 NB products, and
+// with one output block a quarter more for the weights: the LDS is busy 61 % of
+// the 16->16 kernel's cycles, the matrix cores 39 %) and by the wavefronts' scalar
+// and address work. 16->16 at 96x128x128: 45 us in k_conv3, 34 with one double
+// buffered block per CU and the weights in registers, 32 so; the latter without
+// loads 31, with one of the 14 products 24. Halo rows in an LDS ring along x (1.5
+// halo rows per output row instead of 3): 34. At 120x200x200 163 -> 104; 16->48
+// 100 -> 65; 32->32 at 60x100x100 70 -> 46, 96->32 180 -> 116; 48->16 at
+// 120x200x200 337 -> 278.
 template <int NB, bool ONE>
-__global__ __launch_bounds__(512, 2) void k_conv_pipe(
+__global__ __launch_bounds__(512, NB == 1 ? 4 : 2) void k_conv_pipe(
     const uint16_t* __restrict__ src, int lds, int kc, const uint16_t* __restrict__ w, const float* __restrict__ bias,
     uint16_t* __restrict__ dst, int ldd, int nc, const uint16_t* __restrict__ mask, int ldm, Vol V, int relu,
-    int ntx, int nty, int nbricks, int per_xcd, int vec_out, const uint16_t* __restrict__ src2, int lds2, int kc1,
+    int ntx, int nty, int nbricks, int per_xcd, const uint16_t* __restrict__ src2, int lds2, int kc1,
     uint16_t* __restrict__ dst2, int ldd2, int nc1, int up1) {
   constexpr int MB = 4, TY = 16 * MB, HW = TY + 2, VB = 32, NBC = 16 * NB;
   constexpr int TZ = conv_tz(MB), NT = 128 * TZ, HR = (TZ + 2) * 4;  // halo rows
   constexpr int RPW = HR / (NT / 64);               // halo rows per wavefront
   constexpr int WU = (27 * NBC * 2 + NT - 1) / NT;  // weight granules per thread
   constexpr int HB = HR * HW * VB, WB = 27 * NBC * VB;
-  constexpr bool WR = ONE && NB == 1;  // weights in registers
-  constexpr int WBUF = ONE ? 1 : 2, WL = 2 * HB, ZERO = WL + WBUF * WB;
+  constexpr int HBUF = NB == 1 ? 1 : 2, WBUF = ONE ? 1 : HBUF, WL = HBUF * HB, ZERO = WL + WBUF * WB;
   // halo buffers, weight buffers, zeros (the 28th tap's inputs and weights)
   __shared__ __align__(16) unsigned char smem[ZERO + MB * 512];
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -513,10 +515,6 @@ __global__ __launch_bounds__(512, 2) void k_conv_pipe(
   put(0);
   put_w(0);
   __syncthreads();
-  uint4 wr[WR ? 14 : 1];
-  if (WR)
-#pragma unroll
-    for (int q = 0; q < 14; q++) wr[q] = lds_read16(smem, q == 13 ? w27 : wbase + 2 * q * NBC * VB);
   int buf = 0;
   for (;;) {
     const bool last = ONE || c0 + 16 >= kc;
@@ -524,15 +522,6 @@ __global__ __launch_bounds__(512, 2) void k_conv_pipe(
     const int z = TZ * zt + wz, x = 2 * xt + wx, y0 = yt * TY;
     const long vrow = V.vox(z, x, y0);
     const int nrow = last && z < V.nz && x < V.nx ? (V.ny - y0 < TY ? V.ny - y0 : TY) : 0;
-    // its mask
-    uint2 mk[MB][NB];
-    if (mask && vec_out) {
-#pragma unroll
-      for (int m = 0; m < MB; m++)
-#pragma unroll
-        for (int c = 0; c < NB; c++)
-          mk[m][c] = ld_row8(mask + vrow * ldm + (nb0 + c) * 16, nrow * ldm * 2, ((16 * m + i) * ldm + 4 * g) * 2);
-    }
     if (last) {
       next += step;
       yt += sy;
@@ -545,8 +534,8 @@ __global__ __launch_bounds__(512, 2) void k_conv_pipe(
     const bool more = next < end;
     fetch(more, nc0);
     if (!ONE) fetch_w(nc0);
-    // fragments of the pair (2 q, 2 q + 1), read D pairs ahead of their products
-    constexpr int D = NB > 2 ? 1 : 2;
+    // fragments of the pair (2 q, 2 q + 1), D pairs ahead of their products
+    constexpr int D = NB == 2 ? 2 : 1;
     uint4 a[D + 1][MB], bw[D + 1][NB];
     auto read = [&](int q) {
       const int tl = 2 * q, dy = tl % 3, row = tl / 9 * 4 + tl / 3 % 3;
@@ -554,12 +543,10 @@ __global__ __launch_bounds__(512, 2) void k_conv_pipe(
       const int ao = q < 13 ? pair + buf * HB : hi ? zero_in : last2 + buf * HB;
 #pragma unroll
       for (int m = 0; m < MB; m++) a[q % (D + 1)][m] = lds_read16(smem, ao + row * HW * VB + 16 * m * VB);
-      if (!WR) {
-        const int wb = WBUF > 1 ? buf * WB : 0;
+      const int wb = WBUF > 1 ? buf * WB : 0;
 #pragma unroll
-        for (int c = 0; c < NB; c++)
-          bw[q % (D + 1)][c] = lds_read16(smem, q == 13 && hi ? w27 : wb + wbase + (tl * NBC + 16 * c) * VB);
-      }
+      for (int c = 0; c < NB; c++)
+        bw[q % (D + 1)][c] = lds_read16(smem, q == 13 && hi ? w27 : wb + wbase + (tl * NBC + 16 * c) * VB);
     };
 #pragma unroll
     for (int q = 0; q < D; q++) read(q);
@@ -571,39 +558,39 @@ __global__ __launch_bounds__(512, 2) void k_conv_pipe(
 #pragma unroll
         for (int c = 0; c < NB; c++)
           acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              __builtin_bit_cast(bf8, WR ? wr[WR ? q : 0] : bw[q % (D + 1)][c]), __builtin_bit_cast(bf8, a[q % (D + 1)][m]),
+              __builtin_bit_cast(bf8, bw[q % (D + 1)][c]), __builtin_bit_cast(bf8, a[q % (D + 1)][m]),
               ONE && q == 0 ? f4{0.f, 0.f, 0.f, 0.f} : acc[m][c], 0, 0, 0);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
     if (last) {
+      uint2 mk[MB][NB];
+      if (mask)
+#pragma unroll
+        for (int m = 0; m < MB; m++)
+#pragma unroll
+          for (int c = 0; c < NB; c++)
+            mk[m][c] = ld_row8(mask + vrow * ldm + (nb0 + c) * 16, nrow * ldm * 2, ((16 * m + i) * ldm + 4 * g) * 2);
       // D[channel 4 g + j][voxel i] of each (row block, column block)
 #pragma unroll
       for (int c = 0; c < NB; c++) {
-        const int n0 = (nb0 + c) * 16, n = n0 + 4 * g;
-        const int od = n0 < nc1 ? ldd : ldd2;
+        const int n0 = (nb0 + c) * 16, od = n0 < nc1 ? ldd : ldd2;
         uint16_t* const out = n0 < nc1 ? dst + vrow * ldd + n0 : dst2 + vrow * ldd2 + (n0 - nc1);
 #pragma unroll
         for (int m = 0; m < MB; m++) {
-          const int v = 16 * m + i;
           f4 r = acc[m][c] + bn[c];
           if (relu)
 #pragma unroll
             for (int jj = 0; jj < 4; jj++) r[jj] = fmaxf(r[jj], 0.f);
-          if (vec_out) {
-            if (mask) {
-              if (!(__uint_as_float(mk[m][c].x << 16) > 0.f)) r[0] = 0.f;
-              if (!(__uint_as_float(mk[m][c].x & 0xFFFF0000u) > 0.f)) r[1] = 0.f;
-              if (!(__uint_as_float(mk[m][c].y << 16) > 0.f)) r[2] = 0.f;
-              if (!(__uint_as_float(mk[m][c].y & 0xFFFF0000u) > 0.f)) r[3] = 0.f;
-            }
-            typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
-            st_row8(out, nrow * od * 2, (v * od + 4 * g) * 2, __builtin_bit_cast(uint2, __builtin_convertvector(r, bf4)));
-          } else if (v < nrow) {
-#pragma unroll
-            for (int jj = 0; jj < 4; jj++)
-              out[(long)v * od + 4 * g + jj] = f2bf(mask && !(bf2f(mask[(vrow + v) * ldm + n + jj]) > 0.f) ? 0.f : r[jj]);
+          if (mask) {
+            if (!(__uint_as_float(mk[m][c].x << 16) > 0.f)) r[0] = 0.f;
+            if (!(__uint_as_float(mk[m][c].x & 0xFFFF0000u) > 0.f)) r[1] = 0.f;
+            if (!(__uint_as_float(mk[m][c].y << 16) > 0.f)) r[2] = 0.f;
+            if (!(__uint_as_float(mk[m][c].y & 0xFFFF0000u) > 0.f)) r[3] = 0.f;
           }
+          typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
+          st_row8(out, nrow * od * 2, ((16 * m + i) * od + 4 * g) * 2,
+                  __builtin_bit_cast(uint2, __builtin_convertvector(r, bf4)));
         }
       }
       if (!ONE)
@@ -613,7 +600,8 @@ __global__ __launch_bounds__(512, 2) void k_conv_pipe(
           for (int c = 0; c < NB; c++) acc[m][c] = f4{0.f, 0.f, 0.f, 0.f};
     }
     if (!more) break;
-    buf ^= 1;
+    if (HBUF > 1) buf ^= 1;
+    else __syncthreads();
     put(buf);
     if (!ONE) put_w(buf);
     c0 = nc0;
@@ -1507,20 +1495,20 @@ int efwi_nn_conv3_cat(const uint16_t* src, int lds, int kc1, int up1, const uint
   const int per_xcd = (int)((bricks + 7) / 8);
   // outputs (and mask) as 8- and 16-byte granules where the pointers allow
   const int vec_out = (uintptr_t)dst % 16 == 0 && (uintptr_t)dst2 % 16 == 0 && (!mask || (uintptr_t)mask % 16 == 0);
-  // Rows of 64 voxels or more in mode 0: the pipelined kernel, one block per CU,
-  // with the most output blocks that still give every CU three bricks or more
-  // (a last round of few bricks costs as much as a full one: 32->16 at 48x64x64,
-  // 384 bricks, 13.3 us against k_conv3's 12.7; 16->32, 384 bricks at two blocks
-  // 12.5 us, 768 at one 11.6 against 14.5). Three blocks' weights fit LDS only
-  // with one chunk of input channels.
-  if (MB == 4 && mode == 0 && bricks <= INT_MAX - 8L * device_cus()) {
+  // Rows of 64 voxels or more in mode 0: the pipelined kernel (one block per CU,
+  // with one output block two) with the most output blocks that still give every
+  // CU one and a half bricks, or two with one output block (48x64x64, 384 bricks:
+  // 32->32 18.6 us at two output blocks and 21.6 at one against k_conv3's 21.1,
+  // 96->32 42.5 and 50.5 against 47.7; 32->16 13.3 against 12.7). Three output
+  // blocks' weights fit LDS only with one chunk of input channels.
+  if (MB == 4 && mode == 0 && vec_out && bricks <= INT_MAX - 8L * device_cus()) {
     const int most = kc == 16 ? 3 : 2;
     for (int nb = most; nb >= 1; nb--) {
-      if (nbt % nb || bricks * (nbt / nb) < (nb > 1 ? 3L : 2L) * device_cus()) continue;
-      const dim3 pgrid(8u * std::max(1, std::min(per_xcd, device_cus() / 8 / (nbt / nb))), (unsigned)(nbt / nb));
+      if (nbt % nb || 2 * bricks * (nbt / nb) < (nb > 1 ? 3L : 4L) * device_cus()) continue;
+      const dim3 pgrid(8u * std::max(1, std::min(per_xcd, (nb == 1 ? 2 : 1) * device_cus() / 8 / (nbt / nb))), (unsigned)(nbt / nb));
 #define EFWI_NN_CONV_PIPE(B, ONE)                                                                               \
   hipLaunchKernelGGL((k_conv_pipe<B, ONE>), pgrid, dim3(512), 0, s, src, lds, kc, w, bias, dst, ldd, nc, mask, ldm, \
-                     V, relu, ntx, nty, (int)bricks, per_xcd, vec_out, src2, lds2, kc1, dst2, ldd2, nc1, up1 ? 1 : 0)
+                     V, relu, ntx, nty, (int)bricks, per_xcd, src2, lds2, kc1, dst2, ldd2, nc1, up1 ? 1 : 0)
       if (nb == 3) EFWI_NN_CONV_PIPE(3, true);
       else if (nb == 2 && kc == 16) EFWI_NN_CONV_PIPE(2, true);
       else if (nb == 2) EFWI_NN_CONV_PIPE(2, false);
@@ -1536,12 +1524,13 @@ int efwi_nn_conv3_cat(const uint16_t* src, int lds, int kc1, int up1, const uint
   // voxels: 32->32 27.7 -> 22.5 us, 96->32 82 -> 75 us)
   int NB = nbt % 4 == 0 ? 4 : nbt % 3 == 0 ? 3 : nbt % 2 == 0 ? 2 : 1;
   if (bricks * (nbt / NB) < 4L * device_cus()) NB = 1;
+  // (in mode 0, rows of 64 voxels come here for small volumes and unaligned outputs: one block)
+  if (MB == 4 && mode == 0) NB = 1;
   const dim3 grid((unsigned)(8L * per_xcd), (unsigned)(nbt / NB));
 #define EFWI_NN_CONV_LAUNCH(CK, M, B, MODE)                                                                       \
   hipLaunchKernelGGL((k_conv3<CK, M, B, MODE>), grid, dim3(128 * conv_tz(M)), 0, s, src, lds, kc, w, bias, dst,  \
                      ldd, nc, mask, ldm, V, relu, ntz, ntx, nty, per_xcd, vec_out, src2, lds2, kc1, dst2, ldd2,   \
                      nc1, up1 ? 1 : 0)
-  // (rows of 64 voxels that are left to k_conv3 in mode 0 are too few for NB > 1)
 #define EFWI_NN_CONV_MODE(CK, M, B)                                      \
   if (mode == 0) { EFWI_NN_CONV_LAUNCH(CK, M, (M == 4 ? 1 : B), 0); }  \
   else { EFWI_NN_CONV_LAUNCH(CK, M, B, 1); }

@@ -45,7 +45,9 @@ def _host(t):
 PLAIN = [((33, 125, 66), 16, 16, 1, 0, 0), ((31, 129, 64), 16, 32, 0, 16, 0), ((33, 63, 127), 16, 48, 1, 0, 0),
          ((29, 131, 65), 32, 32, 0, 0, 0), ((30, 66, 130), 48, 16, 1, 16, 0), ((33, 125, 66), 16, 16, 1, 16, 4),
          # one brick fewer than the pipelined kernel takes, and just enough
-         ((4, 1022, 64), 16, 16, 0, 0, 0), ((4, 1024, 64), 16, 16, 0, 0, 0)]
+         ((4, 1022, 64), 16, 16, 0, 0, 0), ((4, 1024, 64), 16, 16, 0, 0, 0),
+         # one brick fewer than two output blocks per workgroup take, and just enough
+         ((4, 766, 64), 16, 32, 1, 0, 0), ((4, 768, 64), 32, 32, 1, 0, 0)]
 
 
 @pytest.mark.parametrize("dims,kc,nc,relu,pad,off", PLAIN)
