@@ -375,15 +375,15 @@ __global__ __launch_bounds__(512) void k_conv3(const uint16_t* __restrict__ src,
 }
 
 
-// The convolution (mode 0, aligned rows) of rows of 64 voxels or more with the
+// The convolution (mode 0, aligned outputs) of rows of 32 voxels or more with the
 // loads of the next input chunk in flight over this one's products. A block of
-// eight wavefronts owns bricks as k_conv3's (4 z, 2 x, 64 voxels) and walks every
-// (gridDim.x / 8)-th brick of its XCD's contiguous run, 16 input channels of a
-// brick at a step.
+// eight wavefronts owns bricks of 4 (z) x 2 (x) rows of 16 MB voxels and walks
+// every (gridDim.x / 8)-th brick of its XCD's contiguous run, 16 input channels of
+// a brick at a step.
 //  - Each load instruction stays in one halo row, whose bounds are those of a
 //    descriptor in scalar registers (empty outside the volume and past the last
-//    step): no branch and no address per lane. The last 2 of a row's 66 voxels
-//    take one more load for all of a wavefront's rows.
+//    step): no branch and no address per lane. The last 2 of a row's 16 MB + 2
+//    voxels take one more load for all of a wavefront's rows.
 //  - The weights lie in LDS. The fragments of the next tap pairs are read over a
 //    pair's products.
 //  - D is computed transposed (weights x voxels): a lane holds 4 channels of a
@@ -398,19 +398,19 @@ __global__ __launch_bounds__(512) void k_conv3(const uint16_t* __restrict__ src,
 // with one output block a quarter more for the weights: the LDS is busy 61 % of
 // the 16->16 kernel's cycles, the matrix cores 39 %) and by the wavefronts' scalar
 // and address work. 16->16 at 96x128x128: 45 us in k_conv3, 34 with one double
-// buffered block per CU and the weights in registers, 32 so; the latter without
-// loads 31, with one of the 14 products 24. Halo rows in an LDS ring along x (1.5
-// halo rows per output row instead of 3): 34. At 120x200x200 163 -> 104; 16->48
-// 100 -> 65; 32->32 at 60x100x100 70 -> 46, 96->32 180 -> 116; 48->16 at
-// 120x200x200 337 -> 278.
-template <int NB, bool ONE>
+// buffered block per CU and the weights in registers (31 without its loads, 24 with
+// one of the 14 products), 32 so; halo rows in an LDS ring along x (1.5 halo rows
+// per output row instead of 3) 34. At 120x200x200 163 -> 104; 16->48 100 -> 65;
+// 32->32 at 60x100x100 70 -> 46, 96->32 180 -> 116; 48->16 at 120x200x200 337 ->
+// 278; rows of 32 to 63 voxels: 64->64 at 24x32x32 17 -> 12, at 30x50x50 50 -> 37.
+template <int MB, int NB, bool ONE>
 __global__ __launch_bounds__(512, NB == 1 ? 4 : 2) void k_conv_pipe(
     const uint16_t* __restrict__ src, int lds, int kc, const uint16_t* __restrict__ w, const float* __restrict__ bias,
     uint16_t* __restrict__ dst, int ldd, int nc, const uint16_t* __restrict__ mask, int ldm, Vol V, int relu,
     int ntx, int nty, int nbricks, int per_xcd, const uint16_t* __restrict__ src2, int lds2, int kc1,
     uint16_t* __restrict__ dst2, int ldd2, int nc1, int up1) {
-  constexpr int MB = 4, TY = 16 * MB, HW = TY + 2, VB = 32, NBC = 16 * NB;
-  constexpr int TZ = conv_tz(MB), NT = 128 * TZ, HR = (TZ + 2) * 4;  // halo rows
+  constexpr int TY = 16 * MB, HW = TY + 2, VB = 32, NBC = 16 * NB, NM = MB / 2;  // NM: 64-granule loads of a row
+  constexpr int TZ = 4, NT = 128 * TZ, HR = (TZ + 2) * 4;  // halo rows
   constexpr int RPW = HR / (NT / 64);               // halo rows per wavefront
   constexpr int WU = (27 * NBC * 2 + NT - 1) / NT;  // weight granules per thread
   constexpr int HB = HR * HW * VB, WB = 27 * NBC * VB;
@@ -439,11 +439,11 @@ __global__ __launch_bounds__(512, NB == 1 ? 4 : 2) void k_conv_pipe(
   // the coordinates of the next brick, and those of a step
   int yt = next % nty, xt = next / nty % ntx, zt = next / nty / ntx;
   const int sy = step % nty, sx = step / nty % ntx, sz = step / nty / ntx;
-  uint4 hq[RPW * 2], tq, wq[WU];  // halo rows, their last voxels, weights
+  uint4 hq[RPW * NM], tq, wq[WU];  // halo rows, their last voxels, weights
   bool tok = false;
   const int gr16 = 16 * (lane & 1);
   // the row and voxel of the lane's granule of the last two voxels
-  const int trow = wv * RPW + (lane >> 2), tvox = 64 + ((lane >> 1) & 1);
+  const int trow = wv * RPW + (lane >> 2), tvox = TY + ((lane >> 1) & 1);
   auto fetch = [&](bool live, int c0) {
     const int z0 = TZ * zt - 1, x0 = 2 * xt - 1, y0 = yt * TY;
     const bool second = !ONE && c0 >= kc1;
@@ -462,8 +462,8 @@ __global__ __launch_bounds__(512, NB == 1 ? 4 : 2) void k_conv_pipe(
       const int r = wv * RPW + u, hz = r >> 2, hx = r & 3;
       const bool in = (unsigned)(z0 + hz) < (unsigned)V.nz && (unsigned)(x0 + hx) < (unsigned)V.nx;
       const unsigned char* const row = base + (unsigned long)(unsigned)(((hz + ush) >> ush) * unx + ((hx + ush) >> ush)) * rb;
-      hq[2 * u] = ld_row(row, in ? bytes : 0, voff0);
-      hq[2 * u + 1] = ld_row(row, in ? bytes : 0, voff + (32 >> ush) * (int)sl2);
+      hq[NM * u] = ld_row(row, in ? bytes : 0, voff0);
+      if (NM == 2) hq[NM * u + NM - 1] = ld_row(row, in ? bytes : 0, voff + (32 >> ush) * (int)sl2);
     }
     const int hz = trow >> 2, hx = trow & 3;
     tok = live && lane < 4 * RPW && (unsigned)(z0 + hz) < (unsigned)V.nz && (unsigned)(x0 + hx) < (unsigned)V.nx &&
@@ -487,7 +487,7 @@ __global__ __launch_bounds__(512, NB == 1 ? 4 : 2) void k_conv_pipe(
 #pragma unroll
     for (int u = 0; u < RPW; u++)
 #pragma unroll
-      for (int m = 0; m < 2; m++) st16(p + (u * HW + 32 * m) * VB, hq[2 * u + m]);
+      for (int m = 0; m < NM; m++) st16(p + (u * HW + 32 * m) * VB, hq[NM * u + m]);
     if (lane < 4 * RPW)
       st16(smem + buf * HB + (trow * HW + tvox) * VB + 16 * ((lane & 1) ^ granule_swizzle<16>(tvox)),
            tok ? tq : uint4{0u, 0u, 0u, 0u});
@@ -1492,31 +1492,36 @@ int efwi_nn_conv3_cat(const uint16_t* src, int lds, int kc1, int up1, const uint
   const int TZ = conv_tz(MB);
   const int ntz = (nz + TZ - 1) / TZ, ntx = (nx + 1) / 2, nty = (ny + 16 * MB - 1) / (16 * MB);
   const long bricks = (long)ntz * ntx * nty;
-  const int per_xcd = (int)((bricks + 7) / 8);
   // outputs (and mask) as 8- and 16-byte granules where the pointers allow
   const int vec_out = (uintptr_t)dst % 16 == 0 && (uintptr_t)dst2 % 16 == 0 && (!mask || (uintptr_t)mask % 16 == 0);
-  // Rows of 64 voxels or more in mode 0: the pipelined kernel (one block per CU,
-  // with one output block two) with the most output blocks that still give every
-  // CU one and a half bricks, or two with one output block (48x64x64, 384 bricks:
-  // 32->32 18.6 us at two output blocks and 21.6 at one against k_conv3's 21.1,
-  // 96->32 42.5 and 50.5 against 47.7; 32->16 13.3 against 12.7). Three output
-  // blocks' weights fit LDS only with one chunk of input channels.
-  if (MB == 4 && mode == 0 && vec_out && bricks <= INT_MAX - 8L * device_cus()) {
-    const int most = kc == 16 ? 3 : 2;
-    for (int nb = most; nb >= 1; nb--) {
-      if (nbt % nb || 2 * bricks * (nbt / nb) < (nb > 1 ? 3L : 4L) * device_cus()) continue;
-      const dim3 pgrid(8u * std::max(1, std::min(per_xcd, (nb == 1 ? 2 : 1) * device_cus() / 8 / (nbt / nb))), (unsigned)(nbt / nb));
-#define EFWI_NN_CONV_PIPE(B, ONE)                                                                               \
-  hipLaunchKernelGGL((k_conv_pipe<B, ONE>), pgrid, dim3(512), 0, s, src, lds, kc, w, bias, dst, ldd, nc, mask, ldm, \
-                     V, relu, ntx, nty, (int)bricks, per_xcd, src2, lds2, kc1, dst2, ldd2, nc1, up1 ? 1 : 0)
-      if (nb == 3) EFWI_NN_CONV_PIPE(3, true);
-      else if (nb == 2 && kc == 16) EFWI_NN_CONV_PIPE(2, true);
-      else if (nb == 2) EFWI_NN_CONV_PIPE(2, false);
-      else if (kc == 16) EFWI_NN_CONV_PIPE(1, true);
-      else EFWI_NN_CONV_PIPE(1, false);
+  // Rows of 32 voxels or more in mode 0: the pipelined kernel, with three (one
+  // chunk of input channels; more weights do not fit LDS) or two output blocks per
+  // workgroup where one would give every CU more than one workgroup (64->64 at
+  // 24x32x32, 384 workgroups of one: 12.6 us at two, 16.5 at one, 18.3 in k_conv3;
+  // at 16x32x32, 256 of one: 11.8, 10.9, 14.8). With 16 input channels and short
+  // rows a workgroup per CU has nothing to overlap: k_conv3 there (16->16 at
+  // 24x32x32 5.3 us against 5.7).
+  const long pbricks = (long)((nz + 3) / 4) * ntx * nty;
+  const bool many = pbricks * nbt > device_cus();
+  if (MB >= 2 && mode == 0 && vec_out && pbricks <= INT_MAX - 8L * device_cus() && (many || MB == 4 || kc > 16)) {
+    const int nb = many && kc == 16 && nbt % 3 == 0 ? 3 : many && nbt % 2 == 0 ? 2 : 1;
+    const int pxcd = (int)((pbricks + 7) / 8);
+    const dim3 pgrid(8u * std::max(1, std::min(pxcd, (nb == 1 ? 2 : 1) * device_cus() / 8 / (nbt / nb))),
+                     (unsigned)(nbt / nb));
+#define EFWI_NN_CONV_PIPE(M, B, ONE)                                                                              \
+  hipLaunchKernelGGL((k_conv_pipe<M, B, ONE>), pgrid, dim3(512), 0, s, src, lds, kc, w, bias, dst, ldd, nc, mask, ldm, \
+                     V, relu, ntx, nty, (int)pbricks, pxcd, src2, lds2, kc1, dst2, ldd2, nc1, up1 ? 1 : 0)
+#define EFWI_NN_CONV_PIPE_NB(M)                                 \
+  if (nb == 3) EFWI_NN_CONV_PIPE(M, 3, true);                  \
+  else if (nb == 2 && kc == 16) EFWI_NN_CONV_PIPE(M, 2, true); \
+  else if (nb == 2) EFWI_NN_CONV_PIPE(M, 2, false);            \
+  else if (kc == 16) EFWI_NN_CONV_PIPE(M, 1, true);            \
+  else EFWI_NN_CONV_PIPE(M, 1, false)
+    if (MB == 4) { EFWI_NN_CONV_PIPE_NB(4); }
+    else { EFWI_NN_CONV_PIPE_NB(2); }
+#undef EFWI_NN_CONV_PIPE_NB
 #undef EFWI_NN_CONV_PIPE
-      return nn_check(s);
-    }
+    return nn_check(s);
   }
   // where the bricks times the output-block groups would give fewer than four
   // workgroups per CU (the coarser levels), one block per workgroup: more
@@ -1524,15 +1529,16 @@ int efwi_nn_conv3_cat(const uint16_t* src, int lds, int kc1, int up1, const uint
   // voxels: 32->32 27.7 -> 22.5 us, 96->32 82 -> 75 us)
   int NB = nbt % 4 == 0 ? 4 : nbt % 3 == 0 ? 3 : nbt % 2 == 0 ? 2 : 1;
   if (bricks * (nbt / NB) < 4L * device_cus()) NB = 1;
-  // (in mode 0, rows of 64 voxels come here for small volumes and unaligned outputs: one block)
-  if (MB == 4 && mode == 0) NB = 1;
+  // (in mode 0, rows of 32 voxels or more come here with unaligned outputs and in small volumes: one block)
+  if (MB >= 2 && mode == 0) NB = 1;
+  const int per_xcd = (int)((bricks + 7) / 8);
   const dim3 grid((unsigned)(8L * per_xcd), (unsigned)(nbt / NB));
 #define EFWI_NN_CONV_LAUNCH(CK, M, B, MODE)                                                                       \
   hipLaunchKernelGGL((k_conv3<CK, M, B, MODE>), grid, dim3(128 * conv_tz(M)), 0, s, src, lds, kc, w, bias, dst,  \
                      ldd, nc, mask, ldm, V, relu, ntz, ntx, nty, per_xcd, vec_out, src2, lds2, kc1, dst2, ldd2,   \
                      nc1, up1 ? 1 : 0)
 #define EFWI_NN_CONV_MODE(CK, M, B)                                      \
-  if (mode == 0) { EFWI_NN_CONV_LAUNCH(CK, M, (M == 4 ? 1 : B), 0); }  \
+  if (mode == 0) { EFWI_NN_CONV_LAUNCH(CK, M, (M >= 2 ? 1 : B), 0); }  \
   else { EFWI_NN_CONV_LAUNCH(CK, M, B, 1); }
 #define EFWI_NN_CONV_NB(CK, M)                              \
   if (NB == 4) { EFWI_NN_CONV_MODE(CK, M, 4) }             \

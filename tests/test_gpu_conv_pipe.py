@@ -1,5 +1,6 @@
-"""The pipelined convolution on the GPU at the edges of its range: volumes of
-just enough bricks, partial bricks in every direction, one to three output
+"""The pipelined convolution on the GPU at the edges of its range: rows of 32 to
+130 voxels, the smallest volumes, partial bricks in every direction, numbers of
+bricks around the ones where the output blocks per workgroup change, one to three output
 blocks per workgroup, one and several chunks of input channels, inputs kept as
 a coarse and a fine tensor, outputs split over two tensors, masks, strided and
 unaligned rows.
@@ -44,10 +45,13 @@ def _host(t):
 # (4 channels: 8-byte granules are not aligned)
 PLAIN = [((33, 125, 66), 16, 16, 1, 0, 0), ((31, 129, 64), 16, 32, 0, 16, 0), ((33, 63, 127), 16, 48, 1, 0, 0),
          ((29, 131, 65), 32, 32, 0, 0, 0), ((30, 66, 130), 48, 16, 1, 16, 0), ((33, 125, 66), 16, 16, 1, 16, 4),
-         # one brick fewer than the pipelined kernel takes, and just enough
-         ((4, 1022, 64), 16, 16, 0, 0, 0), ((4, 1024, 64), 16, 16, 0, 0, 0),
-         # one brick fewer than two output blocks per workgroup take, and just enough
-         ((4, 766, 64), 16, 32, 1, 0, 0), ((4, 768, 64), 32, 32, 1, 0, 0)]
+         # as many workgroups of one output block as CUs, and more
+         ((4, 256, 64), 32, 32, 1, 0, 0), ((4, 258, 64), 32, 32, 1, 0, 0), ((16, 32, 32), 64, 64, 0, 0, 0),
+         ((24, 32, 32), 64, 64, 1, 16, 0), ((23, 33, 50), 16, 48, 1, 0, 0), ((15, 31, 40), 16, 48, 0, 0, 0),
+         ((41, 51, 33), 16, 16, 1, 0, 0),
+         # small volumes and short rows
+         ((1, 1, 32), 32, 16, 0, 0, 0), ((1, 2, 64), 16, 16, 1, 0, 0), ((5, 7, 33), 48, 16, 1, 16, 0),
+         ((9, 6, 63), 32, 32, 0, 0, 0), ((5, 3, 95), 16, 32, 1, 0, 0), ((9, 6, 47), 32, 16, 1, 0, 4)]
 
 
 @pytest.mark.parametrize("dims,kc,nc,relu,pad,off", PLAIN)
@@ -79,7 +83,8 @@ def test_convolution(dims, kc, nc, relu, pad, off, masked):
 
 @pytest.mark.parametrize("dims,k1,k2,n1,n2,up", [((34, 126, 66), 32, 16, 16, 0, 1), ((36, 62, 130), 64, 32, 32, 0, 1),
                                                  ((33, 63, 129), 16, 0, 32, 16, 0), ((33, 65, 127), 32, 0, 64, 32, 0),
-                                                 ((31, 129, 65), 16, 32, 16, 0, 0)])
+                                                 ((31, 129, 65), 16, 32, 16, 0, 0), ((12, 22, 34), 64, 32, 32, 0, 1),
+                                                 ((2, 2, 62), 16, 16, 16, 0, 1), ((25, 33, 35), 64, 0, 64, 32, 0)])
 def test_joined_inputs_and_outputs(dims, k1, k2, n1, n2, up):
     from efwi import _native as N
     rng = np.random.default_rng(sum(dims) + k1)
