@@ -665,18 +665,19 @@ __global__ void k_flip_many(FlipSet S) {
 // the bias gradient of their m block) into part[chunk][27 mc kc + m]; a chunk's
 // partials are 27 mc kc + mc floats.
 //
-// Bound by the instructions of a step (54 products, 48 LDS reads and about 180
+// Bound by the instructions of a step (54 products, 48 LDS reads and about 140
 // scalar and 60 vector instructions that fetch and store the next rows, at two
-// wavefronts per SIMD: 27 accumulators and two steps' rows take 210 registers)
+// wavefronts per SIMD: 27 accumulators and two steps' rows take 208 registers)
 // and, at 16x16 channels, by the fixed cost of a block (ring start, sums of the
 // wavefronts, partials). Before, operands were transposed by shifts and 8-byte
 // LDS stores, a wavefront read 19 KB of LDS per 432 matrix-core cycles, and
 // every load had its own bounds branches. With k_sum_chunks, at 12 bricks per
-// block: 96x128x128 voxels 16x16 channels 83 -> 37 us, 75x101x131 84 -> 35;
-// 16x48 at 24 bricks 172 -> 80. With the ring but loads behind bounds branches
-// 40 us; one step in flight instead of two changes nothing then. Blocks of a
-// chunk on different XCDs (n block slowest): 16x48 122 us, 32x96 at 48x64x64
-// 96 against 48.
+// block: 96x128x128 voxels 16x16 channels 83 -> 37 us, 75x101x131 84 -> 33;
+// 16x48 at 24 bricks 172 -> 76. With the ring but loads behind bounds branches
+// 40 us; one step in flight instead of two changes nothing then. Row addresses by
+// 64-bit products per plane instead of one per step: 38.5, 35 and 81 us. Blocks of
+// a chunk on different XCDs (n block slowest): 16x48 122 us, 32x96 at 48x64x64 96
+// against 48.
 typedef __attribute__((address_space(3))) unsigned char lds_u8;
 __device__ __forceinline__ bf8 tr_fragment(const lds_u8* p) {
   struct {
@@ -730,20 +731,28 @@ __global__ __launch_bounds__(256, 2) void k_wgrad(const uint16_t* __restrict__ d
 #pragma unroll
   for (int u = 0; u < NB; u++) b_off[u] = (((((lane + 64 * u) >> 1) - 1) >> (int)up) + 1) * (int)sl * 2 + gr2;
   const int a_row = TY == 64 ? wv >> 1 : wv & 1, a_half = TY == 64 ? 32 * (wv & 1) : 0, a_plane = TY == 64 ? 0 : wv >> 1;
-  const int ush = (int)up, unx = V.nx >> ush, uny = V.ny >> ush;
+  const int ush = (int)up, unx = V.nx >> ush;
+  // bytes of a row, and to the next load's plane
+  const unsigned a_rb = (unsigned)V.ny * ldp * 2, b_rb = (unsigned)(V.ny >> ush) * (unsigned)sl * 2;
+  const long a_step = (TY == 64 ? 1L : 2L) * V.nx * (long)a_rb;
   auto fetch = [&](bool live, uint4 (&qa)[NA], uint4 (&qb)[NB]) {
     const int y0 = fy * TY, ya = y0 + a_half, xa = 2 * fp - 1 + a_row;
     const int na = V.ny - ya < 32 ? V.ny - ya : 32;
     const int a_bytes = live && na > 0 && (unsigned)xa < (unsigned)V.nx ? na * ldp * 2 : 0;
+    const int za = 2 * fz - 1 + a_plane;
+    // (signed: the first plane may lie before the volume, and the others follow from it)
+    const unsigned char* row_a =
+        reinterpret_cast<const unsigned char*>(dpre + mb * 16 + (long)ya * ldp) + (long)(za * V.nx + xa) * (long)a_rb;
 #pragma unroll
     for (int u = 0; u < NA; u++) {
-      const int z = 2 * fz - 1 + (TY == 64 ? u : 2 * u + a_plane);
-      qa[u] = ld_row(dpre + V.vox(z, xa, ya) * ldp + mb * 16, (unsigned)z < (unsigned)V.nz ? a_bytes : 0, a_off);
+      qa[u] = ld_row(row_a, (unsigned)(za + (TY == 64 ? u : 2 * u)) < (unsigned)V.nz ? a_bytes : 0, a_off);
+      row_a += a_step;
     }
     const int z = 2 * fz + (wv >> 1), x = 2 * fp - 2 + (wv & 1);
     const int nv = ((V.ny - y0) >> ush) + 1 < TY + 2 ? ((V.ny - y0) >> ush) + 1 : TY + 2;
     const int b_bytes = live && (unsigned)z < (unsigned)V.nz && (unsigned)x < (unsigned)V.nx ? nv * (int)sl * 2 : 0;
-    const uint16_t* const row = sb + (((long)(z >> ush) * unx + (x >> ush)) * uny + (y0 >> ush) - 1) * sl + scol;
+    const unsigned char* const row = reinterpret_cast<const unsigned char*>(sb + scol + (long)((y0 >> ush) - 1) * sl) +
+                                     (long)((z >> ush) * unx + (x >> ush)) * (long)b_rb;
 #pragma unroll
     for (int u = 0; u < NB; u++)
       qb[u] = ld_row(row, b_bytes, u == 0 && fy == 0 && lane < 2 ? (int)0x80000000 : b_off[u]);  // y = -1
@@ -757,7 +766,7 @@ __global__ __launch_bounds__(256, 2) void k_wgrad(const uint16_t* __restrict__ d
   };
   auto put = [&](int slot, int par, const uint4 (&qa)[NA], const uint4 (&qb)[NB]) {
 #pragma unroll
-    for (int u = 0; u < NA; u++) st16(smem + slot * A_SLOT + (tid + 256 * u) * 16, qa[u]);
+    for (int u = 0; u < NA; u++) st16(smem + slot + (tid + 256 * u) * 16, qa[u]);
 #pragma unroll
     for (int u = 0; u < NB; u++)
       if (lane + 64 * u < 2 * (TY + 2)) st16(smem + A_BYTES + par * B_BUF + wv * B_ROW + (lane + 64 * u) * 16, qb[u]);
@@ -777,7 +786,7 @@ __global__ __launch_bounds__(256, 2) void k_wgrad(const uint16_t* __restrict__ d
       for (int dxi = 0; dxi < 3; dxi++) {
         // the dpre row of tap dx = dxi - 1: x0 + xr - dx, of the four from x0 - 1
         const int r = xr + 2 - dxi;
-        const lds_u8* const ap = l0 + (r < 2 ? prev : cur) * A_SLOT + (2 * zp + (r & 1)) * A_ROW + c * 1024;
+        const lds_u8* const ap = l0 + (r < 2 ? prev : cur) + (2 * zp + (r & 1)) * A_ROW + c * 1024;
 #pragma unroll
         for (int dzi = 0; dzi < 3; dzi++) {
           const bf8 a = tr_fragment(ap + 2 * (2 - dzi) * A_ROW);
@@ -800,7 +809,7 @@ __global__ __launch_bounds__(256, 2) void k_wgrad(const uint16_t* __restrict__ d
   const int steps = (int)(b1 - b0 + (b1 - 1) / ntx - b0 / ntx + 1);
   int pc = fp;               // pair of the current step
   bool first = true;         // no pair of this column before it
-  int prev = 2, cur = 0;     // ring slots of the previous and the current pair
+  int prev = 2 * A_SLOT, cur = 0;  // ring slots (bytes) of the previous and the current pair
   uint4 qa0[NA], qb0[NB], qa1[NA], qb1[NB];
   auto step = [&](int s, uint4 (&qa)[NA], uint4 (&qb)[NB], const uint4 (&na)[NA], const uint4 (&nbq)[NB]) {
     fetch(s + 2 < steps, qa, qb);
@@ -808,7 +817,7 @@ __global__ __launch_bounds__(256, 2) void k_wgrad(const uint16_t* __restrict__ d
     first = pc == ntx;
     pc = first ? 0 : pc + 1;
     prev = cur;
-    cur = cur == 2 ? 0 : cur + 1;
+    cur = cur == 2 * A_SLOT ? 0 : cur + A_SLOT;
     if (s + 1 < steps) put(cur, (s + 1) & 1, na, nbq);
     __syncthreads();
   };
