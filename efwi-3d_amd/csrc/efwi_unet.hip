@@ -733,8 +733,7 @@ __global__ __launch_bounds__(256, 2) void k_wgrad(const uint16_t* __restrict__ d
   const int a_row = TY == 64 ? wv >> 1 : wv & 1, a_half = TY == 64 ? 32 * (wv & 1) : 0, a_plane = TY == 64 ? 0 : wv >> 1;
   const int ush = (int)up, unx = V.nx >> ush;
   // bytes of a row, and to the next load's plane
-  const unsigned a_rb = (unsigned)V.ny * ldp * 2, b_rb = (unsigned)(V.ny >> ush) * (unsigned)sl * 2;
-  const long a_step = (TY == 64 ? 1L : 2L) * V.nx * (long)a_rb;
+  const long a_rb = (long)V.ny * ldp * 2, b_rb = (long)(V.ny >> ush) * sl * 2, a_step = (TY == 64 ? 1L : 2L) * V.nx * a_rb;
   auto fetch = [&](bool live, uint4 (&qa)[NA], uint4 (&qb)[NB]) {
     const int y0 = fy * TY, ya = y0 + a_half, xa = 2 * fp - 1 + a_row;
     const int na = V.ny - ya < 32 ? V.ny - ya : 32;
@@ -742,7 +741,7 @@ __global__ __launch_bounds__(256, 2) void k_wgrad(const uint16_t* __restrict__ d
     const int za = 2 * fz - 1 + a_plane;
     // (signed: the first plane may lie before the volume, and the others follow from it)
     const unsigned char* row_a =
-        reinterpret_cast<const unsigned char*>(dpre + mb * 16 + (long)ya * ldp) + (long)(za * V.nx + xa) * (long)a_rb;
+        reinterpret_cast<const unsigned char*>(dpre + mb * 16 + (long)ya * ldp) + ((long)za * V.nx + xa) * a_rb;
 #pragma unroll
     for (int u = 0; u < NA; u++) {
       qa[u] = ld_row(row_a, (unsigned)(za + (TY == 64 ? u : 2 * u)) < (unsigned)V.nz ? a_bytes : 0, a_off);
@@ -752,7 +751,7 @@ __global__ __launch_bounds__(256, 2) void k_wgrad(const uint16_t* __restrict__ d
     const int nv = ((V.ny - y0) >> ush) + 1 < TY + 2 ? ((V.ny - y0) >> ush) + 1 : TY + 2;
     const int b_bytes = live && (unsigned)z < (unsigned)V.nz && (unsigned)x < (unsigned)V.nx ? nv * (int)sl * 2 : 0;
     const unsigned char* const row = reinterpret_cast<const unsigned char*>(sb + scol + (long)((y0 >> ush) - 1) * sl) +
-                                     (long)((z >> ush) * unx + (x >> ush)) * (long)b_rb;
+                                     ((long)(z >> ush) * unx + (x >> ush)) * b_rb;
 #pragma unroll
     for (int u = 0; u < NB; u++)
       qb[u] = ld_row(row, b_bytes, u == 0 && fy == 0 && lane < 2 ? (int)0x80000000 : b_off[u]);  // y = -1
@@ -1512,7 +1511,11 @@ int efwi_nn_conv3_cat(const uint16_t* src, int lds, int kc1, int up1, const uint
   // 24x32x32 5.3 us against 5.7).
   const long pbricks = (long)((nz + 3) / 4) * ntx * nty;
   const bool many = pbricks * nbt > device_cus();
-  if (MB >= 2 && mode == 0 && vec_out && pbricks <= INT_MAX - 8L * device_cus() && (many || MB == 4 || kc > 16)) {
+  // (its row numbers, row bytes and weight offsets are 32-bit)
+  const long row_bytes = 2L * ny * std::max(std::max(lds, lds2), std::max(ldd, std::max(ldd2, ldm)));
+  const bool fits = (long)nz * nx <= INT_MAX / 2 && row_bytes <= INT_MAX && 54L * nc * kc <= INT_MAX &&
+                    pbricks <= INT_MAX - 8L * device_cus();
+  if (MB >= 2 && mode == 0 && vec_out && fits && (many || MB == 4 || kc > 16)) {
     const int nb = many && kc == 16 && nbt % 3 == 0 ? 3 : many && nbt % 2 == 0 ? 2 : 1;
     const int pxcd = (int)((pbricks + 7) / 8);
     const dim3 pgrid(8u * std::max(1, std::min(pxcd, (nb == 1 ? 2 : 1) * device_cus() / 8 / (nbt / nb))),
