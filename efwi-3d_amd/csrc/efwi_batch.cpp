@@ -17,11 +17,15 @@ namespace efwi {
 
 static constexpr int kGraphSteps = 16;  // time steps per captured graph
 
-void Ctx::release_batch() {
+void Ctx::drop_batch_graphs() {
   if (batch.gf) hipGraphExecDestroy(batch.gf);
   if (batch.gb) hipGraphExecDestroy(batch.gb);
-  if (batch.cs) hipStreamDestroy(batch.cs);
   batch.gf = batch.gb = nullptr;
+}
+
+void Ctx::release_batch() {
+  drop_batch_graphs();
+  if (batch.cs) hipStreamDestroy(batch.cs);
   batch.cs = nullptr;
 }
 
@@ -79,7 +83,6 @@ int Ctx::ensure_batch(int n, int nring) {
     if ((rc = alloc((void**)&ring_k, sizeof(float) * ring_floats))) return rc;
     batch.ring.push_back(ring_k);
   }
-  if (n <= batch.n) return EFWI_OK;
   const size_t fs = G.fs;
   for (int k = batch.n; k < n; k++) {
     Groups g{};
@@ -99,8 +102,13 @@ int Ctx::ensure_batch(int n, int nring) {
     batch.rec_cap.push_back(0);
     batch.nrec.push_back(0);
   }
-  if ((rc = alloc((void**)&batch.shots_dev, sizeof(ShotDev) * n))) return rc;
-  batch.n = n;
+  if (batch.shots_cap < sizeof(ShotDev) * n) {
+    // the captured graphs hold the table's address
+    HIP_TRY(hipStreamSynchronize(batch.cs));
+    drop_batch_graphs();
+    if ((rc = grow(this, (void**)&batch.shots_dev, &batch.shots_cap, sizeof(ShotDev) * n))) return rc;
+  }
+  batch.n = std::max(batch.n, n);
   return EFWI_OK;
 }
 

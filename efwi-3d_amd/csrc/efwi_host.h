@@ -67,6 +67,7 @@ struct BatchState {
   std::vector<size_t> seis_cap, rec_cap;
   std::vector<int> nrec;
   ShotDev* shots_dev = nullptr;
+  size_t shots_cap = 0;
   unsigned* counters = nullptr;  // 2 launches per step x 8 queues
   int* it_dev = nullptr;
   hipStream_t cs = nullptr;
@@ -182,6 +183,7 @@ struct Ctx {
   int run_batch(const efwi_shot* shots, int n, int calc_id, const float* const* obs, float* const* syn,
                 double* misfits, int use_graph, hipStream_t s);
   int batch_gradient(int shot, float* gl, float* gm, float* gr, int on_host, hipStream_t s);
+  void drop_batch_graphs();
   void release_batch();
 };
 

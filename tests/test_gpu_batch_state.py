@@ -1,0 +1,63 @@
+"""What a context keeps from one batch to the next (shot table, captured graphs,
+boundary rings, launch settings): a batch gives the results of the same shots
+run one by one whatever batches ran before it."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _workload(nt, n=24, npml=6):
+    from efwi import synth
+    return synth.small(n=n, npml=npml, nt=nt)
+
+
+def _shots(w, count, seed, nrec=5):
+    """Shots with seeded sources and receivers inside the stencil box."""
+    from efwi.propagator import ShotSpec
+    rng = np.random.default_rng(seed)
+    (nz, nx, ny), p, stf = w.grid.shape, w.grid.npml, w.shots[0].stf
+    inner = lambda: tuple(int(rng.integers(p, n - p)) for n in (nz, nx, ny))  # noqa: E731
+    box = lambda: [int(rng.integers(2, n - 2)) for n in (nz, nx, ny)]  # noqa: E731
+    return [ShotSpec(inner(), stf, np.array([box() for _ in range(nrec)], np.int32)) for _ in range(count)]
+
+
+def _obs(w, shots, seed):
+    rng = np.random.default_rng(seed)
+    return [torch.from_numpy(rng.standard_normal((3, len(s.rec), w.grid.nt)).astype(np.float32)) for s in shots]
+
+
+def _open(w):
+    from efwi.propagator import Propagator
+    P = Propagator(w.grid)
+    P.set_model(*(torch.from_numpy(a) for a in w.model))
+    return P
+
+
+def _check(w, shots, obs, misfits, syns, grads):
+    with _open(w) as P:
+        for k, s in enumerate(shots):
+            P.zero_gradient()
+            j, syn, _ = P.run_shot(s, 1, obs[k], want_syn=True)
+            assert misfits[k] == j, k
+            assert torch.equal(syns[k], syn), k
+            for a, b in zip(grads[k], P.gradient()):
+                assert b.abs().max() > 0 or len(s.rec) == 0
+                assert torch.equal(a, b), k
+
+
+@pytest.mark.parametrize("use_graph", [True, False])
+def test_batch_after_a_larger_one(use_graph):
+    """A batch between two others of one size makes the shot table grow: the
+    second of them replays no graph of the first one's table."""
+    w = _workload(40)
+    first, larger, then = _shots(w, 2, 1), _shots(w, 5, 2), _shots(w, 2, 3)
+    o1, o2 = _obs(w, first, 4), _obs(w, then, 5)
+    print(f"[gpu] batch of 2, of 5 (graph={use_graph}), of 2 on {w.grid.shape}", flush=True)
+    with _open(w) as P:
+        P.run_batch(first, 1, o1)
+        P.run_batch(larger, 2, use_graph=use_graph)
+        misfits, syns = P.run_batch(then, 1, o2, want_syn=True)
+        grads = [P.batch_gradient(k) for k in range(2)]
+        _check(w, then, o2, misfits, syns, grads)
