@@ -26,6 +26,7 @@
 #include <climits>
 #include <cstdint>
 #include <mutex>
+#include <type_traits>
 
 #include "../../include/efwi_nn.h"
 
@@ -667,7 +668,7 @@ __global__ void k_flip_many(FlipSet S) {
 //
 // Bound by the instructions of a step (54 products, 48 LDS reads and about 140
 // scalar and 60 vector instructions that fetch and store the next rows, at two
-// wavefronts per SIMD: 27 accumulators and two steps' rows take 208 registers)
+// wavefronts per SIMD: 27 accumulators and two steps' rows take 214 registers)
 // and, at 16x16 channels, by the fixed cost of a block (ring start, sums of the
 // wavefronts, partials). Before, operands were transposed by shifts and 8-byte
 // LDS stores, a wavefront read 19 KB of LDS per 432 matrix-core cycles, and
@@ -697,6 +698,7 @@ __global__ __launch_bounds__(256, 2) void k_wgrad(const uint16_t* __restrict__ d
   constexpr int S_BYTES = A_BYTES + 2 * B_BUF > R_BYTES ? A_BYTES + 2 * B_BUF : R_BYTES;
   constexpr int NA = 8 * TY * 2 / 256, NB = (2 * (TY + 2) + 63) / 64;  // 16-byte loads per thread
   __shared__ __align__(16) unsigned char smem[S_BYTES];
+  __shared__ int nan_seen;
   float* red = reinterpret_cast<float*>(smem);  // after the last brick
   const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   // the channel blocks of a chunk go to one XCD (blocks are dealt to the 8 XCDs in turn), one after the other
@@ -714,17 +716,14 @@ __global__ __launch_bounds__(256, 2) void k_wgrad(const uint16_t* __restrict__ d
   const int scol = second ? nb * 16 - kc1 : nb * 16;
   // up1: src is the coarse tensor whose nearest upsampling is the input
   const bool up = up1 && !second;
-  float bsum = 0.f;  // lane (i, g): dpre channel mb * 16 + i over its voxels
+  float bsum;  // lane (i, g): dpre channel mb * 16 + i over its voxels
   f4 acc[27];
-#pragma unroll
-  for (int t = 0; t < 27; t++) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
   // Pair p of column (zt, yt): dpre rows 2 p - 1, 2 p of the planes 2 zt - 1 .. 2 zt + 2
   // and, per wavefront, one of the src rows 2 p - 2, 2 p - 1 of the planes 2 zt, 2 zt + 1,
   // voxels y0 - 1 .. y0 + TY. Every load instruction stays in one row, whose bounds are those of
   // a buffer descriptor in scalar registers (empty outside the volume and past the last step):
   // what is out of range reads as zero without a branch or an address per lane.
-  int fp = __builtin_amdgcn_readfirstlane((int)(b0 % ntx)), fz = __builtin_amdgcn_readfirstlane((int)(b0 / ntx % ntz)),
-      fy = __builtin_amdgcn_readfirstlane((int)(b0 / ((long)ntx * ntz)));
+  int fp, fz, fy;  // (p, zt, yt) of the next step to fetch
   const int gr2 = (tid & 1) * 16;
   const int a_off = (lane >> 1) * ldp * 2 + gr2;  // voxel lane / 2 of the row's 32 of this instruction
   int b_off[NB];                                  // from the voxel before the row's first
@@ -772,11 +771,13 @@ __global__ __launch_bounds__(256, 2) void k_wgrad(const uint16_t* __restrict__ d
   };
   const lds_u8* const l0 = (const lds_u8*)smem + 8 * lane;
   const int zp = wv >> 1, sub = wv & 1;
-  // the brick between the pairs in slots `prev` and `cur`
-  auto products = [&](int prev, int cur, int par) {
+  // the brick between the pairs in slots `prev` and `cur`, its first src row at (z, x)
+  auto products = [&](auto checked, int z, int x, int prev, int cur, int par) {
+    constexpr bool CHECKED = decltype(checked)::value;
 #pragma unroll
     for (int rr = 0; rr < (TY == 64 ? 2 : 1); rr++) {
       const int xr = TY == 64 ? rr : sub, c = TY == 64 ? sub : 0;
+      const bool src_in = z + zp < V.nz && x + xr < V.nx;
       const lds_u8* const bp = l0 + A_BYTES + par * B_BUF + (zp * 2 + xr) * B_ROW + c * 1024;
       bf8 b[3];
 #pragma unroll
@@ -795,62 +796,94 @@ __global__ __launch_bounds__(256, 2) void k_wgrad(const uint16_t* __restrict__ d
 #pragma unroll
             for (int k = 0; k < 4; k++) bsum += __uint_as_float(u[k] << 16) + __uint_as_float(u[k] & 0xFFFF0000u);
           }
+          if (!CHECKED || (src_in && (unsigned)(x + r - 1) < (unsigned)V.nx && (unsigned)(z + zp + 1 - dzi) < (unsigned)V.nz)) {
 #pragma unroll
-          for (int d = 0; d < 3; d++) {
-            const int t = 9 * dzi + 3 * dxi + d;
-            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[d], acc[t], 0, 0, 0);
+            for (int d = 0; d < 3; d++) {
+              const int t = 9 * dzi + 3 * dxi + d;
+              acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[d], acc[t], 0, 0, 0);
+            }
           }
         }
       }
     }
   };
-  // one step per pair; the first of a column only brings its rows
+  // the sums over the block's bricks: one step per pair, the first of a column only
+  // brings its rows. `checked`: without the products of rows outside the volume
   const int steps = (int)(b1 - b0 + (b1 - 1) / ntx - b0 / ntx + 1);
-  int pc = fp;               // pair of the current step
-  bool first = true;         // no pair of this column before it
-  int prev = 2 * A_SLOT, cur = 0;  // ring slots (bytes) of the previous and the current pair
-  uint4 qa0[NA], qb0[NB], qa1[NA], qb1[NB];
-  auto step = [&](int s, uint4 (&qa)[NA], uint4 (&qb)[NB], const uint4 (&na)[NA], const uint4 (&nbq)[NB]) {
-    fetch(s + 2 < steps, qa, qb);
-    if (!first) products(prev, cur, s & 1);
-    first = pc == ntx;
-    pc = first ? 0 : pc + 1;
-    prev = cur;
-    cur = cur == 2 * A_SLOT ? 0 : cur + A_SLOT;
-    if (s + 1 < steps) put(cur, (s + 1) & 1, na, nbq);
+  auto walk = [&](auto checked) {
+    fp = __builtin_amdgcn_readfirstlane((int)(b0 % ntx));
+    fz = __builtin_amdgcn_readfirstlane((int)(b0 / ntx % ntz));
+    fy = __builtin_amdgcn_readfirstlane((int)(b0 / ((long)ntx * ntz)));
+    bsum = 0.f;
+#pragma unroll
+    for (int t = 0; t < 27; t++) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
+    int pc = fp, pz = fz;            // pair and z tile of the current step
+    bool first = true;               // no pair of this column before it
+    int prev = 2 * A_SLOT, cur = 0;  // ring slots (bytes) of the previous and the current pair
+    uint4 qa0[NA], qb0[NB], qa1[NA], qb1[NB];
+    auto step = [&](int s, uint4 (&qa)[NA], uint4 (&qb)[NB], const uint4 (&na)[NA], const uint4 (&nbq)[NB]) {
+      fetch(s + 2 < steps, qa, qb);
+      if (!first) products(checked, 2 * pz, 2 * pc - 2, prev, cur, s & 1);
+      first = pc == ntx;
+      pc = first ? 0 : pc + 1;
+      if (first) pz = pz + 1 == ntz ? 0 : pz + 1;
+      prev = cur;
+      cur = cur == 2 * A_SLOT ? 0 : cur + A_SLOT;
+      if (s + 1 < steps) put(cur, (s + 1) & 1, na, nbq);
+      __syncthreads();
+    };
+    fetch(true, qa0, qb0);
+    fetch(true, qa1, qb1);  // a block has at least one brick, so at least two steps
+    put(0, 0, qa0, qb0);
     __syncthreads();
-  };
-  fetch(true, qa0, qb0);
-  fetch(true, qa1, qb1);  // a block has at least one brick, so at least two steps
-  put(0, 0, qa0, qb0);
-  __syncthreads();
 #pragma unroll 1
-  for (int s = 0; s < steps; s += 2) {
-    step(s, qa0, qb0, qa1, qb1);
-    if (s + 1 < steps) step(s + 1, qa1, qb1, qa0, qb0);
-  }
+    for (int s = 0; s < steps; s += 2) {
+      step(s, qa0, qb0, qa1, qb1);
+      if (s + 1 < steps) step(s + 1, qa1, qb1, qa0, qb0);
+    }
+  };
   // sum of the four wavefronts, 9 taps at a time; lane (i, g) holds
   // D[m = 4 g + j][n = i] of each tap
   const long W = 27L * mc * kc, stride = W + mc;
+  auto partials = [&]() {
+    float any = 0.f;
+    // (opaque, or the 54 addresses of a first call stay in registers for a second)
+    int ch = chunk, mcs = mc;
+    asm volatile("" : "+s"(ch), "+s"(mcs));
 #pragma unroll
-  for (int p = 0; p < 3; p++) {
+    for (int p = 0; p < 3; p++) {
 #pragma unroll
-    for (int tt = 0; tt < 9; tt++)
+      for (int tt = 0; tt < 9; tt++)
 #pragma unroll
-      for (int j = 0; j < 4; j++) red[(tt * 4 + wv) * 256 + lane * 4 + j] = acc[9 * p + tt][j];
-    __syncthreads();
-    const int l = tid >> 2, j = tid & 3;
-    const int m = mb * 16 + 4 * (l >> 4) + j, n = nb * 16 + (l & 15);
+        for (int j = 0; j < 4; j++) red[(tt * 4 + wv) * 256 + lane * 4 + j] = acc[9 * p + tt][j];
+      __syncthreads();
+      const int l = tid >> 2, j = tid & 3;
+      const int m = mb * 16 + 4 * (l >> 4) + j, n = nb * 16 + (l & 15);
 #pragma unroll
-    for (int tt = 0; tt < 9; tt++) {
-      const float s = red[(tt * 4 + 0) * 256 + tid] + red[(tt * 4 + 1) * 256 + tid] + red[(tt * 4 + 2) * 256 + tid] +
-                      red[(tt * 4 + 3) * 256 + tid];
-      part[(long)chunk * stride + ((long)(9 * p + tt) * mc + m) * kc + n] = s;
-      // dw is summed from the partials by atomics after this kernel: the
-      // first chunk's blocks clear it
-      if (chunk == 0) dw[((long)(9 * p + tt) * mc + m) * kc + n] = 0.f;
+      for (int tt = 0; tt < 9; tt++) {
+        const float s = red[(tt * 4 + 0) * 256 + tid] + red[(tt * 4 + 1) * 256 + tid] + red[(tt * 4 + 2) * 256 + tid] +
+                        red[(tt * 4 + 3) * 256 + tid];
+        part[(long)ch * stride + ((long)(9 * p + tt) * mcs + m) * kc + n] = s;
+        any += s;
+        // dw is summed from the partials by atomics after this kernel: the
+        // first chunk's blocks clear it
+        if (ch == 0) dw[((long)(9 * p + tt) * mcs + m) * kc + n] = 0.f;
+      }
+      if (p == 2 && any != any) nan_seen = 1;
+      __syncthreads();
     }
+  };
+  if (tid == 0) nan_seen = 0;
+  walk(std::false_type{});
+  partials();
+  // The zeros of a row outside the volume meet rows inside it: an infinity (or NaN)
+  // there gives NaN in taps that do not touch it. A block with a NaN in its partials
+  // walks its bricks again without those products. (With the checks in every walk
+  // 16x16 channels at 96x128x128 took 39 us instead of 37, 16x48 87 instead of 77.)
+  if (__builtin_amdgcn_readfirstlane(nan_seen)) {
     __syncthreads();
+    walk(std::true_type{});
+    partials();
   }
   if (bias) {
     red[tid] = bsum;  // tid = 64 wv + 16 g + i
