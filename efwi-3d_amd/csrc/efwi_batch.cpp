@@ -46,8 +46,9 @@ int Ctx::batch_group_size(int n, bool grad) const {
   long fit = (long)(kGroupBytes / ((double)G.fs * kStateFields));
   if (grad && fit > 1) {
     size_t free_b = 0, total_b = 0;
+    const double ring_b = (double)B.n * 9 * (cfg.nt - 1) * sizeof(float);
     if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) free_b = 0;
-    fit = std::min(fit, (long)(std::max(batch.ring_cap, free_b / 2) / ring_bytes_of_shot()));
+    fit = std::min(fit, (long)std::max((double)batch.ring.size(), 0.5 * (double)free_b / ring_b));
   }
   if (fit < 2) return 0;
   const int groups = (int)((n + fit - 1) / fit);
@@ -75,8 +76,13 @@ int Ctx::ensure_batch(int n, int nring) {
     if ((rc = alloc((void**)&batch.it_dev, sizeof(int) * 64))) return rc;
     batch.cus = device_cus(cfg.device);
   }
+  const size_t ring_floats = (size_t)B.n * 9 * (size_t)(cfg.nt - 1);
   // rings: one per shot of a group (groups run one after another)
-  if ((rc = grow(this, (void**)&batch.ring, &batch.ring_cap, ring_bytes_of_shot() * std::min(n, nring)))) return rc;
+  while ((int)batch.ring.size() < std::min(n, nring)) {
+    float* ring_k = nullptr;
+    if ((rc = alloc((void**)&ring_k, sizeof(float) * ring_floats))) return rc;
+    batch.ring.push_back(ring_k);
+  }
   const size_t fs = G.fs;
   for (int k = batch.n; k < n; k++) {
     Groups g{};
@@ -106,19 +112,8 @@ int Ctx::ensure_batch(int n, int nring) {
   return EFWI_OK;
 }
 
-// The rings of a batch are kept for the next one up to kRingKeep bytes, else
-// given back when it ends: a program can have what it had before the call. At
-// that size the allocation and its release take 0.6 ms, a batch that fills the
-// rings 50 or more (84^3 cells, 8 shots, 1200 steps: 15.4 GB of rings, 730 ms).
 int Ctx::run_batch(const efwi_shot* shots, int n, int calc_id, const float* const* obs, float* const* syn,
                    double* misfits, int use_graph, hipStream_t s) {
-  const int rc = run_batch_shots(shots, n, calc_id, obs, syn, misfits, use_graph, s);
-  if (batch.ring_cap > kRingKeep) drop(this, (void**)&batch.ring, &batch.ring_cap);
-  return rc;
-}
-
-int Ctx::run_batch_shots(const efwi_shot* shots, int n, int calc_id, const float* const* obs, float* const* syn,
-                         double* misfits, int use_graph, hipStream_t s) {
   if (n < 1 || !shots) return fail(EFWI_ERR_ARG, "a batch needs at least one shot");
   if (calc_id < 0 || calc_id > 2) return fail(EFWI_ERR_ARG, "invalid calc_id " + std::to_string(calc_id));
   if (!model_set) return fail(EFWI_ERR_STATE, "efwi_set_model was not called");
@@ -188,7 +183,7 @@ int Ctx::run_batch_shots(const efwi_shot* shots, int n, int calc_id, const float
     d.nrec = nrec_k;
     d.syn_t = batch.syn_t[k];
     d.res_t = batch.res_t[k];
-    d.ring = calc_id == EFWI_CALC_GRADIENT && gsz0 > 0 ? batch.ring + k % gsz * (ring_bytes_of_shot() / sizeof(float)) : nullptr;
+    d.ring = calc_id == EFWI_CALC_GRADIENT && gsz0 > 0 ? batch.ring[k % gsz] : nullptr;
   }
   // receivers in the velocity kernels where every shot's can be
   bool fold_rec = recv_foldable(Tile{1, 1}, G, true) && (!grad || recv_foldable(Tile{1, 1}, G, false));

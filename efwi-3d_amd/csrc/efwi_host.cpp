@@ -192,19 +192,14 @@ int Ctx::alloc(void** p, size_t bytes) {
   return EFWI_OK;
 }
 
-void drop(Ctx* c, void** p, size_t* cap) {
+int grow(Ctx* c, void** p, size_t* cap, size_t need) {
+  if (*cap >= need) return EFWI_OK;
   if (*p) {
-    c->allocs.erase(std::remove(c->allocs.begin(), c->allocs.end(), *p), c->allocs.end());
+    for (auto& q : c->allocs)
+      if (q == *p) q = nullptr;
     hipFree(*p);
     c->bytes_held -= (long long)*cap;
   }
-  *p = nullptr;
-  *cap = 0;
-}
-
-int grow(Ctx* c, void** p, size_t* cap, size_t need) {
-  if (*cap >= need) return EFWI_OK;
-  drop(c, p, cap);
   int rc = c->alloc(p, need);
   *cap = rc == EFWI_OK ? need : 0;
   return rc;

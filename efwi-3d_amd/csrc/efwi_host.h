@@ -61,9 +61,7 @@ struct RecvMap {
 struct BatchState {
   int n = 0;
   std::vector<Groups> F;
-  std::vector<float*> stf, syn_t, obs_t, res_t;
-  float* ring = nullptr;  // boundary rings of a group's shots, one after another
-  size_t ring_cap = 0;    // bytes
+  std::vector<float*> ring, stf, syn_t, obs_t, res_t;
   std::vector<long*> rec;
   std::vector<RecvMap> recv;
   std::vector<size_t> seis_cap, rec_cap;
@@ -179,13 +177,9 @@ struct Ctx {
   // automatic groups: state bytes of a launch's shots, arrays per shot
   static constexpr double kGroupBytes = 384e6;
   static constexpr int kStateFields = 2 * F_WAVE_COUNT + P_PSI_COUNT + M_COUNT;
-  static constexpr size_t kRingKeep = size_t(4) << 30;  // bytes of rings kept between batches
-  size_t ring_bytes_of_shot() const { return sizeof(float) * 9 * (size_t)B.n * (size_t)(cfg.nt - 1); }
   int batch_group_size(int n, bool grad) const;
   void bind_state(const Groups& g);
   int ensure_batch(int n, int nring);
-  int run_batch_shots(const efwi_shot* shots, int n, int calc_id, const float* const* obs, float* const* syn,
-                      double* misfits, int use_graph, hipStream_t s);
   int run_batch(const efwi_shot* shots, int n, int calc_id, const float* const* obs, float* const* syn,
                 double* misfits, int use_graph, hipStream_t s);
   int batch_gradient(int shot, float* gl, float* gm, float* gr, int on_host, hipStream_t s);
@@ -193,7 +187,6 @@ struct Ctx {
   void release_batch();
 };
 
-void drop(Ctx* c, void** p, size_t* cap);
 int grow(Ctx* c, void** p, size_t* cap, size_t need);
 void wave_of(float* base, size_t fsf, Wave& W);
 void psi_of(float* base, size_t fsf, Psi& P);

@@ -211,8 +211,7 @@ int efwi_batch_config(efwi_ctx* ctx, int take, int static_pct);
  * efwi_run_shot runs it); 0 (default): automatic, groups of as many shots as
  * keep their state within about 1.5 times the Infinity Cache and their rings
  * within half of the free memory, the single-shot kernels where that is one.
- * Rings of more than 4 GiB in all are freed when the call ends. Results do
- * not depend on it. */
+ * Results do not depend on it. */
 int efwi_batch_group(efwi_ctx* ctx, int shots_per_launch);
 /* Gradient (lambda, mu, rho) of shot `shot` of the last efwi_run_batch. */
 int efwi_batch_gradient(efwi_ctx* ctx, int shot, float* g_lambda, float* g_mu, float* g_rho, int on_host,

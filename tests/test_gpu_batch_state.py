@@ -61,30 +61,3 @@ def test_batch_after_a_larger_one(use_graph):
         misfits, syns = P.run_batch(then, 1, o2, want_syn=True)
         grads = [P.batch_gradient(k) for k in range(2)]
         _check(w, then, o2, misfits, syns, grads)
-
-
-def test_rings_given_back():
-    """Boundary rings beyond 4 GiB are freed when the batch ends (four of 2 GB
-    here), smaller ones kept, and later batches are not affected."""
-    w = _workload(700, n=52, npml=10)
-    shots = _shots(w, 8, 6)
-    obs = _obs(w, shots, 7)
-    print(f"[gpu] rings of batches of 8 and 1 on {w.grid.shape}, nt={w.grid.nt}", flush=True)
-    with _open(w) as P:
-        P.batch_group(4)
-        free = torch.cuda.mem_get_info()[0]
-        P.run_batch(shots, 1, obs)
-        taken = free - torch.cuda.mem_get_info()[0]
-        without = P.device_bytes
-        P.batch_group(1)
-        P.run_batch(shots[:1], 1, obs[:1])
-        ring = P.device_bytes - without
-        assert 4 * ring > 4 << 30 and taken < 2 * ring
-        P.run_batch(shots[1:2], 1, obs[1:2])
-        assert P.device_bytes == without + ring  # kept
-        P.batch_group(4)
-        misfits, syns = P.run_batch(shots, 1, obs, want_syn=True)
-        assert P.device_bytes == without
-        pick = (0, 3, 5)
-        _check(w, [shots[k] for k in pick], [obs[k] for k in pick], [misfits[k] for k in pick], [syns[k] for k in pick],
-               [P.batch_gradient(k) for k in pick])
