@@ -39,7 +39,11 @@ void Ctx::release_batch() {
 // 72^3 (84 MB, n = 8): single 55.5, 2: 48.9, 4: 46.2, 8: 52.5; 84^3 (114 MB, n = 8):
 // single 67.2, 2: 60.3, 3: 60.1, 4: 64.8; 84x104x104 (188 MB, n = 6): single
 // 44.0, 2: 42.7, 3: 49.4; 84x140x140 (277 MB, n = 4): single 31.2, 2: 36.1. The
-// boundary rings of a group (one per shot) take at most half of the free memory.
+// boundary rings of a group (one per shot, kept for the next batch) take at most
+// half of the free and a sixteenth of all memory: the single-shot kernels hold one
+// ring, and a program that runs beside them counts on the rest. (Rings freed when
+// a batch ends cost more than they give: the driver clears freed memory at 33 GB/s,
+// 30 ms per GB where a batch that fills it takes 50.)
 int Ctx::batch_group_size(int n, bool grad) const {
   if (batch.group > 0) return std::min(batch.group, n);
   if (batch.group < 0) return 0;
@@ -48,7 +52,8 @@ int Ctx::batch_group_size(int n, bool grad) const {
     size_t free_b = 0, total_b = 0;
     const double ring_b = (double)B.n * 9 * (cfg.nt - 1) * sizeof(float);
     if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) free_b = 0;
-    fit = std::min(fit, (long)std::max((double)batch.ring.size(), 0.5 * (double)free_b / ring_b));
+    const double most = std::min(0.5 * (double)free_b, (double)total_b / 16);
+    fit = std::min(fit, (long)std::max((double)batch.ring.size(), most / ring_b));
   }
   if (fit < 2) return 0;
   const int groups = (int)((n + fit - 1) / fit);

@@ -210,7 +210,8 @@ int efwi_batch_config(efwi_ctx* ctx, int take, int static_pct);
  * through the single-shot kernels (each shot on its own state, as
  * efwi_run_shot runs it); 0 (default): automatic, groups of as many shots as
  * keep their state within about 1.5 times the Infinity Cache and their rings
- * within half of the free memory, the single-shot kernels where that is one.
+ * within half of the free and a sixteenth of all memory, the single-shot
+ * kernels where that is one.
  * Results do not depend on it. */
 int efwi_batch_group(efwi_ctx* ctx, int shots_per_launch);
 /* Gradient (lambda, mu, rho) of shot `shot` of the last efwi_run_batch. */

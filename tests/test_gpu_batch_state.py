@@ -61,3 +61,20 @@ def test_batch_after_a_larger_one(use_graph):
         misfits, syns = P.run_batch(then, 1, o2, want_syn=True)
         grads = [P.batch_gradient(k) for k in range(2)]
         _check(w, then, o2, misfits, syns, grads)
+
+
+def test_rings_of_a_batch_are_bounded():
+    """Shots whose boundary rings are large (11 GB each here) do not each get
+    one in the automatic mode: after a batch the context holds less than one
+    ring more than after a single shot."""
+    w = _workload(4000, n=52, npml=10)
+    shots = _shots(w, 3, 6)
+    obs = _obs(w, shots, 7)
+    print(f"[gpu] rings of a batch of 3 on {w.grid.shape}, nt={w.grid.nt}", flush=True)
+    with _open(w) as P:
+        before = P.device_bytes
+        P.run_shot(shots[0], 1, obs[0])
+        after_shot = P.device_bytes
+        misfits, _ = P.run_batch(shots, 1, obs)
+        assert P.device_bytes - after_shot < after_shot - before
+        assert misfits == [P.run_shot(s, 0, o)[0] for s, o in zip(shots, obs)]
