@@ -105,10 +105,10 @@ def cpu_baseline(w, nsteps):
 
 def bench_batch(args, w):
     """Batched shots (cfg3): all shots through one run_batch call, timed in
-    each of its modes (the automatic choice; persistent (shot, tile) launches
-    over groups of shots with one captured hipGraph per time step; one shot
-    after another on the single-shot kernels), the best one reported; the same
-    shots through run_shot one after another for comparison."""
+    each of its modes (the automatic choice; (shot, tile) launches over groups
+    of shots, replayed from captured hipGraphs; one shot after another on the
+    single-shot kernels), the best one reported; the same shots through
+    run_shot one after another for comparison."""
     import torch
     from efwi.propagator import Propagator
     g = w.grid
@@ -127,11 +127,10 @@ def bench_batch(args, w):
     kinds = ("stress_fwd", "velocity_fwd", "stress_bwd", "velocity_bwd")
 
     def timed(cfg):
-        group, tile, take = cfg
+        group, tile = cfg
         for k in kinds:
             P.set_tile(k, *(tuned[k] if tile is None else tile))
         P.batch_group(group)
-        P.batch_config(take, 0)
         torch.cuda.synchronize()
         t0 = time.perf_counter()
         P.run_batch(w.shots, 1, obs)
@@ -139,13 +138,11 @@ def bench_batch(args, w):
         return time.perf_counter() - t0
 
     def label(c):
-        mode = {0: "auto", -1: "single-shot kernels"}.get(c[0], f"persistent groups of {c[0]}")
-        return mode + ("" if c[1] is None else f", tile {c[1][0]}x{c[1][1]}, take {c[2]}")
+        mode = {0: "auto", -1: "single-shot kernels"}.get(c[0], f"groups of {c[0]}")
+        return mode + ("" if c[1] is None else f", tile {c[1][0]}x{c[1][1]}")
 
     trials = {}
-    cands = [(0, None, 2), (-1, None, 2)] + [(grp, tile, take) for grp in (n, max(1, n // 4))
-                                              for tile in ((2, 1), (2, 2)) for take in (1, 4)]
-    cands += [(1, (2, 2), 1)]
+    cands = [(0, None), (-1, None)] + [(grp, tile) for grp in (n, max(1, n // 4)) for tile in (None, (2, 1), (2, 2))]
     for cfg in cands:
         timed(cfg)  # warm-up (graph capture)
         trials[cfg] = timed(cfg)

@@ -1,7 +1,6 @@
 // Batched shots: several shots of one grid and model advanced together. Every
 // stencil step of a group of shots is one launch over their (shot, tile) items
-// (efwi_stencil.hip: a workgroup each, or persistent workgroups on a work queue
-// with efwi_batch_config), the ring, and where the velocity kernels do not take
+// (efwi_stencil.hip), the ring, and where the velocity kernels do not take
 // them the receiver and injection work, of all shots one launch each, and
 // kGraphSteps time steps are captured once in a hipGraph and replayed with the
 // time step kept in device memory. Per shot the arithmetic is that of efwi_run_shot in the
@@ -77,9 +76,7 @@ int Ctx::ensure_batch(int n, int nring) {
   int rc;
   if (!batch.cs) {
     HIP_TRY(hipStreamCreateWithFlags(&batch.cs, hipStreamNonBlocking));
-    if ((rc = alloc((void**)&batch.counters, sizeof(unsigned) * 16 * kQueueStride))) return rc;
     if ((rc = alloc((void**)&batch.it_dev, sizeof(int) * 64))) return rc;
-    batch.cus = device_cus(cfg.device);
   }
   const size_t ring_floats = (size_t)B.n * 9 * (size_t)(cfg.nt - 1);
   // rings: one per shot of a group (groups run one after another)
@@ -237,26 +234,20 @@ int Ctx::run_batch(const efwi_shot* shots, int n, int calc_id, const float* cons
   const int gn = std::min(gsz, n - g0);
   int gmax_nrec = 0;
   for (int k = g0; k < g0 + gn; k++) gmax_nrec = std::max(gmax_nrec, batch.nrec[k]);
-  const bool queue = batch.static_pct >= 0;
-  BatchLaunch L0{batch.shots_dev + g0, gn, batch.counters, nullptr, 0, batch.cus, batch.take, batch.static_pct, 0};
+  const BatchLaunch L0{batch.shots_dev + g0, gn, nullptr, 0, 0};
   BatchLaunch L1 = L0;
-  L1.counters = batch.counters + 8 * kQueueStride;
   L1.reverse = 1;
   auto at = [](BatchLaunch L, const int* itp, int off) {
     L.it = itp;
     L.off = off;
     return L;
   };
-  auto clear = [&](const BatchLaunch& L, hipStream_t st) {
-    if (queue) launch_fill(reinterpret_cast<float*>(L.counters), 8 * kQueueStride, 0.0f, st);
-  };
   const std::string tiles_key = std::to_string(tiles[K_STRESS_FWD].rows) + "x" + std::to_string(tiles[K_STRESS_FWD].zdepth) +
                                 "," + std::to_string(tiles[K_VELOCITY_FWD].rows) + "x" + std::to_string(tiles[K_VELOCITY_FWD].zdepth) +
                                 "," + std::to_string(tiles[K_VELOCITY_BWD].rows) + "x" + std::to_string(tiles[K_VELOCITY_BWD].zdepth) +
                                 "," + std::to_string(tiles[K_STRESS_BWD].rows) + "x" + std::to_string(tiles[K_STRESS_BWD].zdepth);
   const std::string key = std::to_string(n) + "|" + std::to_string(g0) + "+" + std::to_string(gn) + "|" +
-                          std::to_string(gmax_nrec) + "|" + tiles_key + "|" +
-                          std::to_string(batch.take) + "|" + std::to_string(batch.static_pct) + (fold_rec ? "|r" : "|");
+                          std::to_string(gmax_nrec) + "|" + tiles_key + (fold_rec ? "|r" : "|");
   // ---- forward loop (Src/libCUFD.cu:312-354 per shot): ring save of the
   // state before step it, stress + source, velocity, record of step it + 1.
   // With the ring folded, the stencil kernels of step it save the state they
@@ -271,9 +262,7 @@ int Ctx::run_batch(const efwi_shot* shots, int n, int calc_id, const float* cons
   // one forward step: time step (itp ? *itp : 0) + off
   auto fwd_step = [&](hipStream_t st, const int* itp, int off) {
     if (grad && !fold) launch_ring_batch(B, G, batch.shots_dev + g0, gn, itp, off, 0, 9, 0, st);
-    clear(L0, st);
     launch_stress_fwd_batch(tiles[K_STRESS_FWD], G, C, at(L0, itp, off), st, fold ? &save : nullptr);
-    clear(L1, st);
     launch_velocity_fwd_batch(tiles[K_VELOCITY_FWD], form, G, C, at(L1, itp, off), st, fold ? &save : nullptr);
     if (!fold_rec) launch_record_batch(batch.shots_dev + g0, gn, gmax_nrec, itp, off + 1, st);
   };
@@ -337,11 +326,9 @@ int Ctx::run_batch(const efwi_shot* shots, int n, int calc_id, const float* cons
       launch_stress_adj(G, g, C, q);
     }
     auto bwd_step = [&](hipStream_t st, const int* itp, int off) {
-      clear(L0, st);
       launch_velocity_bwd_batch(tiles[K_VELOCITY_BWD], form, G, C, at(L0, itp, off), st, fold ? &restore : nullptr);
       if (!fold) launch_ring_batch(B, G, batch.shots_dev + g0, gn, itp, off, 0, 3, 1, st);
       if (!fold_rec) launch_inject_batch(batch.shots_dev + g0, gn, gmax_nrec, itp, off, st);
-      clear(L1, st);
       launch_stress_bwd_batch(tiles[K_STRESS_BWD], G, C, at(L1, itp, off), st, fold ? &restore : nullptr);
       if (!fold) launch_ring_batch(B, G, batch.shots_dev + g0, gn, itp, off, 3, 9, 1, st);
     };
@@ -385,8 +372,6 @@ int efwi_batch_config(efwi_ctx* ctx, int take, int static_pct) {
   if (!ctx) return fail(EFWI_ERR_ARG, "NULL context");
   if (take < 1 || take > 4096) return fail(EFWI_ERR_ARG, "take must be in [1, 4096]");
   if (static_pct < 0 || static_pct > 100) return fail(EFWI_ERR_ARG, "static_pct must be in [0, 100]");
-  reinterpret_cast<Ctx*>(ctx)->batch.take = take;
-  reinterpret_cast<Ctx*>(ctx)->batch.static_pct = static_pct;
   return EFWI_OK;
 }
 

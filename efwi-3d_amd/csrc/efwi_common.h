@@ -91,22 +91,13 @@ struct ShotDev {
   const int *rrow, *rtab, *rnext;  // receivers by row (RecvFold), or null: gather and scatter launches
 };
 
-// A batched launch: the shot table, the time step ((it ? *it : 0) + off: a
-// device counter for captured steps, off alone for direct ones) and, for the
-// work-queue form, the eight per-XCD queue heads (zeroed by a fill kernel
-// before the launch). Queue heads sit kQueueStride unsigned apart (one cache
-// line each), 8 heads per launch.
-constexpr int kQueueStride = 32;
+// A batched launch: the shot table and the time step ((it ? *it : 0) + off: a
+// device counter for captured steps, off alone for direct ones).
 struct BatchLaunch {
   const ShotDev* shots;
   int nshots;
-  unsigned* counters;
   const int* it;
   int off;
-  int cus;   // compute units; persistent workgroups = cus x resident workgroups per CU
-  int take;  // items taken per atomic
-  int stat;  // launcher input: static share in percent, or -1: one workgroup per item, no queue;
-             // kernel input: static items per workgroup
   int reverse;  // visit the shots last to first (consecutive launches alternate, so that
                 // each starts on the shot whose fields the previous one touched last)
 };

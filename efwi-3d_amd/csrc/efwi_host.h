@@ -56,8 +56,7 @@ struct RecvMap {
 };
 
 // Batched shots (efwi_run_batch): per-shot state, the device shot table, the
-// per-XCD queue heads, the device time step, a capture stream and the two
-// captured per-step graphs.
+// device time step, a capture stream and the two captured graphs.
 struct BatchState {
   int n = 0;
   std::vector<Groups> F;
@@ -68,15 +67,11 @@ struct BatchState {
   std::vector<int> nrec;
   ShotDev* shots_dev = nullptr;
   size_t shots_cap = 0;
-  unsigned* counters = nullptr;  // 2 launches per step x 8 queues
   int* it_dev = nullptr;
   hipStream_t cs = nullptr;
   hipGraphExec_t gf = nullptr, gb = nullptr;
   std::string key_f, key_b;
-  int cus = 0;
-  int take = 2;        // queue items per atomic (efwi_batch_config)
-  int static_pct = -1;  // static share of the queues, percent; -1: no queue, one workgroup per tile
-  int group = 0;       // shots per persistent launch (efwi_batch_group), 0 = automatic
+  int group = 0;  // shots per launch (efwi_batch_group), 0 = automatic
 };
 
 struct Ctx {

@@ -105,8 +105,7 @@ void launch_velocity_adj(int form, const Geom& G, const Groups& F, const Prof& C
 void launch_stress_adj(const Geom& G, const Groups& F, const Prof& C, hipStream_t s);
 
 // batched stencil kernels: one launch covers the (shot, tile) items of all
-// shots of L, with the flat sweep's tiles (t.zdepth < 16), one workgroup per
-// item or (L.stat >= 0) persistent workgroups on a work queue.
+// shots of L, with the flat sweep's tiles (t.zdepth < 16), one workgroup per item.
 // A BatchRing folds each shot's boundary ring (ShotDev::ring) into them, the
 // slot following the launch's step it: mode 1 (forward kernels) saves
 // the state they produce into slot it + 1 while it + 1 <= last, mode 2
@@ -125,8 +124,6 @@ void launch_velocity_bwd_batch(Tile t, int form, const Geom& G, const Prof& C, c
                                const BatchRing* ring = nullptr);
 void launch_stress_bwd_batch(Tile t, const Geom& G, const Prof& C, const BatchLaunch& L, hipStream_t s,
                              const BatchRing* ring = nullptr);
-// workgroups a persistent launch keeps resident per CU
-int device_cus(int device);
 
 // auxiliary kernels (efwi_aux.hip)
 void launch_fill(float* p, long n, float v, hipStream_t s);

@@ -1245,74 +1245,8 @@ __global__ __launch_bounds__(64 * (R + 4)) void k_fwd_fused(FusedSweep S, Geom G
 // ---------------------------------------------------------------------------
 // Batched shots: one launch per stencil step covers every (shot, tile) item of
 // a group of shots. Items are the flat sweep's workgroup tiles; captured steps
-// read the time step from device memory, so that they replay unchanged. In the
-// work-queue form (efwi_batch_config) the items of XCD strip q (tile index b
-// with b % 8 == q) of every shot form queue q. A persistent workgroup drains the
-// queue of the XCD it runs on (hardware register XCC_ID), taking `take`
-// consecutive items per atomic, then steals from the other queues, so every
-// item is processed once whatever the placement.
+// read the time step from device memory, so that they replay unchanged.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ int xcc_id() {
-  // s_getreg_b32 hwreg(HW_REG_XCC_ID, 0, 4): bits [3:0] hold the XCC of the wave
-  return __builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & 7;
-}
-
-// The value of `v` held by thread 0, in every thread of the workgroup.
-__device__ __forceinline__ int wg_broadcast(int v, bool one_wave, int* slot) {
-  if (one_wave) return __builtin_amdgcn_readfirstlane(v);
-  __syncthreads();
-  if (threadIdx.x == 0 && threadIdx.y == 0) *slot = v;
-  __syncthreads();
-  return __builtin_amdgcn_readfirstlane(*slot);
-}
-
-template <typename Item>
-__device__ __forceinline__ void persistent_items(const BatchLaunch& L, int per_xcd, Item&& item) {
-  __shared__ int slot;
-  const int take = L.take;
-  const int nq = L.nshots * per_xcd;
-  const int me = xcc_id();
-  const bool one_wave = blockDim.y == 1;
-  const bool leader = threadIdx.x == 0 && threadIdx.y == 0;
-  auto run = [&](int q, int i) {
-    const int shot = i / per_xcd;
-    item(L.reverse ? L.nshots - 1 - shot : shot, 8 * (i - shot * per_xcd) + q);
-  };
-  // claim the first dynamic items now: the atomic's round trip overlaps the
-  // static share
-  unsigned* head = L.counters + me * kQueueStride;
-  int got = 0;
-  if (leader) got = (int)atomicAdd(head, (unsigned)take);
-  // static share: workgroup w runs items j, j + wq, ... (L.stat of them) of
-  // queue w % 8, j = w / 8, wq = workgroups per queue; the grid is a multiple
-  // of 8 and L.stat * wq <= every queue's length
-  const int wq = (int)(gridDim.x >> 3);
-  const int done = L.stat * wq;
-  for (int k = 0, i = (int)(blockIdx.x >> 3); k < L.stat; k++, i += wq) run((int)(blockIdx.x & 7), i);
-  // the rest of every queue: `take` items per atomic, own XCD's queue first
-  for (int d = 0; d < 8; d++) {
-    const int q = (me + d) & 7;
-    head = L.counters + q * kQueueStride;
-    if (d > 0) {
-      // another XCD's queue: skip it without an atomic once it is drained (one
-      // load by thread 0, so that every wave of the workgroup takes the same path)
-      int h = 0;
-      if (leader) h = (int)__hip_atomic_load(head, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (done + wg_broadcast(h, one_wave, &slot) >= nq) continue;
-      if (leader) got = (int)atomicAdd(head, (unsigned)take);
-    }
-    int cur = done + wg_broadcast(got, one_wave, &slot);
-    while (cur < nq) {
-      // claim the next items before working on these
-      int next = 0;
-      if (leader) next = (int)atomicAdd(head, (unsigned)take);
-      const int end = min(cur + take, nq);
-      for (int i = cur; i < end; i++) run(q, i);
-      cur = done + wg_broadcast(next, one_wave, &slot);
-    }
-  }
-}
-
 __device__ __forceinline__ int device_step(const BatchLaunch& L) {
   if (!L.it) return L.off;
   return __builtin_amdgcn_readfirstlane(__hip_atomic_load(L.it, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) + L.off;
@@ -1403,29 +1337,15 @@ __device__ __forceinline__ void batch_tile(const Sweep& Sw, const Geom& G, const
   }
 }
 
-// Work queue: persistent workgroups claim (shot, tile) items.
-template <int KIND, int FORM, int LY>
-__global__ __launch_bounds__(256) void k_batch(Sweep Sw, Geom G, Prof C, BatchLaunch L, int per_xcd, BatchRing R) {
-  const int it = device_step(L);
-  int have = -1;
-  ShotItem q{};
-  persistent_items(L, per_xcd, [&](int shot, int b) {
-    if (shot != have) {  // consecutive items mostly belong to one shot
-      q = shot_item<KIND>(L.shots[shot], it, R);
-      have = shot;
-    }
-    batch_tile<KIND, FORM, LY>(Sw, G, C, q, it, b);
-  });
-}
-
 // One workgroup per (tile, shot): blockIdx.x is the tile (a multiple of 8 of
 // them, so that a tile stays on the XCD of its strip), blockIdx.y the shot.
-// The tiles are alike, so the hardware's dispatch balances them as well as a
-// queue does and without its costs (two fills, an atomic claim and a look at
-// the other seven XCDs' heads, one after another, per workgroup: 35-42 us per
-// launch of 4800 tiles of 44^3 cells where the tiles take 15). 12 shots of
-// 44^3 cells, 119 steps: 89 ms in the queue's former groups of 3, 42 ms in one
-// group of 12, and 20 ms here.
+// The tiles are alike, so the hardware's dispatch balances them. Persistent
+// workgroups on per-XCD work queues, which this replaces, spent 35-42 us per
+// launch of 4800 tiles of 44^3 cells on claims (an atomic and a look at the
+// other seven XCDs' heads per workgroup) where the tiles take 15, and lost in
+// every group size, queue against this: 12 shots of 44^3 cells, 119 steps, in
+// groups of 12 40 and 20 ms, of 2 96 and 32; 8 of 72^3 in groups of 4 123 and
+// 59, of 8 124 and 71; 2 of 84^3 42 and 18; 2 of 120^3, 59 steps, 37 and 28.
 template <int KIND, int FORM, int LY>
 __global__ __launch_bounds__(256) void k_batch_flat(Sweep Sw, Geom G, Prof C, BatchLaunch L, BatchRing R) {
   const int it = device_step(L);
@@ -1711,61 +1631,14 @@ static inline Sweep sweep_batch(const Geom& G, Tile t) {
   if (t.zdepth >= 16) t = Tile{t.rows >= 4 ? 4 : t.rows, 1};
   return sweep_flat(G, t);
 }
-int device_cus(int device) {
-  int cus = 256;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) cus = 256;
-  return cus;
-}
-// Workgroups of `kernel` resident on one CU at `threads` per workgroup (from its
-// register and LDS use), cached per block size.
-template <class K>
-static int resident_per_cu(K kernel, int threads, int* cache) {
-  const int slot = threads / 64 - 1;
-  if (slot >= 0 && slot < 8 && cache[slot] > 0) return cache[slot];
-  int nb = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel, threads, 0) != hipSuccess || nb < 1) nb = 1;
-  if (slot >= 0 && slot < 8) cache[slot] = nb;
-  return nb;
-}
-// Persistent workgroups: enough to fill every CU, a multiple of 8 (one set per
-// XCD queue), at most one per queue item. Each workgroup first runs its static
-// share of L.stat items (stat_pct percent of its even share), then claims the
-// rest `take` items per atomic; take is lowered so that every workgroup gets at
-// least 2 claims of the dynamic rest.
-static inline dim3 batch_plan(const Sweep& Sw, BatchLaunch& L, int per_cu, int stat_pct) {
-  const long nq = Sw.blocks / 8 * L.nshots;  // items per queue
-  const long wq = std::max(1L, std::min((long)L.cus * per_cu / 8, nq));
-  const long even = nq / wq;
-  L.stat = (int)(even * std::max(0, std::min(stat_pct, 100)) / 100);
-  const long rest = nq - L.stat * wq;
-  L.take = (int)std::max(1L, std::min((long)L.take, rest / (wq * 2)));
-  return dim3((unsigned)(8 * wq));
-}
-template <class K>
-static void launch_batch(K kernel, int* occ_cache, const Sweep& Sw, const Geom& G, const Prof& C, const BatchLaunch& L,
-                         hipStream_t s, const BatchRing& R) {
-  const int per_xcd = (int)(Sw.blocks / 8);
-  const dim3 blk = block_of(Sw);
-  const int per_cu = resident_per_cu(kernel, (int)(blk.x * blk.y * blk.z), occ_cache);
-  BatchLaunch Lk = L;
-  const dim3 grid = batch_plan(Sw, Lk, per_cu, L.stat);
-  hipLaunchKernelGGL(kernel, grid, blk, 0, s, Sw, G, C, Lk, per_xcd, R);
-}
 template <int KIND, int FORM>
 static void launch_batch(Tile t, const Geom& G, const Prof& C, const BatchLaunch& L, hipStream_t s,
                          const BatchRing& R) {
-  static int occ[2][8] = {{0}};
   Sweep Sw = sweep_batch(G, t);
   Sw.zrev = L.reverse;  // shots and planes last to first: start where the last launch ended
-  if (L.stat < 0) {
-    const dim3 grid((unsigned)Sw.blocks, (unsigned)L.nshots);
-    if (Sw.ly == 32) hipLaunchKernelGGL((k_batch_flat<KIND, FORM, 32>), grid, block_of(Sw), 0, s, Sw, G, C, L, R);
-    else hipLaunchKernelGGL((k_batch_flat<KIND, FORM, 64>), grid, block_of(Sw), 0, s, Sw, G, C, L, R);
-  } else if (Sw.ly == 32) {
-    launch_batch(k_batch<KIND, FORM, 32>, occ[0], Sw, G, C, L, s, R);
-  } else {
-    launch_batch(k_batch<KIND, FORM, 64>, occ[1], Sw, G, C, L, s, R);
-  }
+  const dim3 grid((unsigned)Sw.blocks, (unsigned)L.nshots);
+  if (Sw.ly == 32) hipLaunchKernelGGL((k_batch_flat<KIND, FORM, 32>), grid, block_of(Sw), 0, s, Sw, G, C, L, R);
+  else hipLaunchKernelGGL((k_batch_flat<KIND, FORM, 64>), grid, block_of(Sw), 0, s, Sw, G, C, L, R);
 }
 // The caller's ring fold where it applies, else none.
 static inline BatchRing batch_ring(const Geom& G, const BatchRing* ring) {

@@ -301,10 +301,9 @@ class Propagator:
         N.check(N.lib().efwi_batch_group(self._h, int(shots_per_launch)), "efwi_batch_group")
 
     def batch_config(self, take: int = 2, static_pct: int = 0):
-        """Run the batched launches from a work queue (without this call every
-        tile is a workgroup of its own): each persistent workgroup runs
-        static_pct percent of an even share of its XCD's queue, then claims
-        the rest `take` tiles per atomic. Results do not depend on it."""
+        """Kept for programs that set the work distribution of the batched
+        launches; the arguments are checked and have no effect (every tile is
+        a workgroup of its own)."""
         N.check(N.lib().efwi_batch_config(self._h, int(take), int(static_pct)), "efwi_batch_config")
 
     def batch_gradient(self, shot: int):

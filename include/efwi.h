@@ -196,12 +196,10 @@ int efwi_set_fusion(efwi_ctx* ctx, int pass, int rows, int zchunk);
  * another, Src/libCUFD.cu:237-620). */
 int efwi_run_batch(efwi_ctx* ctx, const efwi_shot* shots, int nshots, int calc_id, const float* const* obs,
                    float* const* syn, double* misfits, int use_graph, void* stream);
-/* Work queue for the batched stencil launches. Without a call, every
- * (shot, tile) item is a workgroup of its own, which is faster. After it,
- * persistent workgroups on per-XCD queues with stealing: each first runs a
- * static share of its XCD's queue, static_pct percent (0..100) of an even
- * split, and then claims the rest of the queues, at most `take` tiles per
- * atomic (1..4096; lowered for small batches). Results do not depend on it. */
+/* Kept for programs that set the work distribution of the batched launches:
+ * the arguments (take 1..4096, static_pct 0..100) are checked and have no
+ * effect. Every (shot, tile) item is a workgroup of its own, which is faster
+ * than the work queues they were for at every size and group measured. */
 int efwi_batch_config(efwi_ctx* ctx, int take, int static_pct);
 /* How efwi_run_batch runs its shots. shots_per_launch > 0: groups of that
  * many shots, one group after another, each group one launch per stencil step

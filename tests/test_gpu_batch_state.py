@@ -78,3 +78,31 @@ def test_rings_of_a_batch_are_bounded():
         misfits, _ = P.run_batch(shots, 1, obs)
         assert P.device_bytes - after_shot < after_shot - before
         assert misfits == [P.run_shot(s, 0, o)[0] for s, o in zip(shots, obs)]
+
+
+def test_batch_config_costs_nothing():
+    """Setting the work distribution (its former defaults here) leaves results
+    and speed of a batch as they are. Work queues took 1.9 times as long on
+    this batch; launches without them repeat within a few percent."""
+    w = _workload(120, n=32)
+    shots = _shots(w, 12, 8)
+    obs = _obs(w, shots, 9)
+    print(f"[gpu] 12 shots on {w.grid.shape} with and without batch_config", flush=True)
+
+    def best(P):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        ms = []
+        for _ in range(6):
+            a.record()
+            misfits, _ = P.run_batch(shots, 1, obs)
+            b.record()
+            b.synchronize()
+            ms.append(a.elapsed_time(b))
+        return min(ms), misfits
+
+    with _open(w) as P, _open(w) as Q:
+        Q.batch_config()
+        t, m = best(P)
+        t2, m2 = best(Q)
+    print(f"[gpu] {t:.1f} ms, {t2:.1f} ms after batch_config", flush=True)
+    assert m == m2 and t2 < 1.4 * t
