@@ -1574,16 +1574,21 @@ int efwi_nn_conv3_cat(const uint16_t* src, int lds, int kc1, int up1, const uint
   // voxels: 32->32 27.7 -> 22.5 us, 96->32 82 -> 75 us)
   int NB = nbt % 4 == 0 ? 4 : nbt % 3 == 0 ? 3 : nbt % 2 == 0 ? 2 : 1;
   if (bricks * (nbt / NB) < 4L * device_cus()) NB = 1;
-  // (in mode 0, rows of 32 voxels or more come here with unaligned outputs and in small volumes: one block)
-  if (MB >= 2 && mode == 0) NB = 1;
+  // Rows of 32 voxels or more in mode 0 come here with unaligned outputs. Several
+  // blocks then pay only where the halo is one chunk or they
+  // are three (unaligned, one block against them: 16->48 at 96x128x128 165 and 136 us,
+  // 16->32 106 and 93, 48->48 384 and 326; but 32->64 at 60x100x100 138 and 177), four
+  // only in rows below 64 voxels (16->64 at 60x100x100 94 us with two, 117 with four;
+  // at 96x128x50 118 and 105).
+  if (MB >= 2 && mode == 0 && NB != 3) NB = kc > 16 ? 1 : MB == 4 ? std::min(NB, 2) : NB;
   const int per_xcd = (int)((bricks + 7) / 8);
   const dim3 grid((unsigned)(8L * per_xcd), (unsigned)(nbt / NB));
 #define EFWI_NN_CONV_LAUNCH(CK, M, B, MODE)                                                                       \
   hipLaunchKernelGGL((k_conv3<CK, M, B, MODE>), grid, dim3(128 * conv_tz(M)), 0, s, src, lds, kc, w, bias, dst,  \
                      ldd, nc, mask, ldm, V, relu, ntz, ntx, nty, per_xcd, vec_out, src2, lds2, kc1, dst2, ldd2,   \
                      nc1, up1 ? 1 : 0)
-#define EFWI_NN_CONV_MODE(CK, M, B)                                      \
-  if (mode == 0) { EFWI_NN_CONV_LAUNCH(CK, M, (M >= 2 ? 1 : B), 0); }  \
+#define EFWI_NN_CONV_MODE(CK, M, B)                                              \
+  if (mode == 0) { EFWI_NN_CONV_LAUNCH(CK, M, (M == 4 && B == 4 ? 2 : B), 0); }  \
   else { EFWI_NN_CONV_LAUNCH(CK, M, B, 1); }
 #define EFWI_NN_CONV_NB(CK, M)                              \
   if (NB == 4) { EFWI_NN_CONV_MODE(CK, M, 4) }             \
