@@ -1385,21 +1385,49 @@ static Sweep make_sweep(int z0, int z1, int x0, int x1, int y0, int y1, Tile t, 
 static inline Sweep sweep_full(const Geom& G, Tile t, int ly) {
   return make_sweep(2, G.nz - 3, 2, G.nx - 3, 2, G.ny - 3, t, ly);
 }
+// Wavefronts per plane and y segment of two-row launches on the XCD with most of
+// them. In the backward kernels a pair whose rows lie on two sides of the C-PML's
+// edge runs both variants and counts twice.
+static int pairs_of_strip(const Geom& G, const Sweep& S, bool bwd) {
+  int most = 0;
+  for (int k = 0, x = S.x0; k < 8; k++) {
+    const int rows = S.rows_base + (k < S.rows_rem ? 1 : 0);
+    int n = (rows + 1) / 2;
+    if (bwd)
+      for (int edge : {G.npml, G.nx - G.npml})  // first row of the interior, of the upper slab
+        if (edge > x && edge < x + rows && (edge - x) % 2) n++;
+    most = std::max(most, n);
+    x += rows;
+  }
+  return most;
+}
 // The flat sweep of a launch. A wavefront covers 64 y cells of one row, or 32
-// of two rows: the latter where it leaves at most 7/8 as many lanes per row
-// (fewer lanes past the row's end, and y C-PML terms in fewer wavefronts) and
+// of two rows: the latter where the XCD with most work has at most 7/8 as many
+// wavefronts then (fewer lanes past the row's end, and y C-PML terms in fewer
+// wavefronts, against half-filled pairs of strips of an odd number of rows) and
 // the rows keep the device busy (at least 16 wavefronts per CU; on smaller
-// grids one wavefront's latency is what counts, and a wavefront with rows of
-// two kinds runs both variants). stress_fwd / velocity_fwd / velocity_bwd /
-// stress_bwd in us, 64 against 32 lanes: 84^3 cells (80 cells per row: 128 and
-// 96 lanes) 15.7 / 14.3 / 30.8 / 28.4 against 13.9 / 12.5 / 26.1 / 23.0;
-// 110x212x212 (256 and 224 lanes) 114 / 83 / 216 / 220 against 105 / 77 / 201 /
-// 183; 160x240x240 (256 lanes either way) 209 / 168 / 368 / 368 against 226 /
-// 185 / 396 / 345.
-static inline Sweep sweep_flat(const Geom& G, Tile t) {
+// grids one wavefront's latency is what counts). The two-row backward kernels
+// run 3 wavefronts per SIMD instead of 4, so where an XCD runs its strip in one
+// or two rounds of resident wavefronts, not where they need one more.
+// stress_fwd / velocity_fwd / velocity_bwd / stress_bwd in us, 64 against 32 lanes:
+// 84^3 cells (C-PML 10; 10 rows of 2 segments per strip, 5 pairs of 3: 15/20)
+// 18.5 / 17.6 / 34.7 / 32.6 against 17.0 / 15.8 / 29.8 / 26.9; 110x212x212 (20;
+// 7/8) 123 / 102 / 203 / 202 against 112 / 93 / 187 / 164; 60x60x84 (10; 7 rows, 4
+// pairs and a C-PML edge: 15/14) 12.9 / 12.2 / 21.7 / 20.1 against 12.5 / 11.9 /
+// 26.0 / 22.1; 60x60x148 (25/21) 15.7 / 15.0 / 27.0 / 24.9 against 15.5 / 14.7 /
+// 34.1 / 29.4; 73x55x77 (15; 6/7 but three rounds instead of two) both backward
+// ones 1.14 times as long in two rows; 160x240x240 (as many segments either way)
+// 209 / 168 / 368 / 368 against 226 / 185 / 396 / 345. Over 44 random grids of 34 to
+// 192 cells per axis the backward kernels of the ones taken take 0.79-0.96 times as
+// long in two rows, of the others 0.94-1.14.
+static inline Sweep sweep_flat(const Geom& G, Tile t, bool bwd, int shots = 1) {
   const Sweep a = sweep_full(G, t, 64), b = sweep_full(G, t, 32);
-  const long waves = (long)(G.nz - 4) * (G.nx - 4) * a.nyb;
-  return 8 * 32 * b.nyb <= 7 * 64 * a.nyb && waves >= 16 * 256 ? b : a;
+  if ((long)(G.nz - 4) * (G.nx - 4) * a.nyb < 16 * 256) return a;
+  const long wa = (long)(a.rows_base + (a.rows_rem ? 1 : 0)) * a.nyb, wb = (long)pairs_of_strip(G, b, bwd) * b.nyb;
+  if (8 * wb > 7 * wa) return a;
+  const long planes = (long)(G.nz - 4) * shots, simds = 4 * 32;  // SIMDs of an XCD
+  const long ra = (wa * planes + 4 * simds - 1) / (4 * simds), rb = (wb * planes + 3 * simds - 1) / (3 * simds);
+  return bwd && ra < 3 && rb > ra ? a : b;
 }
 
 static inline dim3 grid_of(const Sweep& S) { return dim3((unsigned)S.blocks); }
@@ -1454,7 +1482,7 @@ bool launch_stress_fwd(Tile t, const Geom& G, const Groups& F, const Prof& C, co
     EFWI_MARCH(k_stress_fwd_m, 0, Sw, G, F, C, S, it);
     return false;
   }
-  const Sweep Sw = sweep_flat(G, t);
+  const Sweep Sw = sweep_flat(G, t, false);
   const RingFold Rf = fold_for(G, ring);
   EFWI_FLAT(Sw, k_stress_fwd<, Sw, G, F, C, S, it, Rf);
   return Rf.slot != nullptr;
@@ -1465,7 +1493,7 @@ bool launch_stress_fwd(Tile t, const Geom& G, const Groups& F, const Prof& C, co
 // cells velocity 367 -> 351 us, stress 368 -> 359; 200x360x360 876 -> 860 and
 // 917 -> 917; below, and for the two-row wavefronts, one plane is as fast or faster.
 Tile default_bwd_tile(const Geom& G) {
-  const Sweep S = sweep_flat(G, Tile{1, 1});
+  const Sweep S = sweep_flat(G, Tile{1, 1}, true);
   return S.ly == 64 && (long)(G.nz - 4) * (G.nx - 4) * S.nyb >= 256L * 256 ? Tile{1, 2} : Tile{1, 1};
 }
 // Receivers are folded up to 256 (forward) and 128 (backward) wavefronts per
@@ -1494,7 +1522,7 @@ bool launch_velocity_fwd(Tile t, int form, const Geom& G, const Groups& F, const
     }
     return false;
   }
-  Sweep Sw = sweep_flat(G, t);
+  Sweep Sw = sweep_flat(G, t, false);
   Sw.zrev = 1;  // the stress kernel before it ran first to last
   const RingFold Rf = fold_for(G, ring);
   const RecvFold V = recv_for(recv);
@@ -1558,7 +1586,7 @@ bool launch_velocity_bwd(Tile t, int form, const Geom& G, const Groups& F, const
     }
     return Rf.slot != nullptr;
   }
-  const Sweep Sw = sweep_flat(G, t);
+  const Sweep Sw = sweep_flat(G, t, true);
   if (V.row) {
     if (form == 1) EFWI_FLAT(Sw, k_velocity_bwd<1 EFWI_COMMA true EFWI_COMMA true EFWI_COMMA, Sw, G, F, C, Rf, V);
     else EFWI_FLAT(Sw, k_velocity_bwd<0 EFWI_COMMA true EFWI_COMMA true EFWI_COMMA, Sw, G, F, C, Rf, V);
@@ -1583,7 +1611,7 @@ bool launch_stress_bwd(Tile t, const Geom& G, const Groups& F, const Prof& C, co
     hipLaunchKernelGGL((k_stress_bwd<true, 64>), grid_of(rim), block_of(rim), 0, s, rim, G, F, C, S, it, Rf);
     return Rf.slot != nullptr;
   }
-  Sweep Sw = sweep_flat(G, t);
+  Sweep Sw = sweep_flat(G, t, true);
   Sw.zrev = 1;  // the velocity kernel before it ran first to last
   EFWI_FLAT(Sw, k_stress_bwd<true EFWI_COMMA, Sw, G, F, C, S, it, Rf);
   return Rf.slot != nullptr;
@@ -1612,13 +1640,13 @@ bool launch_fwd_fused(int R, int zc, int form, const Geom& G, const Groups& Fi, 
 }
 
 void launch_velocity_adj(int form, const Geom& G, const Groups& F, const Prof& C, hipStream_t s) {
-  const Sweep Sw = sweep_flat(G, Tile{1, 1});
+  const Sweep Sw = sweep_flat(G, Tile{1, 1}, true);
   const RingFold none = fold_for(G, nullptr);
   if (form == 1) EFWI_FLAT(Sw, k_velocity_bwd<1 EFWI_COMMA false EFWI_COMMA false EFWI_COMMA, Sw, G, F, C, none, RecvFold{});
   else EFWI_FLAT(Sw, k_velocity_bwd<0 EFWI_COMMA false EFWI_COMMA false EFWI_COMMA, Sw, G, F, C, none, RecvFold{});
 }
 void launch_stress_adj(const Geom& G, const Groups& F, const Prof& C, hipStream_t s) {
-  const Sweep Sw = sweep_flat(G, Tile{1, 1});
+  const Sweep Sw = sweep_flat(G, Tile{1, 1}, true);
   Source none;
   none.cell = -1;
   none.stf = nullptr;
@@ -1627,14 +1655,14 @@ void launch_stress_adj(const Geom& G, const Groups& F, const Prof& C, hipStream_
 
 // Batched launches (flat tiles only; a zdepth >= 16 shape falls back to its
 // flat counterpart rows x 1).
-static inline Sweep sweep_batch(const Geom& G, Tile t) {
+static inline Sweep sweep_batch(const Geom& G, Tile t, bool bwd, int shots) {
   if (t.zdepth >= 16) t = Tile{t.rows >= 4 ? 4 : t.rows, 1};
-  return sweep_flat(G, t);
+  return sweep_flat(G, t, bwd, shots);
 }
 template <int KIND, int FORM>
 static void launch_batch(Tile t, const Geom& G, const Prof& C, const BatchLaunch& L, hipStream_t s,
                          const BatchRing& R) {
-  Sweep Sw = sweep_batch(G, t);
+  Sweep Sw = sweep_batch(G, t, KIND >= 2, L.nshots);
   Sw.zrev = L.reverse;  // shots and planes last to first: start where the last launch ended
   const dim3 grid((unsigned)Sw.blocks, (unsigned)L.nshots);
   if (Sw.ly == 32) hipLaunchKernelGGL((k_batch_flat<KIND, FORM, 32>), grid, block_of(Sw), 0, s, Sw, G, C, L, R);

@@ -1,0 +1,69 @@
+"""Where the stencil kernels put two rows of 32 cells into a wavefront: grids on
+both sides of the rule, forward and backward kernels apart, against the oracle
+bit for bit, and the time of a grid whose strips of rows pair up badly."""
+import time
+
+import numpy as np
+import pytest
+import torch
+
+from util import oracle_run
+
+pytestmark = pytest.mark.gpu
+
+
+def _workload(n, npml, ny, nt):
+    from efwi import synth
+    w = synth.small(n=n - 2 * npml, npml=npml, nt=nt, ny=ny - 2 * npml)
+    assert w.grid.shape == (n, n, ny)
+    return w
+
+
+# 7 rows per strip and a C-PML edge inside a pair: the forward kernels take two rows, the backward ones one; 12 rows and
+# an edge inside a pair of both outer strips: both take two; 7 rows of 3 segments: both take one
+@pytest.mark.parametrize("n,npml,ny", [(60, 10, 84), (100, 9, 84), (60, 10, 148)])
+def test_pairs_of_rows(orc, n, npml, ny):
+    from efwi.propagator import Propagator
+    w = _workload(n, npml, ny, 24)
+    print(f"[gpu] pairs of rows on {w.grid.shape}, C-PML {npml}", flush=True)
+    obs = [s.astype(np.float32) for s in oracle_run(orc, w, model=w.true, calc_id=2).syn]
+    ref = oracle_run(orc, w, model=w.model, obs=obs, calc_id=1)
+    with Propagator(w.grid) as P:
+        P.set_model(*(torch.from_numpy(a) for a in w.model))
+        P.zero_gradient()
+        _, syn, _ = P.run_shot(w.shots[0], 1, torch.from_numpy(obs[0]), want_syn=True)
+        single = [g.cpu().numpy() for g in P.gradient()]
+        _, syns = P.run_batch(w.shots * 2, 1, [torch.from_numpy(obs[0])] * 2, want_syn=True)
+        batch = [g.cpu().numpy() for g in P.batch_gradient(1)]
+    for s in (syn, syns[1]):
+        assert np.array_equal(s.cpu().numpy(), ref.syn[0].astype(np.float32))
+    for a, c, b in zip(single, batch, (ref.glam, ref.gmu, ref.grho)):
+        assert np.abs(b).max() > 0
+        assert np.array_equal(a, b.astype(np.float32)) and np.array_equal(c, b.astype(np.float32))
+
+
+def test_fewer_rows_take_no_longer():
+    """A gradient on 60 x 60 x 148 cells (7 rows per strip) takes about the time
+    of 60 x 68 x 148 (8 rows, four full pairs); with half-filled pairs and
+    pairs across the C-PML's edge it took 1.14 times as long."""
+    from efwi import synth
+    from efwi.propagator import GridSpec, Propagator, ShotSpec
+    ms = {}
+    for nx in (60, 68):
+        g = GridSpec(60, nx, 148, 10, 200, 10.0, 10.0, 10.0, 1e-3, 15.0, 0)
+        vp = np.full(g.shape, 2500.0, np.float32)
+        stf = synth.ricker_integrated(15.0, g.nt, 1e-3).astype(np.float32)
+        shot = ShotSpec((15, nx // 2, 74), stf, np.array([[13, x, 74] for x in range(12, nx - 12)], np.int32))
+        obs = torch.zeros(3, len(shot.rec), g.nt)
+        with Propagator(g) as P:
+            P.set_model(*(torch.from_numpy(a) for a in synth.lame(vp, vp / 1.73, 310.0 * vp ** 0.25)))
+            times = []
+            for _ in range(7):
+                torch.cuda.synchronize()
+                t = time.perf_counter()
+                P.run_shot(shot, 1, obs)
+                torch.cuda.synchronize()
+                times.append(time.perf_counter() - t)
+        ms[nx] = min(times) * 1e3
+    print(f"[gpu] gradient on 60x60x148 {ms[60]:.1f} ms, on 60x68x148 {ms[68]:.1f}", flush=True)
+    assert ms[60] < 1.07 * ms[68]
