@@ -91,3 +91,28 @@ def test_fewer_rows_take_no_longer():
         ms[nx] = min(times) * 1e3
     print(f"[gpu] gradient on 60x60x148 {ms[60]:.1f} ms, on 60x68x148 {ms[68]:.1f}", flush=True)
     assert ms[60] < 1.07 * ms[68]
+
+
+@pytest.mark.parametrize("ny,depth", [(61 * 64, 2), (60 * 64, 1)])
+def test_backward_shapes_of_large_grids(orc, ny, depth):
+    """On both sides of the rule for two z planes per workgroup: the default
+    shape and the other one give the oracle's gradient."""
+    from efwi.propagator import Propagator
+    w = _workload(37, 4, ny, 16)
+    z, x, y = w.shots[0].src
+    w.shots[0].rec = np.array([(z + 1, x, y), (z + 2, x + 1, y - 2)], np.int32)
+    obs = np.random.default_rng(1).standard_normal((3, 2, w.grid.nt)).astype(np.float32)
+    print(f"[gpu] backward shapes on {w.grid.shape}", flush=True)
+    ref = oracle_run(orc, w, obs=[obs], calc_id=1)
+    for other in (False, True):
+        with Propagator(w.grid) as P:
+            P.set_model(*(torch.from_numpy(a) for a in w.model))
+            for k in ("velocity_bwd", "stress_bwd"):
+                assert P.tiles()[k] == (1, depth)
+                if other:
+                    P.set_tile(k, 1, 3 - depth)
+            P.run_shot(w.shots[0], 1, torch.from_numpy(obs))
+            got = [t.cpu().numpy() for t in P.gradient()]
+        for a, b in zip(got, (ref.glam, ref.gmu, ref.grho)):
+            assert np.abs(b).max() > 0
+            assert np.array_equal(a, b.astype(np.float32))
