@@ -188,7 +188,7 @@ int Ctx::run_batch(const efwi_shot* shots, int n, int calc_id, const float* cons
     d.ring = calc_id == EFWI_CALC_GRADIENT && gsz0 > 0 ? batch.ring[k % gsz] : nullptr;
   }
   // receivers in the velocity kernels where every shot's can be
-  bool fold_rec = recv_foldable(Tile{1, 1}, G);
+  bool fold_rec = recv_foldable(Tile{1, 1}, G, true) && (!grad || recv_foldable(Tile{1, 1}, G, false));
   for (int k = 0; k < n; k++) fold_rec = fold_rec && (batch.recv[k].on || batch.nrec[k] == 0);
   for (int k = 0; k < n; k++) {
     const RecvFold v = fold_rec ? batch.recv[k].fold(batch.nrec[k]) : RecvFold{};

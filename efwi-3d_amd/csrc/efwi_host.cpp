@@ -548,7 +548,7 @@ int Ctx::map_receivers(const efwi_shot* sh, RecvMap& m) {
   constexpr size_t kMaxTab = 1u << 20;
   m.on = false;
   const int n = sh->nrec;
-  if (n <= 0 || !recv_foldable(Tile{1, 1}, G)) return EFWI_OK;
+  if (n <= 0 || !recv_foldable(Tile{1, 1}, G, true)) return EFWI_OK;
   const size_t nrows = (size_t)cfg.nz * cfg.nx, py = (size_t)G.py;
   std::vector<int> host(nrows + n, -1);
   size_t used = 0;
@@ -642,7 +642,7 @@ void Ctx::forward_step(const Groups& Ff, const Wave& Wf, const Source& Sf, int i
   const bool fs = launch_stress_fwd(tiles[K_STRESS_FWD], G, Ff, C, Sf, it, s, src_stencil ? &rf : nullptr);
   prof.end(s);
   if (!src_stencil) launch_add_source(Wf.szz, Wf.sxx, Wf.syy, src_cell, stf_dev, it, G.dt, +1, s);
-  RecvFold rec = record && recv_foldable(tiles[K_VELOCITY_FWD], G) ? recv.fold(nrec) : RecvFold{};
+  RecvFold rec = record && recv_foldable(tiles[K_VELOCITY_FWD], G, true) ? recv.fold(nrec) : RecvFold{};
   if (rec.row) rec.out = syn_t + (size_t)(it + 1) * 3 * nrec;
   prof.begin(K_VELOCITY_FWD, s);
   const bool fv = launch_velocity_fwd(tiles[K_VELOCITY_FWD], cfg.formulation, G, Ff, C, s, &rf, &rec);
@@ -805,7 +805,7 @@ int Ctx::run_shot(const efwi_shot* sh, int calc_id, const float* obs, float* syn
         RingFold rf{};
         rf.B = B;
         rf.slot = ring + slot * 9 * B.n;
-        RecvFold inj = split_bwd == 0 && recv_foldable(tiles[K_VELOCITY_BWD], G) ? recv.fold(nrec) : RecvFold{};
+        RecvFold inj = split_bwd == 0 && recv_foldable(tiles[K_VELOCITY_BWD], G, false) ? recv.fold(nrec) : RecvFold{};
         if (inj.row) inj.res = res_t + (size_t)it * 3 * nrec;
         prof.begin(K_VELOCITY_BWD, s);
         const bool fv = launch_velocity_bwd(tiles[K_VELOCITY_BWD], form, G, F, C, s, &rf, split_bwd == 1, &inj);

@@ -77,7 +77,7 @@ struct RecvFold {
   const float* res;             // backward: the injected step's [3][nrec]
   int nrec;
 };
-bool recv_foldable(Tile t, const Geom& G);
+bool recv_foldable(Tile t, const Geom& G, bool forward);
 // launch shape of the two backward kernels before a caller or the autotuner sets one
 Tile default_bwd_tile(const Geom& G);
 bool launch_stress_fwd(Tile t, const Geom& G, const Groups& F, const Prof& C, const Source& S, int it,

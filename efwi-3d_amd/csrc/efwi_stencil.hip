@@ -1496,16 +1496,15 @@ Tile default_bwd_tile(const Geom& G) {
   const Sweep S = sweep_flat(G, Tile{1, 1}, true);
   return S.ly == 64 && (long)(G.nz - 4) * (G.nx - 4) * S.nyb >= 256L * 256 ? Tile{1, 2} : Tile{1, 1};
 }
-// Receivers are folded up to 128 wavefronts per CU: on larger grids the kernels
-// lose as much or more to the folded form's registers (velocity_bwd of 160x240x240
-// cells 117 -> 123) as the launches cost. Folded against not, a gradient of 44^3
-// cells 3.88 and 4.29 ms for 119 steps, of 84^3 43.7 and 45.1 for 499; the forward pass
-// 84^3 19.7 and 21.0 us per step, 130^3 59.8 and 61.0; above the limit 70x180x180 61.3
-// and 61.8, 84x180x180 72.7 and 72.5, 26x400x400 (every surface cell a receiver) 128.6
-// and 127.5, 64x250x250 127.4 both; a gradient of 160x240x240 165 and 162 ms for 149 steps.
-bool recv_foldable(Tile t, const Geom& G) {
+// Receivers are folded up to 256 (forward) and 128 (backward) wavefronts per
+// CU: on larger grids the kernels lose more to the folded form's registers
+// (velocity_bwd 117 -> 123) than the launches cost. A gradient of 44^3 cells
+// 4.29 -> 3.88 ms for 119 steps, of 84^3 cells 45.1 -> 43.7 ms for 499; the
+// forward pass of 84x180x180 cells 37.2 -> 36.9 ms for 499; a gradient of 160x240x240
+// cells would go from 162 to 165 ms for 149.
+bool recv_foldable(Tile t, const Geom& G, bool forward) {
   const long waves = (long)(G.nz - 4) * (G.nx - 4) * ((G.ny - 3) / 64 + 1);
-  return !marching(t) && waves <= 128 * 256;
+  return !marching(t) && waves <= (forward ? 256 : 128) * 256;
 }
 static inline RecvFold recv_for(const RecvFold* v) { return v ? *v : RecvFold{}; }
 
