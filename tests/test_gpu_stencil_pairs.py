@@ -42,6 +42,31 @@ def test_pairs_of_rows(orc, n, npml, ny):
         assert np.array_equal(a, b.astype(np.float32)) and np.array_equal(c, b.astype(np.float32))
 
 
+# 128 x 128 rows of two segments are 128 wavefronts per CU: receivers in both velocity kernels; one row more: in the
+# forward one; 128 x 256 rows: as many as there; one more: gather and scatter launches
+@pytest.mark.parametrize("nx", [132, 133, 260, 261])
+def test_receivers_on_both_sides_of_the_limits(orc, nx):
+    from efwi import synth
+    from efwi.propagator import GridSpec, Propagator, ShotSpec
+    g = GridSpec(132, nx, 68, 8, 12, 10.0, 10.0, 10.0, 1e-3, 15.0, 0)
+    vp = np.linspace(2000.0, 3000.0, 132, dtype=np.float32)[:, None, None] * np.ones(g.shape, np.float32)
+    model = synth.lame(vp, vp / 1.73, 310.0 * vp ** 0.25)
+    rec = np.array([(13, nx // 2 + x, 34 + y) for x in (-2, 0, 1) for y in (-30, -1, 0, 29)] + [(13, nx // 2, 34)], np.int32)
+    shot = ShotSpec((12, nx // 2, 34), synth.ricker_integrated(15.0, g.nt, 1e-3).astype(np.float32), rec)
+    w = synth.Workload("limit", g, [shot], model, model, vp)
+    obs = np.random.default_rng(nx).standard_normal((3, len(rec), g.nt)).astype(np.float32)
+    print(f"[gpu] receivers on {g.shape}", flush=True)
+    with Propagator(g) as P:
+        P.set_model(*(torch.from_numpy(a) for a in model))
+        P.zero_gradient()
+        _, syn, res = P.run_shot(shot, 1, torch.from_numpy(obs), want_syn=True, want_res=True)
+        got = [t.cpu().numpy() for t in (syn, res, *P.gradient())]
+    ref = oracle_run(orc, w, obs=[obs], calc_id=1)
+    for a, b in zip(got, (ref.syn[0], ref.res[0], ref.glam, ref.gmu, ref.grho)):
+        assert np.abs(b).max() > 0
+        assert np.array_equal(a, b.astype(np.float32))
+
+
 def test_fewer_rows_take_no_longer():
     """A gradient on 60 x 60 x 148 cells (7 rows per strip) takes about the time
     of 60 x 68 x 148 (8 rows, four full pairs); with half-filled pairs and
