@@ -1528,7 +1528,7 @@ int efwi_nn_conv3_cat(const uint16_t* src, int lds, int kc1, int up1, const uint
   const Vol V{nz, nx, ny};
   // bricks of 2 x 2 rows of 64, 32 or 16 voxels along y; 1 to 4 output blocks
   // per wavefront (a divisor of the block count, so no block is partial)
-  const int MB = ny >= 64 ? 4 : ny >= 32 ? 2 : 1;
+  const int cus = device_cus(), MB = ny >= 64 ? 4 : ny >= 32 ? 2 : 1;
   const int nbt = nc / 16;
   const int TZ = conv_tz(MB);
   const int ntz = (nz + TZ - 1) / TZ, ntx = (nx + 1) / 2, nty = (ny + 16 * MB - 1) / (16 * MB);
@@ -1543,15 +1543,15 @@ int efwi_nn_conv3_cat(const uint16_t* src, int lds, int kc1, int up1, const uint
   // rows a workgroup per CU has nothing to overlap: k_conv3 there (16->16 at
   // 24x32x32 5.3 us against 5.7).
   const long pbricks = (long)((nz + 3) / 4) * ntx * nty;
-  const bool many = pbricks * nbt > device_cus();
+  const bool many = pbricks * nbt > cus;
   // (its row numbers, row bytes and weight offsets are 32-bit)
   const long row_bytes = 2L * ny * std::max(std::max(lds, lds2), std::max(ldd, std::max(ldd2, ldm)));
   const bool fits = (long)nz * nx <= INT_MAX / 2 && row_bytes <= INT_MAX && 54L * nc * kc <= INT_MAX &&
-                    pbricks <= INT_MAX - 8L * device_cus();
+                    pbricks <= INT_MAX - 8L * cus;
   if (MB >= 2 && mode == 0 && vec_out && fits && (many || MB == 4 || kc > 16)) {
     const int nb = many && kc == 16 && nbt % 3 == 0 ? 3 : many && nbt % 2 == 0 ? 2 : 1;
     const int pxcd = (int)((pbricks + 7) / 8);
-    const dim3 pgrid(8u * std::max(1, std::min(pxcd, (nb == 1 ? 2 : 1) * device_cus() / 8 / (nbt / nb))),
+    const dim3 pgrid(8u * std::max(1, std::min(pxcd, (nb == 1 ? 2 : 1) * cus / 8 / (nbt / nb))),
                      (unsigned)(nbt / nb));
 #define EFWI_NN_CONV_PIPE(M, B, ONE)                                                                              \
   hipLaunchKernelGGL((k_conv_pipe<M, B, ONE>), pgrid, dim3(512), 0, s, src, lds, kc, w, bias, dst, ldd, nc, mask, ldm, \
@@ -1573,7 +1573,7 @@ int efwi_nn_conv3_cat(const uint16_t* src, int lds, int kc1, int up1, const uint
   // workgroups, whose wavefronts hide each other's load latency (48x64x64
   // voxels: 32->32 27.7 -> 22.5 us, 96->32 82 -> 75 us)
   int NB = nbt % 4 == 0 ? 4 : nbt % 3 == 0 ? 3 : nbt % 2 == 0 ? 2 : 1;
-  if (bricks * (nbt / NB) < 4L * device_cus()) NB = 1;
+  if (bricks * (nbt / NB) < 4L * cus) NB = 1;
   // Rows of 32 voxels or more in mode 0 come here with unaligned outputs. Several
   // blocks then pay only where the halo is one chunk or they
   // are three (unaligned, one block against them: 16->48 at 96x128x128 165 and 136 us,
