@@ -625,12 +625,25 @@ __device__ __forceinline__ void stress_bwd_cell(const Geom& G, const Acc& acc, c
 
 // Per-wavefront dispatch of the backward cells: body gets the flags (X, Z, Y)
 // of the variant as compile-time constants.
-template <typename Body>
+// X and Z are one flag in the marching kernels (APART false): eight variants
+// around their z queues cost more than the C-PML terms they save (velocity_bwd
+// {4, 16} at 120x200x200 345 -> 542 us, stress_bwd {8, 32} 336 -> 435).
+template <bool APART = true, typename Body>
 __device__ __forceinline__ void by_slabs(const Geom& G, const Cell& c, Body&& body) {
   using T = std::true_type;
   using N = std::false_type;
   const int p = G.npml;
   const bool x = in_pml(c.x, G.nx, p), z = in_pml(c.z, G.nz, p), y = __any(in_pml(c.y, G.ny, p)) != 0;
+  if constexpr (!APART) {
+    if (x || z) {
+      if (y) body(T{}, T{}, T{});
+      else body(T{}, T{}, N{});
+    } else {
+      if (y) body(N{}, N{}, T{});
+      else body(N{}, N{}, N{});
+    }
+    return;
+  }
   if (y) {
     if (x) {
       if (z) body(T{}, T{}, T{});
@@ -1042,7 +1055,7 @@ __global__ __launch_bounds__(64 * R) void k_velocity_fwd_m(Sweep Sw, Geom G, Gro
 template <int FORM, int R>
 __global__ __launch_bounds__(64 * R) void k_velocity_bwd_m(Sweep Sw, Geom G, Groups F, Prof C) {
   march<VelocityBwdSlots, R>(Sw, G, F, [&](const Cell& c, const auto& acc) {
-    by_slabs(G, c, [&](auto X, auto Z, auto Y) {
+    by_slabs<false>(G, c, [&](auto X, auto Z, auto Y) {
       velocity_bwd_cell<FORM, true, decltype(X)::value, decltype(Z)::value, decltype(Y)::value>(G, acc, C, c);
     });
   });
@@ -1053,7 +1066,7 @@ __global__ __launch_bounds__(64 * R) void k_stress_bwd_m(Sweep Sw, Geom G, Group
   const unsigned so = source_off(S);
   const float amp = source_amp(S, G, it);
   march<StressBwdSlots, R>(Sw, G, F, [&](const Cell& c, const auto& acc) {
-    by_slabs(G, c, [&](auto X, auto Z, auto Y) {
+    by_slabs<false>(G, c, [&](auto X, auto Z, auto Y) {
       stress_bwd_cell<true, decltype(X)::value, decltype(Z)::value, decltype(Y)::value>(G, acc, C, c, so, amp);
     });
   });

@@ -117,3 +117,23 @@ def test_backward_shapes_of_large_grids(orc, ny, depth):
         for a, b in zip(got, (ref.glam, ref.gmu, ref.grho)):
             assert np.abs(b).max() > 0
             assert np.array_equal(a, b.astype(np.float32))
+
+
+def test_marching_backward_kernels_are_alike():
+    """The marching backward kernels read and write about the same number of
+    fields: velocity_bwd in {4, 16} takes 1.1 times stress_bwd's time (with a
+    variant per set of C-PML axes it took 1.75 times)."""
+    from efwi.propagator import Propagator
+    w = _workload(84, 10, 84, 60)
+    obs = torch.zeros(3, len(w.shots[0].rec), w.grid.nt)
+    with Propagator(w.grid) as P:
+        P.set_model(*(torch.from_numpy(a) for a in w.model))
+        for k in ("velocity_bwd", "stress_bwd"):
+            P.set_tile(k, 4, 16)
+        P.run_shot(w.shots[0], 1, obs)
+        P.profile(True)
+        P.profile_read(reset=True)
+        P.run_shot(w.shots[0], 1, obs)
+        us = {k: ms / n * 1e3 for k, (ms, n) in P.profile_read(reset=True).items() if n}
+    print(f"[gpu] marching velocity_bwd {us['velocity_bwd']:.1f} us, stress_bwd {us['stress_bwd']:.1f}", flush=True)
+    assert us["velocity_bwd"] < 1.4 * us["stress_bwd"]
