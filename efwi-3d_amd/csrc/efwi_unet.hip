@@ -1541,7 +1541,8 @@ int efwi_nn_conv3_cat(const uint16_t* src, int lds, int kc1, int up1, const uint
   // 24x32x32, 384 workgroups of one: 12.6 us at two, 16.5 at one, 18.3 in k_conv3;
   // at 16x32x32, 256 of one: 11.8, 10.9, 14.8). With 16 input channels and short
   // rows a workgroup per CU has nothing to overlap: k_conv3 there (16->16 at
-  // 24x32x32 5.3 us against 5.7).
+  // 24x32x32 5.3 us against 5.7; rows of 64 voxels gain at every size: 4x4x64 5.4
+  // against 5.7 in k_conv3, 16x32x64 5.7 and 6.2, 24x24x130 5.8 and 6.3).
   const long pbricks = (long)((nz + 3) / 4) * ntx * nty;
   const bool many = pbricks * nbt > cus;
   // (its row numbers, row bytes and weight offsets are 32-bit)
