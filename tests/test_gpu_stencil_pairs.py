@@ -137,3 +137,38 @@ def test_marching_backward_kernels_are_alike():
         us = {k: ms / n * 1e3 for k, (ms, n) in P.profile_read(reset=True).items() if n}
     print(f"[gpu] marching velocity_bwd {us['velocity_bwd']:.1f} us, stress_bwd {us['stress_bwd']:.1f}", flush=True)
     assert us["velocity_bwd"] < 1.4 * us["stress_bwd"]
+
+
+def test_scattered_receivers_of_a_short_run(orc):
+    """8000 receivers all over the grid for 19 steps: their tables would cost
+    more than the launches they save (1.17 times the time of the same receivers
+    and one on the outermost cells, which sends them to the launches anyway);
+    seismograms are the oracle's."""
+    from efwi import synth
+    from efwi.propagator import GridSpec, Propagator, ShotSpec
+    g = GridSpec(60, 60, 300, 8, 20, 10.0, 10.0, 10.0, 1e-3, 15.0, 0)
+    vp = np.full(g.shape, 2500.0, np.float32)
+    model = synth.lame(vp, vp / 1.73, 310.0 * vp ** 0.25)
+    rng = np.random.default_rng(0)
+    rec = np.stack([rng.integers(2, n - 2, 8000) for n in g.shape], 1).astype(np.int32)
+    rec[:50] = [30, 30, 150] + rng.integers(-4, 5, (50, 3))  # near the source
+    stf = synth.ricker_integrated(15.0, g.nt, 1e-3).astype(np.float32)
+    shot = ShotSpec((30, 30, 150), stf, rec)
+    outer = ShotSpec((30, 30, 150), stf, np.concatenate([rec, [[0, 0, 0]]]).astype(np.int32))
+    print(f"[gpu] scattered receivers on {g.shape}", flush=True)
+    with Propagator(g) as P:
+        P.set_model(*(torch.from_numpy(a) for a in model))
+        times = {}
+        for _ in range(15):
+            for name, s in (("inside", shot), ("outer", outer)):
+                torch.cuda.synchronize()
+                t = time.perf_counter()
+                _, syn, _ = P.run_shot(s, 2)
+                torch.cuda.synchronize()
+                times.setdefault(name, []).append(time.perf_counter() - t)
+                if name == "inside":
+                    got = syn.cpu().numpy()
+    ref = oracle_run(orc, synth.Workload("scattered", g, [shot], model, model, vp), calc_id=2).syn[0]
+    assert np.abs(ref).max() > 0 and np.array_equal(got, ref.astype(np.float32))
+    print(f"[gpu] {min(times['inside']) * 1e3:.2f} ms, {min(times['outer']) * 1e3:.2f} with one outside", flush=True)
+    assert min(times["inside"]) < 1.08 * min(times["outer"])
