@@ -1,6 +1,8 @@
 """What a context keeps from one batch to the next (shot table, captured graphs,
 boundary rings, launch settings): a batch gives the results of the same shots
 run one by one whatever batches ran before it."""
+import time
+
 import numpy as np
 import pytest
 import torch
@@ -89,23 +91,18 @@ def test_batch_config_costs_nothing():
     obs = _obs(w, shots, 9)
     print(f"[gpu] 12 shots on {w.grid.shape} with and without batch_config", flush=True)
 
-    def best(P):
-        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-        ms = []
-        for _ in range(6):
-            a.record()
-            misfits, _ = P.run_batch(shots, 1, obs)
-            b.record()
-            b.synchronize()
-            ms.append(a.elapsed_time(b))
-        return min(ms), misfits
-
+    ms, misfits = ([], []), [None, None]
     with _open(w) as P, _open(w) as Q:
         Q.batch_config()
-        t, m = best(P)
-        t2, m2 = best(Q)
+        for _ in range(6):
+            for k, prop in enumerate((P, Q)):
+                torch.cuda.synchronize()
+                t = time.perf_counter()
+                misfits[k], _ = prop.run_batch(shots, 1, obs)
+                ms[k].append((time.perf_counter() - t) * 1e3)
+    t, t2 = min(ms[0]), min(ms[1])
     print(f"[gpu] {t:.1f} ms, {t2:.1f} ms after batch_config", flush=True)
-    assert m == m2 and t2 < 1.4 * t
+    assert misfits[0] == misfits[1] and t2 < 1.4 * t
 
 
 @pytest.mark.parametrize("use_graph", [True, False])
